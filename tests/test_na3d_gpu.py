@@ -286,3 +286,33 @@ def test_na3d_wide_window_sampled_rows(gpu):
     ref = O.na3d(q, k, v, (3, 7, 31), ty_rows=rows)
     sel = tuple(np.array(rows).T)
     _check(o[0][sel], ref[0][sel], "wide-window rows")
+
+
+@pytest.mark.parametrize("shape,ks,seed", [
+    ((1, 4, 13, 17, 192), (3, 7, 7), 90),   # 3072 workgroups; one row of the second wave row, one column of the last brick
+    ((2, 3, 9, 33, 86), (3, 5, 9), 91),     # the last y brick's second wave row empty, widest x window
+    ((1, 2, 16, 16, 768), (2, 16, 4), 92),  # y window spans the grid: no chunk is skipped
+    ((1, 12, 4, 8, 256), (5, 4, 3), 93),    # the second wave row of every brick holds no query
+])
+def test_na3d_quad_waves(gpu, shape, ks, seed):
+    """Head dim 64, x windows up to 9, grids of 3072 workgroups and more: the
+    tall bricks with 2 x 2 waves of 4 y x 8 x queries. Heads are independent,
+    so the same call on a few heads (8 y x 4 x waves) must agree up to the
+    order of the row sums and one bf16 rounding, and both with the oracle."""
+    from vidax_amd import _lib, neighborhood_attention_3d
+    B, T, H, W, NH = shape
+    _say(f"na3d quad waves shape={shape} kernel={ks} seed={seed}")
+    g = torch.Generator(device=gpu).manual_seed(seed)
+    q, k, v = (torch.randn((B, T, H, W, NH, 64), generator=g, device=gpu) for _ in range(3))
+    q, k, v = (q * 64 ** -0.5).to(torch.bfloat16), k.to(torch.bfloat16), v.to(torch.bfloat16)
+    assert B * T * -(-H // 8) * -(-W // 16) * NH >= 3072
+    out = neighborhood_attention_3d(q, k, v, ks)
+    launched = _lib.last_launch()
+    assert launched == "na3d_tall_kernel<64>" == _expected_kernel(H, W, ks[2], 64, T, ks[0]), launched
+    heads = [0, NH // 2 + 1, NH - 1]
+    few = [x[..., heads, :].contiguous() for x in (q, k, v)]
+    out_few = neighborhood_attention_3d(*few, ks)
+    torch.cuda.synchronize()
+    ref = O.na3d(*(x.float().cpu().numpy() for x in few), ks)
+    _check(out[..., heads, :].float().cpu().numpy(), ref, "2 x 2 waves vs oracle")
+    _check(out_few.float().cpu().numpy(), ref, "8 y x 4 x waves vs oracle")

@@ -382,19 +382,29 @@ void na3d_wave_kernel(const Na3dArgs a, int n_yb, int n_xb, int n_xg) {
 
 
 // ---------------------------------------------------------------------------
-// Pipelined row-streaming kernel (kw' <= 25). A workgroup of 4 waves owns a
-// brick of 1 (t) x 4 (y) x 32 (x) queries of one head; wave w takes the 4 y
-// rows and x columns 8w..8w+7. The union of the brick's windows is kt' x NY
-// key rows (t', y') of at most 31 + kw' consecutive x positions, and every
-// wave needs every row, so all waves run the same step sequence. The rows are
-// streamed through LDS kRows at a time (2 rows for SEG = 16, 1 for SEG = 32),
-// K and V in separate two-slot rings filled by the DMA path one step ahead;
-// each wave reads the SEG-wide x window it needs from the step's rows, one
-// 32-key chunk. Step s issues QK^T(s+1) and PV(s-1) as one block of
-// D/16 + D/16 MFMA slots interleaved with the masking and softmax of chunk s
-// (as in the flash kernel), so the matrix cores and the VALU work of a wave
-// overlap. With at most 80 KiB of LDS and 256 VGPRs two workgroups share a
-// CU. Head dims 128 and 64 (the LTX-2.5 diffusion VAE's) are instantiated.
+// Row-streaming kernels (kw' <= 25). A workgroup of 4 waves owns a brick of 1
+// (t) x 4 (y) x 32 (x) queries of one head; wave w takes the 4 y rows and x
+// columns 8w..8w+7. The union of the brick's windows is kt' x NY key rows
+// (t', y') of at most 31 + kw' consecutive x positions, and every wave needs
+// every row, so all waves run the same step sequence. The rows are streamed
+// through LDS kRows at a time (2 rows for SEG = 16, 1 for SEG = 32), K and V
+// in separate two-slot rings filled by the DMA path one step ahead; each wave
+// reads the SEG-wide x window it needs from the step's rows, one 32-key chunk.
+// A step has one of two forms:
+// - pipelined (head dim 128 but for the t-stacked bricks, and the 32-key
+//   segments): step s issues QK^T(s+1) and PV(s-1) as one block of D/16 +
+//   D/16 MFMA slots interleaved with the masking and softmax of chunk s (as
+//   in the flash kernel), so that a wave overlaps its own matrix and VALU
+//   work; two workgroups share a CU (three at head dim 64).
+// - block (head dim 64 with 16-key segments, and the t-stacked bricks): step
+//   s takes the softmax of chunk s, then the MFMAs of PV(s) and QK^T(s+1) in
+//   the same score and probability registers. With one set of each a wave
+//   needs 24 registers fewer, so one more wave fits a SIMD, and those waves
+//   overlap each other. Same box, pipelined -> block: 21x45x80 NH=24 (3,7,7)
+//   at head dim 128 (2 -> 3 waves per SIMD) 0.760 -> 0.747 ms; 5x11x60 NH=32
+//   at head dim 64 (1 x 4 x 32 bricks, 2 -> 4) 27.2 -> 23.4 us. The 32-key
+//   segments at head dim 64 (3 -> 4) lost 7 % at a (3,11,15) window and stay
+//   pipelined.
 //
 // The tall geometry (TALL, SEG = 16, 9 < kw' <= 13) uses bricks of
 // 1 x 8 (y) x 16 (x) with waves of 8 y rows x 4 x columns: a wave's x union
@@ -404,36 +414,50 @@ void na3d_wave_kernel(const Na3dArgs a, int n_yb, int n_xb, int n_xg) {
 
 // WIDE: tall bricks 32 x columns wide with 8 waves (each still 8 y x 4 x):
 // the 42-key x union of a row is staged in 48 slots for 32 queries (26 in
-// 32 for 16 with the narrow brick), one workgroup barrier per step for
-// twice the queries.
+// 32 for 16 with the narrow brick). Its two waves per SIMD run half a step
+// apart (kHalfStep: a barrier before each block of the step, waves 4-7 one
+// barrier behind waves 0-3), so that one wave's MFMA block meets the other's
+// softmax block, and only waves 0-3 copy: stage 5 (33x88x160 NH=4 at (11,11,
+// 11), deep bricks) 1.476 -> 1.434 ms.
 // DEEP: wide bricks two t planes deep, 2 (t) x 4 (y) x 32 (x), waves of 2 t x
 // 4 y x 4 x queries: for a t window of kt' planes the union of a wave's
 // windows is (kt' + 1) x (kh' + 3) rows instead of kt' x (kh' + 7), e.g. 12 x
 // 14 against 11 x 18 rows at (11, 11, 11).
 // TSTACK: 2 (t) x 4 (y) x 16 (x) bricks whose four 4 y x 8 x waves sit two
 // per t plane: one stream of (kt' + 1) planes serves both planes' waves, each
-// scoring only the chunks of its own kt' planes (a wave none of whose rows
-// in the previous, current and next chunk lies in its t window only copies).
-template <int SEG, int D, bool TALL = false, bool WIDE = false, bool DEEP = false, bool TSTACK = false>
+// scoring only the chunks of its own kt' planes.
+// QUAD: tall bricks whose four waves sit two by two, each 4 y x 8 x (kw' <=
+// 9): at a (3,7,7) window a wave scores 10 of a plane's 14 rows, 480 keys per
+// query against 672 for 8 y x 4 x waves, and a row is staged in 24 slots
+// instead of 32. The steps are as many, so it pays once the grid keeps the
+// CUs busy (kNaQuadMinGroups).
+template <int SEG, int D, bool TALL = false, bool WIDE = false, bool DEEP = false, bool TSTACK = false, bool QUAD = false>
 struct PipeCfg {
+  static constexpr bool kBlock = (D == 64 && SEG == 16) || TSTACK;  // block form of the step
+  static constexpr bool kHalfStep = WIDE;                           // the two waves of a SIMD half a step apart
+  static constexpr bool kSkip = TSTACK || QUAD;                     // a wave skips chunks outside its t (y) window
+  // block form: row sums of the unrounded probabilities (their x window a
+  // mask per score), or, for the tall bricks, of the packed bf16 ones
+  static constexpr bool kSumF32 = !TALL;
   static_assert(!TALL || SEG == 16, "the tall geometry reads 16-key segments");
   static_assert(!WIDE || TALL, "wide bricks are tall bricks");
   static_assert(!DEEP || WIDE, "deep bricks are wide bricks");
   static_assert(!TSTACK || (!TALL && SEG == 16), "t-stacked bricks hold 1 x 4 x 8 waves on 16-key segments");
-  static constexpr bool kTStack = TSTACK;
+  static_assert(!QUAD || (TALL && !WIDE && D == 64), "quad bricks are narrow tall bricks at head dim 64");
+  static_assert(!kHalfStep || kBlock, "the half-step barriers are between the block form's blocks");
   static constexpr int kWaves = WIDE ? 8 : 4;
   static constexpr int kThreads = kWaves * 64;
   static constexpr int kQT = DEEP || TSTACK ? 2 : 1;     // t planes per brick
   static constexpr int kWT = DEEP ? 2 : 1;               // t planes per wave
-  static constexpr int kWX = TSTACK ? kWaves / 2 : kWaves;  // waves side by side in x
+  static constexpr int kWX = TSTACK || QUAD ? kWaves / 2 : kWaves;  // waves side by side in x
   static constexpr int kBrickY = TALL ? (DEEP ? 4 : 8) : 4;
   static constexpr int kBrickX = TALL ? (WIDE ? 32 : 16) : (TSTACK ? 16 : 32);
   static constexpr int kQX = kBrickX / kWX;              // x columns per wave
-  static constexpr int kQY = 32 / (kQX * kWT);           // y rows per wave (and per brick)
+  static constexpr int kQY = 32 / (kQX * kWT);           // y rows per wave
   static constexpr int kRB = D * 2;                      // bytes of one key
   static constexpr int kRows = SEG == 16 ? 2 : 1;        // key rows per step
   // key slots per LDS row (>= kBrickX - kQX + SEG, a multiple of 8)
-  static constexpr int kNS = TALL ? (WIDE ? 48 : 32) : (TSTACK ? 24 : (SEG == 16 ? 40 : 64));
+  static constexpr int kNS = TALL ? (WIDE ? 48 : QUAD ? 24 : 32) : (TSTACK ? 24 : (SEG == 16 ? 40 : 64));
   // An LDS key row is D/64 half-planes of kNS slots x 128 bytes (d 0-63,
   // then d 64-127); one 1 KiB DMA copy fills 8 slots of one half-plane.
   static constexpr int kHalfL = kNS * 128;               // one half-plane of a row
@@ -443,9 +467,10 @@ struct PipeCfg {
   static constexpr int kK = 0, kV = 2 * kSlot;           // K slots 0,1 then V slots 0,1
   static constexpr int kSmem = 4 * kSlot;
   static constexpr int kCopies = kRows * kRowL / 1024;   // DMA copies per tensor per step
-  // the copies of a step spread over the waves (those past kCopies are skipped;
-  // every wait for them is a wait for all of a wave's copies)
-  static constexpr int kCopiesPerWave = (kCopies + kWaves - 1) / kWaves;
+  // the copies of a step spread over the copying waves (those past kCopies
+  // are skipped; every wait for them is a wait for all of a wave's copies)
+  static constexpr int kCopyWaves = kHalfStep ? 4 : kWaves;
+  static constexpr int kCopiesPerWave = (kCopies + kCopyWaves - 1) / kCopyWaves;
   static constexpr int kQK = D / 16;                     // MFMAs of QK^T per chunk
   static constexpr int kPV = 2 * (D / 32);               // MFMAs of PV per chunk
   static constexpr int kSlots = kQK + kPV;
@@ -453,12 +478,11 @@ struct PipeCfg {
   static_assert(kNS % kKeysPerCopy == 0 && kHalfL % 256 == 0, "whole copies per row, bank-aligned planes");
 };
 
-template <int SEG, int D, bool TALL, bool WIDE = false, bool DEEP = false, bool TSTACK = false>
-__device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int n_xb) {
-  using C = PipeCfg<SEG, D, TALL, WIDE, DEEP, TSTACK>;
-  static_assert(C::kQY == C::kBrickY, "the waves of a t plane sit side by side in x");
+template <int SEG, int D, bool TALL, bool WIDE = false, bool DEEP = false, bool TSTACK = false, bool QUAD = false>
+__device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int n_xb, unsigned char* smem) {
+  using C = PipeCfg<SEG, D, TALL, WIDE, DEEP, TSTACK, QUAD>;
+  static_assert(C::kQY * (QUAD ? 2 : 1) == C::kBrickY, "the waves of a brick cover its y rows");
   static_assert(C::kBrickX - C::kQX + SEG <= C::kNS, "a wave's segment stays inside the LDS row");
-  __shared__ __attribute__((aligned(16))) unsigned char smem[C::kSmem];
   VX_LDS unsigned char* const lds = (VX_LDS unsigned char*)smem;
   const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
 
@@ -500,6 +524,7 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
   // The integer divisions below run on the vector unit; their (uniform)
   // results go back to scalar registers, so the row walk stays scalar.
   auto uni = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+  auto uniform_f32 = [](float x) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x))); };
   head = uni(head);
   const int xb = uni(brick % n_xb);
   const int yb = uni((brick / n_xb) % n_yb);
@@ -518,48 +543,50 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
   const int n_steps = (nrows + C::kRows - 1) / C::kRows;
 
   // ---- this wave's queries: t planes tw..tw+kWT-1 (tw = t, or t + 1 for the
-  // second pair of t-stacked waves), y rows y0..y0+kBrickY-1, x columns
-  // xq0..xq0+kQX-1.
-  const int tw = t + wave / C::kWX;
+  // second pair of t-stacked waves), y rows yw..yw+kQY-1 (yw = y0, or y0 + 4
+  // for the second pair of quad waves), x columns xq0..xq0+kQX-1.
+  const int tw = QUAD ? t : t + wave / C::kWX;
+  const int yw = QUAD ? y0 + wave / C::kWX * C::kQY : y0;
   const int xq0 = x0 + C::kQX * (wave % C::kWX);
   const int ox = uni(window_start(min(xq0, W - 1), W, kw) - X_lo);  // wave's first x slot, <= kBrickX - kQX
 
   // ---- this lane's query and its window.
-  const int tq = tw + col / (C::kQX * C::kQY), yq = y0 + col / C::kQX % C::kQY, xq = xq0 + col % C::kQX;
-  const bool wave_in = y0 < Hs && xq0 < W && tw < T;  // wave-uniform: some query of the wave is in the grid
+  const int tq = tw + col / (C::kQX * C::kQY), yq = yw + col / C::kQX % C::kQY, xq = xq0 + col % C::kQX;
+  const bool wave_in = yw < Hs && xq0 < W && tw < T;  // wave-uniform: some query of the wave is in the grid
   const int tqc = min(tq, T - 1), yqc = min(yq, Hs - 1), xqc = min(xq, W - 1);
   const int sy = window_start(yqc, Hs, kh) - Y_lo;
   const int st = window_start(tqc, T, kt) - t_lo;  // (deep bricks: the lane's first plane in the box)
   const int sx = window_start(xqc, W, kw) - X_lo - ox;  // in [0, SEG - kw]
   // The x window of score register i (key (i/4)*8 + hf*4 + i%4 of the
-  // chunk). kAccMask: a 0 / -inf vector that every chunk's QK^T MFMAs start
-  // from (the first one's accumulator input), so the x window costs no
-  // instruction per score. Otherwise (the tall bricks at head dim 64, whose
-  // short steps need four waves per SIMD, i.e. at most 128 VGPRs, which the
-  // extra accumulator input does not leave) a 0 / 0xffff mask per bf16 half
-  // of each packed probability pair, one v_and_b32 per two scores after the
-  // exponent (an out-of-window score may give +inf there, which the mask
-  // clears before the row sum), and row sums of the bf16 probabilities.
-  constexpr bool kAccMask = !(TALL && D == 64);
+  // chunk). Pipelined form: a 0 / -inf vector that every chunk's QK^T MFMAs
+  // start from (the first one's accumulator input), so the x window costs no
+  // instruction per score. Block form, which has no registers for that
+  // accumulator input: masks after the exponent (an out-of-window score may
+  // give +inf there, which the mask clears before the row sum), 0 / ~0 per
+  // score (the two key rows of a chunk share them) or, for the tall bricks, 0
+  // / 0xffff per bf16 half of each packed probability pair.
   f32x16 xbias;
-  uint32_t xpk[8];
+  uint32_t xpk[4], xm[8];
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
     const int p = (SEG == 16 ? ((i >> 2) & 1) * 8 : (i >> 2) * 8) + hf * 4 + (i & 3);
     const bool in = (unsigned)(p - sx) < (unsigned)kw;
     xbias[i] = in ? 0.0f : -__builtin_inff();
-    if (i & 1)
-      xpk[i >> 1] |= in ? 0xffff0000u : 0u;
-    else
-      xpk[i >> 1] = in ? 0xffffu : 0u;
+    if (i < 8) {
+      xm[i] = in ? ~0u : 0u;
+      if (i & 1)
+        xpk[i >> 1] |= in ? 0xffff0000u : 0u;
+      else
+        xpk[i >> 1] = in ? 0xffffu : 0u;
+    }
   }
-  const f32x16 s_init = kAccMask ? xbias : f32x16{};
+  const f32x16 s_init = C::kBlock ? f32x16{} : xbias;
 
   const int64_t tok_stride = (int64_t)a.NH * D;
   const int64_t head_off = (int64_t)uniform_u64((uint64_t)((int64_t)b * T * Hs * W * tok_stride + (int64_t)head * D));
   const bf16* qg = (const bf16*)a.q + head_off;
-  const bf16* kg = (const bf16*)a.k + head_off;
-  const bf16* vg = (const bf16*)a.v + head_off;
+  const uint64_t kg = uniform_u64((uint64_t)(uintptr_t)((const bf16*)a.k + head_off));
+  const uint64_t vg = uniform_u64((uint64_t)(uintptr_t)((const bf16*)a.v + head_off));
   bf16* og = (bf16*)a.o + head_off;
   auto token = [&](int tt, int yy, int xx) -> int64_t { return ((int64_t)tt * Hs + yy) * W + xx; };
 
@@ -586,7 +613,7 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
   int dma_dst[C::kCopiesPerWave], dma_row[C::kCopiesPerWave];
 #pragma unroll
   for (int p = 0; p < C::kCopiesPerWave; ++p) {
-    const int i = min(wave + C::kWaves * p, C::kCopies - 1);
+    const int i = min(wave % C::kCopyWaves + C::kCopyWaves * p, C::kCopies - 1);
     const int g = i % kGroups;
     const int half = g / kGroupsPerHalf;
     const int pos = C::kKeysPerCopy * (g % kGroupsPerHalf) + srow;
@@ -595,16 +622,15 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
     dma_voff[p] =
         (uint32_t)((int64_t)min(X_lo + pos, W - 1) * tok_stride + half * 64 + ((scol ^ half_swizzle(pos)) * 8)) * 2u;
   }
-  // Box rows are walked with cursors (row index, its y in the box, its token
-  // offset) that advance one row at a time and stop at the last row, so no
-  // step divides by NY.
+  // Box rows are walked with a cursor (its y and plane in the box, its row
+  // t * Hs + y of the grid) that advances one row at a time, so no step
+  // divides by NY. Past the last row it wraps to the box's first plane: those
+  // rows are copied but masked (their index is not below nrows).
   struct Cursor {
-    int r, yr, tr;
-    int64_t tok;
+    int yr, tr, row;
   };
-  const int64_t row_step = (int64_t)W * tok_stride;             // next y
-  const int64_t plane_jump = (int64_t)(Hs - NY) * W * tok_stride;  // last y of a plane -> first y of the next
-  const int64_t tok0 = ((int64_t)t_lo * Hs + Y_lo) * W * tok_stride;  // the box's first row
+  const uint32_t row_bytes = (uint32_t)((int64_t)W * tok_stride * 2);  // below 2^31 (checked on the host)
+  const int row0 = t_lo * Hs + Y_lo;                                   // the box's first row
   // Deep t windows (the t-plane-first brick order) walk their box planes
   // from the one whose t is a multiple of NT, wrapping round: bricks whose
   // boxes share a plane then read it in the same phase of their walks, while
@@ -616,43 +642,33 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
   // The cursor is wave-uniform; moving it through readfirstlane keeps its
   // arithmetic on the scalar unit (left to itself the compiler walked it in
   // 64-bit vector registers: ~60 VALU instructions per step).
+  const int plane_step = Hs - NY + 1;  // last y of a plane -> first y of the next
   auto advance = [&](Cursor& c) {
-    if (c.r + 1 < nrows) {
-      ++c.r;
-      c.tok += row_step;
-      if (++c.yr == NY) {
-        c.yr = 0;
-        if (c.tr + 1 == NT) {  // (a phase walk's wrap to the box's first plane)
-          c.tr = 0;
-          c.tok = tok0;
-        } else {
-          ++c.tr;
-          c.tok += plane_jump;
-        }
-      }
-    }
-    c.r = __builtin_amdgcn_readfirstlane(c.r);
+    const bool last_y = c.yr + 1 == NY, wrap = last_y && c.tr + 1 == NT;
+    c.row = wrap ? row0 : c.row + (last_y ? plane_step : 1);
+    c.tr = wrap ? 0 : c.tr + (last_y ? 1 : 0);
+    c.yr = last_y ? 0 : c.yr + 1;
     c.yr = __builtin_amdgcn_readfirstlane(c.yr);
     c.tr = __builtin_amdgcn_readfirstlane(c.tr);
-    c.tok = (int64_t)uniform_u64((uint64_t)c.tok);
+    c.row = __builtin_amdgcn_readfirstlane(c.row);
   };
-  const Cursor first = {0, 0, p0, tok0 + (int64_t)p0 * (W * (int64_t)Hs) * tok_stride};
-  // The key rows of one step (their token offsets and y in the box), taken
+  const Cursor first = {0, p0, row0 + p0 * Hs};
+  // The key rows of one step (their grid rows and places in the box), taken
   // from the cursor, which moves on by kRows rows. K walks the rows; V and
-  // the window mask use each step's record two steps later, so only one
+  // the window mask use each step's record in later steps, so only one
   // cursor runs (the scalar unit is shared by the CU's 8-16 waves).
   struct StepRows {
-    int64_t tok0, tok1;
+    int row0, row1;
     int yr0, yr1;
     int tr0, tr1;  // (deep bricks: the rows' planes in the box)
   };
   auto next_rows = [&](Cursor& c) -> StepRows {
     StepRows rr;
-    rr.tok0 = c.tok;
+    rr.row0 = c.row;
     rr.yr0 = c.yr;
     rr.tr0 = c.tr;
     advance(c);
-    rr.tok1 = C::kRows == 2 ? c.tok : rr.tok0;
+    rr.row1 = C::kRows == 2 ? c.row : rr.row0;
     rr.yr1 = C::kRows == 2 ? c.yr : rr.yr0;
     rr.tr1 = C::kRows == 2 ? c.tr : rr.tr0;
     if (C::kRows == 2) advance(c);
@@ -662,13 +678,18 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
   // not divide evenly over the waves, the waves below kExtraWaves issue one
   // more. (Making that a compile-time tag of the key loop, as IN below is,
   // made the 8-wave tall kernel spill.)
-  constexpr int kExtraWaves = C::kCopies % C::kWaves;
-  const bool extra = kExtraWaves == 0 || wave < kExtraWaves;  // wave-uniform
-  auto issue = [&](const bf16* base, int slot_off, const StepRows& rr) {
+  constexpr int kExtraWaves = C::kCopies % C::kCopyWaves;
+  const bool extra = kExtraWaves == 0 || wave % C::kCopyWaves < kExtraWaves;  // wave-uniform
+  const bool copier = C::kCopyWaves == C::kWaves || wave < C::kCopyWaves;      // wave-uniform
+  auto copy_row = [&](uint64_t base, int slot_off, const StepRows& rr, int p) __attribute__((always_inline)) {
+    if (kExtraWaves == 0 || p + 1 < C::kCopiesPerWave || extra) {
+      const uint32_t row = (uint32_t)(dma_row[p] ? rr.row1 : rr.row0);
+      lds_dma16_buf(raw_rsrc_u64(base + (uint64_t)row * row_bytes), dma_voff[p], lds_base + slot_off + dma_dst[p]);
+    }
+  };
+  auto issue = [&](uint64_t base, int slot_off, const StepRows& rr) {
 #pragma unroll
-    for (int p = 0; p < C::kCopiesPerWave; ++p)
-      if (kExtraWaves == 0 || p + 1 < C::kCopiesPerWave || extra)
-        lds_dma16_buf(raw_rsrc(base + (dma_row[p] ? rr.tok1 : rr.tok0)), dma_voff[p], lds_base + slot_off + dma_dst[p]);
+    for (int p = 0; p < C::kCopiesPerWave; ++p) copy_row(base, slot_off, rr, p);
   };
   using True = std::integral_constant<bool, true>;
   using False = std::integral_constant<bool, false>;
@@ -718,16 +739,22 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
 #pragma unroll
   for (int db = 0; db < kDB; ++db) O[db] = f32x16{};
   float m_run = kNegBig, l_run = 0.f;
-  const float c2 = a.scale * kLog2e;
+  const float c2 = uniform_f32(a.scale * kLog2e);
 
-  // ---- prologue: K of steps 0 and 1 in flight, V slot 1 zeroed (it stands
-  // in for the V of step -1, paired with P = 0), S = QK^T of chunk 0.
+  // ---- prologue: K of steps 0 and 1 in flight and, block form, V of step 0
+  // (pipelined form: V slot 1 zeroed, which stands in for the V of step -1,
+  // paired with P = 0), S = QK^T of chunk 0.
   Cursor kcur = first;  // rows of the next K step to issue
   StepRows rows_even = next_rows(kcur), rows_odd = next_rows(kcur);  // steps 0 and 1
-  issue(kg, C::kK, rows_even);
-  issue(kg, C::kK + C::kSlot, rows_odd);
-  for (int off = threadIdx.x * 16; off < C::kSlot; off += C::kThreads * 16)
-    *(VX_LDS u32x4*)(lds + C::kV + C::kSlot + off) = u32x4{0, 0, 0, 0};
+  if (copier) {
+    issue(kg, C::kK, rows_even);
+    issue(kg, C::kK + C::kSlot, rows_odd);
+    if (C::kBlock) issue(vg, C::kV, rows_even);
+  }
+  if constexpr (!C::kBlock) {
+    for (int off = threadIdx.x * 16; off < C::kSlot; off += C::kThreads * 16)
+      *(VX_LDS u32x4*)(lds + C::kV + C::kSlot + off) = u32x4{0, 0, 0, 0};
+  }
   // q preparation while the first key rows land (its loads overlap theirs)
   if (a.q_prep != 0) prep_q(qr, hf, token(tqc, yqc, xqc), tqc, yqc, xqc, a);
   wait_vmem<0>();
@@ -737,27 +764,15 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
   for (int ds = 0; ds < C::kQK; ++ds) S = mfma32x32x16(kfrag(lds + C::kK, ds), qr[ds], S);
   bf16x8 Pp[2] = {bf16x8{}, bf16x8{}};
 
-  // One step: consumes S (scores of chunk s) and Pp (probabilities of chunk
-  // s-1), produces Sn (scores of chunk s+1) and P (probabilities of chunk s).
-  // rr: the rows of step s on entry (their K was issued two steps ago), the
-  // rows of step s + 2 on return. IN (compile-time, so that the loop carries
-  // no per-step test of it): some query of this wave lies inside the grid.
-  // t-stacked bricks: whether some row of chunk c (rows r) lies in this
-  // wave's t window (st is the wave's first plane in the box: its lanes
-  // share one t plane)
-  const int st_w = C::kTStack ? uni(st) : 0;
-  auto chunk_active = [&](const StepRows& r, int c) -> bool {
-    if constexpr (!C::kTStack) return true;
-    const int r0 = c * C::kRows;
-    return (r0 < nrows && (unsigned)(r.tr0 - st_w) < (unsigned)kt) ||
-           (r0 + 1 < nrows && (unsigned)(r.tr1 - st_w) < (unsigned)kt);
-  };
+  // One pipelined step: consumes S (scores of chunk s) and Pp (probabilities
+  // of chunk s-1), produces Sn (scores of chunk s+1) and P (probabilities of
+  // chunk s). rr: the rows of step s on entry (their K was issued two steps
+  // ago), the rows of step s + 2 on return. IN (compile-time, so that the loop
+  // carries no per-step test of it): some query of this wave lies inside the
+  // grid.
   auto step = [&](auto in_tag, const int s, f32x16& S, f32x16& Sn, const bf16x8 (&Pp)[2], bf16x8 (&P)[2],
-                  StepRows& rr, const StepRows& rn, bool& act_prev) __attribute__((always_inline)) {
+                  StepRows& rr) __attribute__((always_inline)) {
     constexpr bool IN = decltype(in_tag)::value;
-    // (t-stacked bricks) chunk s's rows are rr's on entry, chunk s+1's rn's
-    const bool act_cur = chunk_active(rr, s), act_next = chunk_active(rn, s + 1);
-    const bool idle = C::kTStack && !act_prev && !act_cur && !act_next;
     // The previous step's copies (K of s+1, V of s-1) have landed once this
     // wave has none outstanding; the barrier publishes everyone's and frees
     // K slot s%2 (K of s, read last step) and V slot s%2 (V of s-2).
@@ -779,33 +794,26 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
     // matrix and softmax work does not queue behind its copies (a wave issues
     // in order, and the CU's load path takes each 1 KiB copy in ~16 cycles).
     auto copy = [&](int j) __attribute__((always_inline)) {
-      const bool isv = j < C::kCopiesPerWave;
-      const int p = isv ? j : j - C::kCopiesPerWave;
-      if (kExtraWaves == 0 || p + 1 < C::kCopiesPerWave || extra) {
-        const StepRows& r = isv ? cur : rr;
-        lds_dma16_buf(raw_rsrc((isv ? vg : kg) + (dma_row[p] ? r.tok1 : r.tok0)), dma_voff[p],
-                      lds_base + (isv ? C::kV : C::kK) + (s & 1) * C::kSlot + dma_dst[p]);
-      }
+      if (j < C::kCopiesPerWave)
+        copy_row(vg, C::kV + (s & 1) * C::kSlot, cur, j);
+      else
+        copy_row(kg, C::kK + (s & 1) * C::kSlot, rr, j - C::kCopiesPerWave);
     };
     constexpr int kStepCopies = 2 * C::kCopiesPerWave;
-    static_assert(kStepCopies <= C::kSlots, "one copy per MFMA slot at most");
+    static_assert(C::kBlock || kStepCopies <= C::kSlots, "one copy per MFMA slot at most");
 
     const VX_LDS unsigned char* kb = lds + C::kK + ((s + 1) & 1) * C::kSlot;  // K of chunk s+1
     const VX_LDS unsigned char* vb = lds + C::kV + ((s + 1) & 1) * C::kSlot;  // V of chunk s-1
     // (IN is the tag's value; the 1 x 4 x 32 bricks pass the runtime flag
     // instead, one loop for all waves: their two loops measured ~1 % slower
     // at the (3,7,7) config, whose x edge holds waves without queries)
-    if (!(IN && (TALL || wave_in)) || idle) {
-      // no query of this wave is inside the grid (the ragged x or y edge),
-      // or (t-stacked bricks) none of chunks s-1, s, s+1 has a row in its t
-      // window: it only copies its share of the rows. An idle step's chunk
-      // s+1 scores start from the x window alone (no row of it counts).
+    if (!(IN && (TALL || wave_in))) {
+      // no query of this wave is inside the grid (the ragged x or y edge): it
+      // only copies its share of the rows
 #pragma unroll
       for (int j = 0; j < kStepCopies; ++j) copy(j);
       P[0] = bf16x8{};
       P[1] = bf16x8{};
-      if (idle) Sn = s_init;
-      act_prev = act_cur;
       return;
     }
     // PV fragment f < kPV: key half j = f / kDB, d block f % kDB; then QK^T.
@@ -816,7 +824,6 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
     // exponent offset per key row: -m_run, or -inf for a row outside the y
     // window (exp2 then gives 0)
     const float mrow[2] = {row_ok[0] ? -m_run : -__builtin_inff(), row_ok[1] ? -m_run : -__builtin_inff()};
-    const bf16x2 one2 = {(bf16)1.0f, (bf16)1.0f};
     float l_tile = 0.f;
     bf16x8 fr[C::kSlots];
     float pf[16];
@@ -830,63 +837,23 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
     // kSlots slots: slot i issues one MFMA (i < kPV: PV(s-1), else QK^T(s+1)),
     // the LDS read two slots ahead, and the mask + exp of kScoresPerSlot
     // scores of chunk s.
-    if constexpr (TALL && D == 64) {
-      // tall bricks at head dim 64: the MFMA block, then the masking and
-      // softmax block, so the two waves of a SIMD alternate between them
-      // (+1.6 % at the (11, 11, 11) window; at head dim 128 and in the
-      // 1 x 4 x 32 bricks the per-slot interleave measured as fast or faster)
 #pragma unroll
-      for (int i = 0; i < C::kSlots; ++i) {
-        if (i + 2 < C::kSlots) fr[i + 2] = frag(i + 2);
-        if (i < C::kPV)
-          O[i % kDB] = mfma32x32x16(fr[i], Pp[i / kDB], O[i % kDB]);
-        else
-          Sn = mfma32x32x16(fr[i], qr[i - C::kPV], Sn);
-        if (i < kStepCopies) copy(i);
-        __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < C::kSlots; ++i) {
+      if (i + 2 < C::kSlots) fr[i + 2] = frag(i + 2);
+      if (i < C::kPV)
+        O[i % kDB] = mfma32x32x16(fr[i], Pp[i / kDB], O[i % kDB]);
+      else
+        Sn = mfma32x32x16(fr[i], qr[i - C::kPV], Sn);
+      if (i < kStepCopies) copy(i);
+#pragma unroll
+      for (int u = 0; u < C::kScoresPerSlot; ++u) {
+        const int e = i * C::kScoresPerSlot + u;
+        pf[e] = fast_exp2(__builtin_fmaf(S[e], c2, mrow[e >> 3]));
+        if (e & 1) pk[e >> 1] = bf16x2{(bf16)pf[e - 1], (bf16)pf[e]};
       }
-#pragma unroll
-      for (int g = 0; g < 2; ++g) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) pf[8 * g + i] = __builtin_fmaf(S[8 * g + i], c2, mrow[g]);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) pf[8 * g + i] = fast_exp2(pf[8 * g + i]);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          // (the tall D = 64 block: kAccMask is false, the x window is xpk)
-          const bf16x2 pr = bf16x2{(bf16)pf[8 * g + 2 * i], (bf16)pf[8 * g + 2 * i + 1]};
-          pk[4 * g + i] = __builtin_bit_cast(bf16x2, __builtin_bit_cast(uint32_t, pr) & xpk[4 * g + i]);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      // row sums of the bf16 probabilities (dot2 with 1, 1): fp32 sums of
-      // the unrounded ones keep pf live past the packing, 5 spills at 128 VGPRs
-      l_tile = 0.f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) l_tile = __builtin_amdgcn_fdot2_f32_bf16(pk[i], one2, l_tile, false);
       __builtin_amdgcn_sched_barrier(0);
-    } else {
-#pragma unroll
-      for (int i = 0; i < C::kSlots; ++i) {
-        if (i + 2 < C::kSlots) fr[i + 2] = frag(i + 2);
-        if (i < C::kPV)
-          O[i % kDB] = mfma32x32x16(fr[i], Pp[i / kDB], O[i % kDB]);
-        else
-          Sn = mfma32x32x16(fr[i], qr[i - C::kPV], Sn);
-        if (i < kStepCopies) copy(i);
-#pragma unroll
-        for (int u = 0; u < C::kScoresPerSlot; ++u) {
-          const int e = i * C::kScoresPerSlot + u;
-          static_assert(kAccMask, "the per-slot form runs with the accumulator-start x window");
-          pf[e] = fast_exp2(__builtin_fmaf(S[e], c2, mrow[e >> 3]));
-          if (e & 1) pk[e >> 1] = bf16x2{(bf16)pf[e - 1], (bf16)pf[e]};
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      l_tile = sum16(pf);
     }
+    l_tile = sum16(pf);
 #pragma unroll
     for (int j = 0; j < 2; ++j)
       P[j] = __builtin_shufflevector(__builtin_shufflevector(pk[4 * j], pk[4 * j + 1], 0, 1, 2, 3),
@@ -898,77 +865,222 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
     // always lands here) -> raise m_run to the chunk max, rescale O and l and
     // recompute the chunk's probabilities.
     if (__builtin_amdgcn_ballot_w64(l_tile > kSumLimit || is_nan_bits(l_tile)) != 0) {
-      // (with kAccMask the scores carry the x window; without it xpk holds it)
+      // (the scores carry the x window)
       float mx = -__builtin_inff();
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const bool in = row_ok[i >> 3] && (kAccMask || ((xpk[i >> 1] >> ((i & 1) * 16)) & 1u) != 0);
-        mx = __builtin_fmaxf(mx, in ? S[i] : -__builtin_inff());
-      }
+      for (int i = 0; i < 16; ++i) mx = __builtin_fmaxf(mx, row_ok[i >> 3] ? S[i] : -__builtin_inff());
       const float mn = __builtin_fmaxf(m_run, halves_max(mx) * c2);
       const float alpha = fast_exp2(m_run - mn);
       m_run = mn;
       l_run *= alpha;
 #pragma unroll
       for (int db = 0; db < kDB; ++db) O[db] *= alpha;
-      if constexpr (kAccMask) {
-        const float mr[2] = {row_ok[0] ? -mn : -__builtin_inff(), row_ok[1] ? -mn : -__builtin_inff()};
+      const float mr[2] = {row_ok[0] ? -mn : -__builtin_inff(), row_ok[1] ? -mn : -__builtin_inff()};
 #pragma unroll
-        for (int e = 0; e < 16; ++e) pf[e] = fast_exp2(__builtin_fmaf(S[e], c2, mr[e >> 3]));
+      for (int e = 0; e < 16; ++e) pf[e] = fast_exp2(__builtin_fmaf(S[e], c2, mr[e >> 3]));
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          bf16x8 pv;
+      for (int j = 0; j < 2; ++j) {
+        bf16x8 pv;
 #pragma unroll
-          for (int r = 0; r < 8; ++r) pv[r] = (bf16)pf[8 * j + r];
-          P[j] = pv;
-        }
-        l_tile = sum16(pf);
-      } else {
-        const float mr[2] = {row_ok[0] ? -mn : -__builtin_inff(), row_ok[1] ? -mn : -__builtin_inff()};
-        l_tile = 0.f;
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          bf16x8 pv;
-#pragma unroll
-          for (int r = 0; r < 8; ++r) pv[r] = (bf16)fast_exp2(__builtin_fmaf(S[8 * j + r], c2, mr[j]));
-          u32x4 w = __builtin_bit_cast(u32x4, pv);
-#pragma unroll
-          for (int q = 0; q < 4; ++q) w[q] &= xpk[4 * j + q];
-          pv = __builtin_bit_cast(bf16x8, w);
-          P[j] = pv;
-          l_tile = sum8(pv, l_tile);
-        }
+        for (int r = 0; r < 8; ++r) pv[r] = (bf16)pf[8 * j + r];
+        P[j] = pv;
       }
+      l_tile = sum16(pf);
     }
     l_run += l_tile;
-    act_prev = act_cur;
   };
 
-  f32x16 S2;
-  bf16x8 P2[2];
-  // the key loop; the tall bricks run one copy for the waves with queries
-  // and one for the others
-  bool act_prev = false;  // chunk -1 (none)
-  auto key_loop = [&](auto in_tag) __attribute__((always_inline)) {
-    int s = 0;
-    for (; s + 1 < n_steps; s += 2) {
-      step(in_tag, s, S, S2, Pp, P2, rows_even, rows_odd, act_prev);
-      step(in_tag, s + 1, S2, S, P2, Pp, rows_odd, rows_even, act_prev);
+  // ---- block form.
+  // Whether some row of chunk c (rows r) lies in this wave's t window
+  // (t-stacked bricks: st is the wave's first plane in the box, its lanes
+  // share one t plane) or in the union of its y windows (quad bricks).
+  const int st_w = TSTACK ? uni(st) : 0;
+  const int sy_w = QUAD ? uni(window_start(min(yw, Hs - 1), Hs, kh) - Y_lo) : 0;
+  const int ny_w = QUAD ? uni(window_start(min(yw + C::kQY - 1, Hs - 1), Hs, kh) - Y_lo) + kh - sy_w : 0;
+  auto chunk_active = [&](const StepRows& r, int c) -> bool {
+    if constexpr (!C::kSkip) return true;
+    const int r0 = c * C::kRows;
+    const bool in0 = QUAD ? (unsigned)(r.yr0 - sy_w) < (unsigned)ny_w : (unsigned)(r.tr0 - st_w) < (unsigned)kt;
+    const bool in1 = QUAD ? (unsigned)(r.yr1 - sy_w) < (unsigned)ny_w : (unsigned)(r.tr1 - st_w) < (unsigned)kt;
+    return (r0 < nrows && in0) || (r0 + 1 < nrows && in1);
+  };
+  // The probabilities of the chunk in S against the exponent offsets m0, m1 of
+  // its two key rows (-m_run, or -inf for a row outside the lane's y or t
+  // window): exponent, x window, bf16 packing into Pp; returns their sum.
+  const bf16x2 one2 = {(bf16)1.0f, (bf16)1.0f};
+  auto chunk_probs = [&](float m0, float m1) __attribute__((always_inline)) -> float {
+    float l = 0.f;
+    bf16x2 pk[8];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      float pf[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) pf[i] = __builtin_fmaf(S[8 * j + i], c2, j == 0 ? m0 : m1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) pf[i] = fast_exp2(pf[i]);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (C::kSumF32) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) pf[i] = __uint_as_float(__float_as_uint(pf[i]) & xm[i]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) pk[4 * j + i] = bf16x2{(bf16)pf[2 * i], (bf16)pf[2 * i + 1]};
+        l += ((pf[0] + pf[1]) + (pf[2] + pf[3])) + ((pf[4] + pf[5]) + (pf[6] + pf[7]));
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const bf16x2 pr = bf16x2{(bf16)pf[2 * i], (bf16)pf[2 * i + 1]};
+          pk[4 * j + i] = __builtin_bit_cast(bf16x2, __builtin_bit_cast(uint32_t, pr) & xpk[i]);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
-    if (s < n_steps) {
-      step(in_tag, s, S, S2, Pp, P2, rows_even, rows_odd, act_prev);
-      Pp[0] = P2[0];
-      Pp[1] = P2[1];
+    if constexpr (!C::kSumF32) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) l = __builtin_amdgcn_fdot2_f32_bf16(pk[i], one2, l, false);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      Pp[j] = __builtin_shufflevector(__builtin_shufflevector(pk[4 * j], pk[4 * j + 1], 0, 1, 2, 3),
+                                      __builtin_shufflevector(pk[4 * j + 2], pk[4 * j + 3], 0, 1, 2, 3),
+                                      0, 1, 2, 3, 4, 5, 6, 7);
+    __builtin_amdgcn_sched_barrier(0);
+    return l;
+  };
+  // One block step: the softmax of chunk s (scores in S), then PV(s) and
+  // QK^T(s+1) into S. rr: the rows of step s on entry, of step s + 2 on
+  // return; rn: those of step s + 1. COPY: this wave issues copies.
+  auto block_step = [&](auto in_tag, auto copy_tag, const int s, StepRows& rr,
+                        const StepRows& rn) __attribute__((always_inline)) {
+    constexpr bool IN = decltype(in_tag)::value, COPY = decltype(copy_tag)::value;
+    const bool in = IN && (TALL || wave_in);
+    if (C::kHalfStep) __syncthreads();
+    const bool act_cur = in && chunk_active(rr, s), act_next = in && chunk_active(rn, s + 1);
+    if (act_cur) {
+      bool row_ok[2];
+#pragma unroll
+      for (int h2 = 0; h2 < 2; ++h2)
+        row_ok[h2] = s * 2 + h2 < nrows && (unsigned)((h2 == 0 ? rr.yr0 : rr.yr1) - sy) < (unsigned)kh &&
+                     (C::kQT == 1 || (unsigned)((h2 == 0 ? rr.tr0 : rr.tr1) - st) < (unsigned)kt);
+      // (wave priority 1 in the softmax, ahead of the other workgroups' waves
+      // on the SIMD: 5x22x40 NH=16 (3,7,7) 24.1 -> 23.0 us; on the MFMA block
+      // instead 24.5 us, and either form slows the half-step bricks by 1-2 %)
+      if (!C::kHalfStep) __builtin_amdgcn_s_setprio(1);
+      float l_tile = chunk_probs(row_ok[0] ? -m_run : -__builtin_inff(), row_ok[1] ? -m_run : -__builtin_inff());
+      // rare (the pipelined step's rule): raise m_run to the chunk max,
+      // rescale O and l and recompute the chunk's probabilities
+      if (__builtin_amdgcn_ballot_w64(l_tile > kSumLimit || is_nan_bits(l_tile)) != 0) {
+        float mx = -__builtin_inff();
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const uint32_t xin = C::kSumF32 ? xm[i & 7] : (xpk[(i & 7) >> 1] >> ((i & 1) * 16)) & 1u;
+          mx = __builtin_fmaxf(mx, row_ok[i >> 3] && xin != 0 ? S[i] : -__builtin_inff());
+        }
+        const float mn = __builtin_fmaxf(m_run, halves_max(mx) * c2);
+        const float alpha = fast_exp2(m_run - mn);
+        m_run = mn;
+        l_run *= alpha;
+#pragma unroll
+        for (int db = 0; db < kDB; ++db) O[db] *= alpha;
+        l_tile = chunk_probs(row_ok[0] ? -mn : -__builtin_inff(), row_ok[1] ? -mn : -__builtin_inff());
+      }
+      l_run += l_tile;
+      if (!C::kHalfStep) __builtin_amdgcn_s_setprio(0);
+    }
+    // K of s+1 and V of s have landed once this wave's copies of the last
+    // step have; the barrier publishes everyone's and frees the slots of K
+    // of s and V of s-1, read in the last step's MFMAs (with half steps, by
+    // waves 4-7 between the last two barriers).
+    if (COPY) wait_vmem<0>();
+    __syncthreads();
+    const StepRows cur = rn;
+    rr = next_rows(kcur);
+    // copies: V of step s + 1, then K of step s + 2, one per MFMA slot
+    auto copy = [&](int j) __attribute__((always_inline)) {
+      if (j < C::kCopiesPerWave)
+        copy_row(vg, C::kV + ((s + 1) & 1) * C::kSlot, cur, j);
+      else
+        copy_row(kg, C::kK + (s & 1) * C::kSlot, rr, j - C::kCopiesPerWave);
+    };
+    constexpr int kStepCopies = 2 * C::kCopiesPerWave;
+    static_assert(!C::kBlock || kStepCopies <= C::kSlots, "one copy per MFMA slot at most");
+    if (!act_cur && !act_next) {
+      // no query of this wave in the grid, or no row of either chunk in its
+      // window: it only copies (its next chunk's scores are not used)
+#pragma unroll
+      for (int j = 0; j < kStepCopies; ++j)
+        if (COPY) copy(j);
+      return;
+    }
+    if (C::kSkip && !act_cur) Pp[0] = Pp[1] = bf16x8{};
+    const VX_LDS unsigned char* kb = lds + C::kK + ((s + 1) & 1) * C::kSlot;  // K of chunk s+1
+    const VX_LDS unsigned char* vb = lds + C::kV + (s & 1) * C::kSlot;        // V of chunk s
+    auto frag = [&](int i) -> bf16x8 {
+      return i < C::kPV ? vfrag(vb, i / kDB, i % kDB) : kfrag(kb, i - C::kPV);
+    };
+    bf16x8 fr[C::kSlots];
+    fr[0] = frag(0);
+    fr[1] = frag(1);
+    S = f32x16{};
+#pragma unroll
+    for (int i = 0; i < C::kSlots; ++i) {
+      if (i + 2 < C::kSlots) fr[i + 2] = frag(i + 2);
+      if (i < C::kPV)
+        O[i % kDB] = mfma32x32x16(fr[i], Pp[i / kDB], O[i % kDB]);
+      else
+        S = mfma32x32x16(fr[i], qr[i - C::kPV], S);
+      if (COPY && i < kStepCopies) copy(i);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
-  if (!TALL || wave_in)
-    key_loop(True{});
-  else
-    key_loop(False{});
-  // ---- PV of the last chunk (its V was issued by the last step).
-  wait_vmem<0>();
-  __syncthreads();
-  {
+
+  // ---- the key loop; the tall bricks run one copy for the waves with
+  // queries and one for the others
+  if constexpr (C::kBlock) {
+    auto block_loop = [&](auto in_tag, auto copy_tag) __attribute__((always_inline)) {
+      int s = 0;
+      for (; s + 1 < n_steps; s += 2) {
+        block_step(in_tag, copy_tag, s, rows_even, rows_odd);
+        block_step(in_tag, copy_tag, s + 1, rows_odd, rows_even);
+      }
+      if (s < n_steps) block_step(in_tag, copy_tag, s, rows_even, rows_odd);
+    };
+    if (C::kHalfStep && !copier) {
+      __syncthreads();  // half a step behind the copying waves
+      if (wave_in)
+        block_loop(True{}, False{});
+      else
+        block_loop(False{}, False{});
+    } else {
+      if (!TALL || wave_in)
+        block_loop(True{}, True{});
+      else
+        block_loop(False{}, True{});
+      if (C::kHalfStep) __syncthreads();  // the other waves' last one
+      wait_vmem<0>();  // (the last steps' copies, of rows past the box, still write to LDS)
+    }
+  } else {
+    f32x16 S2;
+    bf16x8 P2[2];
+    auto key_loop = [&](auto in_tag) __attribute__((always_inline)) {
+      int s = 0;
+      for (; s + 1 < n_steps; s += 2) {
+        step(in_tag, s, S, S2, Pp, P2, rows_even);
+        step(in_tag, s + 1, S2, S, P2, Pp, rows_odd);
+      }
+      if (s < n_steps) {
+        step(in_tag, s, S, S2, Pp, P2, rows_even);
+        Pp[0] = P2[0];
+        Pp[1] = P2[1];
+      }
+    };
+    if (!TALL || wave_in)
+      key_loop(True{});
+    else
+      key_loop(False{});
+    // PV of the last chunk (its V was issued by the last step)
+    wait_vmem<0>();
+    __syncthreads();
     const VX_LDS unsigned char* vb = lds + C::kV + ((n_steps - 1) & 1) * C::kSlot;
 #pragma unroll
     for (int i = 0; i < C::kPV; ++i) O[i % kDB] = mfma32x32x16(vfrag(vb, i / kDB, i % kDB), Pp[i / kDB], O[i % kDB]);
@@ -976,27 +1088,35 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
 
   const float lt = halves_sum(l_run);
   const float inv = lt > 0.f ? 1.0f / lt : 0.f;
-  store_na_rows<kDB, C::kQX, C::kQY>(O, inv, og, tok_stride, tw, y0, xq0, T, Hs, W, lane);
+  store_na_rows<kDB, C::kQX, C::kQY>(O, inv, og, tok_stride, tw, yw, xq0, T, Hs, W, lane);
 }
 
-// Three waves per SIMD for the 32-key segments at head dim 64 (146 VGPRs,
-// three 32 KiB workgroups per CU): 33x88x160 NH=4 at a (5,5,21) window
-// 1.02 -> 0.94 ms. The 16-key form gained at 21x45x80 NH=24 (-9 %) but lost
-// at 33x88x160 NH=4 (+3.5 %) and keeps two.
+// Head dim 64: three waves per SIMD for the 32-key segments (three 32 KiB
+// workgroups per CU; 33x88x160 NH=4 at a (5,5,21) window 1.02 -> 0.94 ms),
+// four for the 16-key ones (block form, four 40 KiB workgroups).
 template <int SEG, int D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 && SEG == 32 ? 3 : 2,
-                                                                       D == 64 && SEG == 32 ? 3 : 2)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? (SEG == 32 ? 3 : 4) : 2,
+                                                                       D == 64 ? (SEG == 32 ? 3 : 4) : 2)))
 void na3d_pipe_kernel(const Na3dArgs a, int n_yb, int n_xb) {
-  na3d_pipe_body<SEG, D, false>(a, n_yb, n_xb);
+  __shared__ __attribute__((aligned(16))) unsigned char smem[PipeCfg<SEG, D>::kSmem];
+  na3d_pipe_body<SEG, D, false>(a, n_yb, n_xb, smem);
 }
 
 // Head dim 64: four waves per SIMD (at most 128 VGPRs; the workgroup's 32 KiB
 // of LDS allows four per CU), so that more workgroups cover each other's
 // per-step waits: 2.56 -> 2.31 ms at the (11, 11, 11) window on 33x88x160.
+// quad: the 2 x 2 waves of 4 y x 8 x (head dim 64, kw' <= 9).
 template <int D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : 2, D == 64 ? 4 : 2)))
-void na3d_tall_kernel(const Na3dArgs a, int n_yb, int n_xb) {
-  na3d_pipe_body<16, D, true>(a, n_yb, n_xb);
+void na3d_tall_kernel(const Na3dArgs a, int n_yb, int n_xb, int quad) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem[PipeCfg<16, D, true>::kSmem];
+  if constexpr (D == 64) {
+    if (quad) {
+      na3d_pipe_body<16, D, true, false, false, false, true>(a, n_yb, n_xb, smem);
+      return;
+    }
+  }
+  na3d_pipe_body<16, D, true>(a, n_yb, n_xb, smem);
 }
 
 // Head dim 64, grids whose width rounds up to the same multiple of 16 and 32
@@ -1005,7 +1125,8 @@ void na3d_tall_kernel(const Na3dArgs a, int n_yb, int n_xb) {
 template <int D>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void na3d_tall_wide_kernel(const Na3dArgs a, int n_yb, int n_xb) {
-  na3d_pipe_body<16, D, true, true>(a, n_yb, n_xb);
+  __shared__ __attribute__((aligned(16))) unsigned char smem[PipeCfg<16, D, true, true>::kSmem];
+  na3d_pipe_body<16, D, true, true>(a, n_yb, n_xb, smem);
 }
 
 // Head dim 64, deep t windows: the wide bricks two t planes deep (2 x 4 x 32,
@@ -1013,16 +1134,24 @@ void na3d_tall_wide_kernel(const Na3dArgs a, int n_yb, int n_xb) {
 template <int D>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void na3d_deep_kernel(const Na3dArgs a, int n_yb, int n_xb) {
-  na3d_pipe_body<16, D, true, true, true>(a, n_yb, n_xb);
+  __shared__ __attribute__((aligned(16))) unsigned char smem[PipeCfg<16, D, true, true, true>::kSmem];
+  na3d_pipe_body<16, D, true, true, true>(a, n_yb, n_xb, smem);
 }
 
 // Head dim 128, windows up to 9 wide and t windows of 2 and more: the
-// t-stacked 2 x 4 x 16 bricks, two workgroups of 48 KiB per CU.
+// t-stacked 2 x 4 x 16 bricks, three workgroups of 48 KiB per CU (168 VGPRs).
 template <int D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
 void na3d_tstack_kernel(const Na3dArgs a, int n_yb, int n_xb) {
-  na3d_pipe_body<16, D, false, false, false, true>(a, n_yb, n_xb);
+  __shared__ __attribute__((aligned(16))) unsigned char smem[PipeCfg<16, D, false, false, false, true>::kSmem];
+  na3d_pipe_body<16, D, false, false, false, true>(a, n_yb, n_xb, smem);
 }
+
+// Workgroups from which the tall bricks at head dim 64 with kw' <= 9 take the
+// 2 x 2 waves (12 per CU). Same box, (3,7,7) windows, 8 x 4 -> 4 x 8 waves:
+// 720 workgroups 24.1 -> 24.8 us, 1296 37.3 -> 39.6, 1680 46.2 -> 47.0, 2592
+// 68.2 -> 68.2, 15120 458 -> 425; 4080 at (5,9,9) 182 -> 170.
+constexpr int64_t kNaQuadMinGroups = 3072;
 
 }  // namespace
 
@@ -1035,10 +1164,11 @@ int launch_na3d_fwd(const Na3dArgs& a, void* stream, const char** launched) {
       const int n_xb = (a.W + 15) / 16;
       dim3 grid((unsigned)a.T * n_yb * n_xb, a.NH, a.B);
       if (a.D == 128) {
-        hipLaunchKernelGGL((na3d_tall_kernel<128>), grid, dim3(256), 0, st, a, n_yb, n_xb);
+        hipLaunchKernelGGL((na3d_tall_kernel<128>), grid, dim3(256), 0, st, a, n_yb, n_xb, 0);
         *launched = "na3d_tall_kernel<128>";
       } else {
-        hipLaunchKernelGGL((na3d_tall_kernel<64>), grid, dim3(256), 0, st, a, n_yb, n_xb);
+        const int quad = a.kw <= 9 && (int64_t)grid.x * grid.y * grid.z >= kNaQuadMinGroups;
+        hipLaunchKernelGGL((na3d_tall_kernel<64>), grid, dim3(256), 0, st, a, n_yb, n_xb, quad);
         *launched = "na3d_tall_kernel<64>";
       }
       return (int)hipGetLastError();
