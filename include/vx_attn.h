@@ -120,6 +120,36 @@ int32_t vx_flash_attn_noalloc_fwd(const void* q, const void* k, const void* v, v
                                   const int64_t* out_strides, float scale, void* stream);
 
 /*
+ * Key masks in the form the flash entry points take, in one launch: validity
+ * bytes (0 = masked) and fp32 biases of seq_k keys per batch item, read at any
+ * element strides {batch, key} (0 for broadcast dims), written to rows of
+ * round_up(seq_k, 64) keys, row_stride elements apart (a multiple of 64; the
+ * padding is invalid, its bias -inf), and kv_len[b] = the last key that is
+ * valid and whose bias is above -inf, plus 1 (0 if there is none). valid or
+ * bias may be NULL, and so may every output (a row output needs its input).
+ * The row outputs are 16-byte aligned.
+ * Serves the mask handling of src/vidax/core/attention.py:467-533 and
+ * src/vidax/models/hunyuan_video/common/dit_layers.py:183-186.
+ */
+int32_t vx_key_masks_fwd(const uint8_t* valid, const int64_t* valid_strides, const float* bias,
+                         const int64_t* bias_strides, int32_t batch, int32_t seq_k, int32_t* kv_len,
+                         uint8_t* valid_rows, float* bias_rows, int64_t row_stride, void* stream);
+
+/*
+ * A per-(query, key) bias in the form vx_flash_attn_bias_fwd takes, in one
+ * launch: out[b, h, q, k] = bias + (mask ? 0 : -inf), a contiguous
+ * (batch, num_heads, seq_q, round_up(seq_k, 64)) fp32 array, 16-byte aligned,
+ * whose padding is 0. bias (fp32) and mask (bytes, 0 = masked) are read at
+ * any element strides {batch, head, query, key} (0 for broadcast dims);
+ * either may be NULL. batch, num_heads and seq_q are the extents to write
+ * (1 for a dim both broadcast).
+ * Serves src/vidax/core/attention.py:282,533.
+ */
+int32_t vx_full_bias_fwd(const float* bias, const int64_t* bias_strides, const uint8_t* mask,
+                         const int64_t* mask_strides, int32_t batch, int32_t num_heads, int32_t seq_q, int32_t seq_k,
+                         float* out, void* stream);
+
+/*
  * Workspace bytes vx_flash_attn_ws_fwd uses for this shape on the current
  * device (0 when it does not split, or on failure). Head dim 64 or 128.
  */

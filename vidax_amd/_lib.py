@@ -45,6 +45,8 @@ EXPORTED_SYMBOLS = (
     "vx_flash_attn_split_plan",
     "vx_flash_attn_noalloc_fwd",
     "vx_debug_clock_stamp",
+    "vx_key_masks_fwd",
+    "vx_full_bias_fwd",
 )
 
 _lock = threading.Lock()
@@ -139,6 +141,10 @@ def lib() -> ctypes.CDLL:
                                                                ctypes.POINTER(_i64)]
             h.vx_debug_clock_stamp.restype = _i32
             h.vx_debug_clock_stamp.argtypes = [_p, _i32, ctypes.POINTER(_i32), _p]
+            h.vx_key_masks_fwd.restype = _i32
+            h.vx_key_masks_fwd.argtypes = [_p, _i64p, _p, _i64p, _i32, _i32, _p, _p, _p, _i64, _p]
+            h.vx_full_bias_fwd.restype = _i32
+            h.vx_full_bias_fwd.argtypes = [_p, _i64p, _p, _i64p, _i32, _i32, _i32, _i32, _p, _p]
             h.vx_last_launch.restype = ctypes.c_char_p
             h.vx_last_launch.argtypes = []
             _lib = h

@@ -63,48 +63,94 @@ def _aligned(t: torch.Tensor, max_seq_stride: Optional[int] = None) -> torch.Ten
     return t if ok else t.contiguous()
 
 
+def _strides(x: torch.Tensor, dims) -> ctypes.Array:
+    """Element strides of x's dims, 0 where the extent is 1 (broadcast)."""
+    return (ctypes.c_int64 * len(dims))(*[0 if x.shape[d] == 1 else x.stride(d) for d in dims])
+
+
+def _stream(dev) -> ctypes.c_void_p:
+    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+
+
+class _KeyMasks:
+    """Key masks as the kernels take them, from one launch (vx_key_masks_fwd):
+    validity bytes and fp32 biases in rows of round_up(Sk, 64) keys, padded
+    with invalid / -inf keys, and kv_len = last unmasked key + 1 per batch item
+    (0 if none). valid (B, Sk) bool and bias (B, Sk) fp32 may be views of any
+    strides; the addresses below point into `buf`."""
+
+    def __init__(self, valid: Optional[torch.Tensor], bias: Optional[torch.Tensor], want_len: bool,
+                 want_rows: bool = True):
+        x = valid if valid is not None else bias
+        B, Sk = x.shape
+        dev = x.device
+        self.stride = (Sk + 63) // 64 * 64
+        self.bias_off = (B * 4 + 15) // 16 * 16 if want_len else 0
+        self.valid_off = self.bias_off + (B * self.stride * 4 if want_rows and bias is not None else 0)
+        nbytes = self.valid_off + (B * self.stride if want_rows and valid is not None else 0)
+        self.buf = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        base = self.buf.data_ptr()
+        self.kv_len = base if want_len else None
+        self.bias = base + self.bias_off if want_rows and bias is not None else None
+        self.valid = base + self.valid_off if want_rows and valid is not None else None
+        with torch.cuda.device(dev):
+            _lib.raise_for(_lib.lib().vx_key_masks_fwd(
+                valid.data_ptr() if valid is not None else None, _strides(valid, (0, 1)) if valid is not None else None,
+                bias.data_ptr() if bias is not None else None, _strides(bias, (0, 1)) if bias is not None else None,
+                B, Sk, self.kv_len, self.valid, self.bias, self.stride, _stream(dev)))
+
+
 def _mask_rows(x: torch.Tensor, sk: int, dtype: torch.dtype, fill) -> torch.Tensor:
-    """(B, Sk) -> (B, round_up(Sk, 64)) contiguous copy in `dtype`, padded with `fill`
-    (the kernel stages the mask in whole 64-key tiles)."""
-    b = x.shape[0]
-    width = (sk + 63) // 64 * 64
-    out = torch.full((b, width), fill, dtype=dtype, device=x.device)
-    out[:, :sk] = x.to(dtype)
-    return out
+    """(B, Sk) validity (uint8, fill 0) or biases (float32, fill -inf) as the
+    key-mask rows of the kernels: (B, round_up(Sk, 64)) contiguous."""
+    if (dtype, fill) not in ((torch.uint8, 0), (torch.float32, float("-inf"))):
+        raise ValueError("key-mask rows are uint8 filled with 0 or float32 filled with -inf")
+    m = _KeyMasks(x.to(torch.bool) if dtype == torch.uint8 else None,
+                  x.to(torch.float32) if dtype == torch.float32 else None, want_len=False)
+    return m.buf.view(dtype).reshape(x.shape[0], m.stride)
 
 
 def _last_valid_plus_one(valid: torch.Tensor) -> torch.Tensor:
     """(B, Sk) bool -> int32 (B,) index of the last valid key + 1 (0 if none), on device."""
-    sk = valid.shape[-1]
-    pos = torch.arange(1, sk + 1, device=valid.device, dtype=torch.int32)
-    return (valid.to(torch.int32) * pos).amax(dim=-1).to(torch.int32).contiguous()
+    m = _KeyMasks(valid.to(torch.bool), None, want_len=True, want_rows=False)
+    return m.buf.view(torch.int32)[:valid.shape[0]]
 
 
-def _full_bias(bias, B: int, H: int, Sq: int, Sk: int, dev) -> Tuple[torch.Tensor, Tuple[int, int, int]]:
-    """A bias broadcastable to (B, H, Sq, Sk) -- every dim 1 or full, as
-    `jnp.broadcast_to` accepts (`src/vidax/core/attention.py:282,533`) -- as
-    the kernel reads it: fp32, keys contiguous, every query row readable for
-    round_up(Sk, 64) keys, 16-byte aligned, strides multiples of 4 (0 for
-    broadcast dims). A key dim of 1 is expanded; copies only when the given
-    tensor does not already have that form."""
-    x = torch.as_tensor(bias, device=dev)
-    while x.dim() < 4:
-        x = x.unsqueeze(0)
-    if x.dim() != 4 or any(x.shape[i] not in (1, n) for i, n in enumerate((B, H, Sq, Sk))):
-        raise ValueError(f"bias of shape {tuple(bias.shape)} is not broadcastable to (B, H, Sq, Sk) = "
-                         f"({B}, {H}, {Sq}, {Sk})")
-    x = x.to(torch.float32)
-    if x.shape[3] != Sk:
-        x = x.expand(x.shape[0], x.shape[1], x.shape[2], Sk)
+def _full_bias(bias, B: int, H: int, Sq: int, Sk: int, dev, mask=None) -> Tuple[torch.Tensor, Tuple[int, int, int]]:
+    """A bias, a boolean mask (False: -inf) or both, each broadcastable to
+    (B, H, Sq, Sk) -- every dim 1 or full, as `jnp.broadcast_to` accepts
+    (`src/vidax/core/attention.py:282,533`) -- as the kernel reads it: fp32,
+    keys contiguous, every query row readable for round_up(Sk, 64) keys,
+    16-byte aligned, strides multiples of 4 (0 for broadcast dims). A bias
+    that has that form already is passed as it is; anything else is written in
+    one launch (vx_full_bias_fwd)."""
+    def expand(t, what):
+        x = torch.as_tensor(t, device=dev)
+        while x.dim() < 4:
+            x = x.unsqueeze(0)
+        if x.dim() != 4 or any(x.shape[i] not in (1, n) for i, n in enumerate((B, H, Sq, Sk))):
+            raise ValueError(f"{what} of shape {tuple(t.shape)} is not broadcastable to (B, H, Sq, Sk) = "
+                             f"({B}, {H}, {Sq}, {Sk})")
+        return x
+
+    x = expand(bias, "bias").to(torch.float32) if bias is not None else None
+    m = expand(mask, "mask").to(torch.bool) if mask is not None else None
     width = (Sk + 63) // 64 * 64
-    ok = (x.stride(3) == 1 and Sk == width and x.data_ptr() % 16 == 0 and
-          all(x.stride(i) % 4 == 0 for i in range(3)))
-    if not ok:
-        pad = torch.zeros(x.shape[:3] + (width,), dtype=torch.float32, device=dev)
-        pad[..., :Sk] = x
-        x = pad
-    strides = tuple(0 if x.shape[i] == 1 else x.stride(i) for i in range(3))
-    return x, strides
+    if m is None and (x.shape[3] == Sk and x.stride(3) == 1 and Sk == width and x.data_ptr() % 16 == 0 and
+                      all(x.stride(i) % 4 == 0 for i in range(3))):
+        return x, tuple(0 if x.shape[i] == 1 else x.stride(i) for i in range(3))
+    lead = [max(t.shape[i] for t in (x, m) if t is not None) for i in range(3)]
+    if x is not None and not x.is_cuda:
+        out = torch.zeros(lead + [width], dtype=torch.float32, device=dev)
+        out[..., :Sk] = x if m is None else x.masked_fill(~m, float("-inf"))
+    else:
+        out = torch.empty(lead + [width], dtype=torch.float32, device=dev)
+        with torch.cuda.device(out.device):
+            _lib.raise_for(_lib.lib().vx_full_bias_fwd(
+                x.data_ptr() if x is not None else None, _strides(x, range(4)) if x is not None else None,
+                m.data_ptr() if m is not None else None, _strides(m, range(4)) if m is not None else None,
+                lead[0], lead[1], lead[2], Sk, out.data_ptr(), _stream(out.device)))
+    return out, tuple(0 if lead[i] == 1 else out.stride(i) for i in range(3))
 
 
 def flash_supported(batch: int, seq_q: int, seq_k: int, num_heads: int, head_dim: int) -> bool:
@@ -151,9 +197,29 @@ def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *,
     it suits the short sequences that use it.
     """
     _check_qkv(q, k, v)
+    B, Sk = q.shape[0], k.shape[1]
+    dev = q.device
+    _require_supported(B, q.shape[1], Sk, q.shape[2], q.shape[3])
+    kvd = kbd = kv_len_t = masks = None
+    if kv_len is not None:
+        kv_len_t = torch.as_tensor(kv_len, device=dev).to(torch.int32).reshape(B).contiguous()
+    if key_valid is not None:
+        kvd = torch.as_tensor(key_valid, device=dev).reshape(B, Sk).to(torch.bool)
+    if key_bias is not None:
+        kbd = torch.as_tensor(key_bias, device=dev).reshape(B, Sk).to(torch.float32)
+    if kvd is not None or kbd is not None:
+        masks = _KeyMasks(kvd, kbd, want_len=False)
+    return _flash(q, k, v, scale, kv_len_t.data_ptr() if kv_len_t is not None else None, masks, bias, None, out)
+
+
+def _flash(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional[float], kv_len: Optional[int],
+           masks: Optional[_KeyMasks], bias, mask, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The launch behind the entry points: q, k and v checked, kv_len the
+    address of int32 (B,) lengths, masks the prepared key masks, bias and mask
+    broadcastable to (B, H, Sq, Sk) or None."""
     B, Sq, H, D = q.shape
     Sk = k.shape[1]
-    _require_supported(B, Sq, Sk, H, D)
+    dev = q.device
     if scale is None:
         scale = D ** -0.5
     scale = float(scale)
@@ -163,33 +229,18 @@ def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *,
         out = torch.empty((B, Sq, H, D), dtype=q.dtype, device=q.device)
     elif out.shape != (B, Sq, H, D) or out.dtype != q.dtype or out.stride(-1) != 1 or out.device != q.device:
         raise ValueError("out must be a (B, Sq, H, D) bf16 tensor with a contiguous head dim, on q's device")
-    dev = q.device
-    kv_len_t = key_valid_t = key_bias_t = None
-    stride = 0
-    if kv_len is not None:
-        kv_len_t = torch.as_tensor(kv_len, device=dev).to(torch.int32).reshape(B).contiguous()
-    if key_valid is not None:
-        kvd = torch.as_tensor(key_valid, device=dev).reshape(B, Sk).to(torch.bool)
-        key_valid_t = _mask_rows(kvd, Sk, torch.uint8, 0)
-        stride = key_valid_t.shape[1]
-    if key_bias is not None:
-        kbd = torch.as_tensor(key_bias, device=dev).reshape(B, Sk).to(torch.float32)
-        key_bias_t = _mask_rows(kbd, Sk, torch.float32, float("-inf"))
-        stride = key_bias_t.shape[1]
+    key_valid, key_bias, stride = (masks.valid, masks.bias, masks.stride) if masks is not None else (None, None, 0)
     L = _lib.lib()
-    stream = torch.cuda.current_stream(dev).cuda_stream
-    if bias is not None:
-        fb, fbs = _full_bias(bias, B, H, Sq, Sk, dev)
+    stream = _stream(dev)
+    if bias is not None or mask is not None:
+        fb, fbs = _full_bias(bias, B, H, Sq, Sk, dev, mask)
         with torch.cuda.device(dev):
             rc = L.vx_flash_attn_bias_fwd(
-                q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-                kv_len_t.data_ptr() if kv_len_t is not None else None,
-                key_valid_t.data_ptr() if key_valid_t is not None else None,
-                key_bias_t.data_ptr() if key_bias_t is not None else None,
+                q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), kv_len, key_valid, key_bias,
                 stride, fb.data_ptr(), _lib.strides3(fbs), B, Sq, Sk, H, D,
                 _lib.strides3(q.stride()[:3]), _lib.strides3(k.stride()[:3]),
                 _lib.strides3(v.stride()[:3]), _lib.strides3(out.stride()[:3]),
-                ctypes.c_float(scale), ctypes.c_void_p(stream))
+                ctypes.c_float(scale), stream)
         _lib.raise_for(rc)
         return out
     with torch.cuda.device(dev):
@@ -197,18 +248,14 @@ def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *,
         # that round's query tiles over two key halves (fp32 partials in a
         # workspace from torch's caching allocator)
         # (calls with a key bias never split: no workspace)
-        ws_bytes = 0 if key_bias_t is not None else int(L.vx_flash_attn_workspace_size(B, Sq, Sk, H, D))
+        ws_bytes = 0 if key_bias is not None else int(L.vx_flash_attn_workspace_size(B, Sq, Sk, H, D))
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
         rc = L.vx_flash_attn_ws_fwd(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-            kv_len_t.data_ptr() if kv_len_t is not None else None,
-            key_valid_t.data_ptr() if key_valid_t is not None else None,
-            key_bias_t.data_ptr() if key_bias_t is not None else None,
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), kv_len, key_valid, key_bias,
             stride, B, Sq, Sk, H, D,
             _lib.strides3(q.stride()[:3]), _lib.strides3(k.stride()[:3]),
             _lib.strides3(v.stride()[:3]), _lib.strides3(out.stride()[:3]),
-            ctypes.c_float(scale), ws.data_ptr() if ws is not None else None, ws_bytes,
-            ctypes.c_void_p(stream))
+            ctypes.c_float(scale), ws.data_ptr() if ws is not None else None, ws_bytes, stream)
     _lib.raise_for(rc)
     return out
 
@@ -296,29 +343,22 @@ def dot_product_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     B, Sq, H, D = q.shape
     Sk = k.shape[1]
     _require_supported(B, Sq, Sk, H, D)
-    sm_scale = D ** -0.5 if scale is None else scale
-    key_bias = key_valid = kv_len = full = None
-    valid = None
+    key_bias = key_valid = masks = full = full_mask = None
     if bias is not None:
         kb = _key_only(torch.as_tensor(bias, device=q.device), B, Sk, "bias")
         if kb is None:
-            full = torch.as_tensor(bias, device=q.device).to(torch.float32)
+            full = bias
         else:
             key_bias = kb.to(torch.float32)
-            valid = key_bias > float("-inf")
     if mask is not None:
         km = _key_only(torch.as_tensor(mask, device=q.device), B, Sk, "mask")
         if km is None:
-            m = torch.as_tensor(mask, device=q.device).to(torch.bool)
-            add = torch.zeros(m.shape, dtype=torch.float32, device=q.device).masked_fill_(~m, float("-inf"))
-            full = add if full is None else full + add
+            full_mask = mask
         else:
             key_valid = km.to(torch.bool)
-            valid = key_valid if valid is None else (valid & key_valid)
-    if valid is not None:
-        kv_len = _last_valid_plus_one(valid)
-    return flash_attention(q, k, v, scale=sm_scale, kv_len=kv_len, key_valid=key_valid,
-                           key_bias=key_bias, bias=full)
+    if key_valid is not None or key_bias is not None:
+        masks = _KeyMasks(key_valid, key_bias, want_len=True)
+    return _flash(q, k, v, scale, masks.kv_len if masks is not None else None, masks, full, full_mask)
 
 
 def masked_self_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
@@ -344,6 +384,7 @@ def masked_self_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         out = flash_attention(q, k, v, scale=scale)
     else:
         kv = torch.as_tensor(key_valid, device=q.device).reshape(b, k.shape[1]).to(torch.bool)
-        kv_len = _last_valid_plus_one(kv)
-        out = flash_attention(q, k, v, scale=scale, kv_len=kv_len, key_valid=kv)
+        _require_supported(b, s, k.shape[1], h, d)
+        masks = _KeyMasks(kv, None, want_len=True)
+        out = _flash(q, k, v, scale, masks.kv_len, masks, None, None)
     return out.reshape(b, s, h * d)

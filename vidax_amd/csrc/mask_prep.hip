@@ -1,0 +1,151 @@
+// Mask preparation of the flash kernels for gfx950: the caller's masks, in
+// whatever strides and widths they come, to the forms the attention kernels
+// stage, one launch each. As chains of six to eight elementwise and reduction
+// launches they took more time than the attention itself: masked
+// self-attention B=2 H=24 S=256 56.6 -> 29.0 us a call, a full bias with a
+// padding mask B=2 H=8 S=512 D=64 63.5 -> 34.2 us, a key bias H=24 S=8192 686
+// -> 677 us.
+#include "vx_gfx950.hpp"
+#include "vx_kernels.h"
+
+#include <algorithm>
+
+namespace vx {
+namespace {
+
+constexpr uint32_t kNegInfBits = 0xff800000u;
+constexpr uint32_t kQuietNanBits = 0x7fc00000u;
+
+// ---- key masks: one workgroup per batch item, 16 keys per thread and pass.
+// Validity bytes and fp32 biases of the keys go to rows padded to whole
+// 64-key tiles (padding invalid, -inf), and the index of the last key that is
+// valid and whose bias is above -inf, plus one, to kv_len. Latency-bound (a
+// row is a few KiB to 0.5 MiB): the loads of a pass are independent 16-byte
+// ones where base and key stride allow, and a row needs no second launch.
+constexpr int kKeyThreads = 1024;
+constexpr int kKeysPerThread = 16;
+
+__global__ __launch_bounds__(kKeyThreads) void key_mask_kernel(const KeyMaskArgs a) {
+  __shared__ int wave_last[kKeyThreads / 64];
+  const int b = blockIdx.x;
+  const int width = (a.Sk + 63) & ~63;
+  const uint8_t* vp = a.valid != nullptr ? a.valid + b * a.valid_strides[0] : nullptr;
+  const float* bp = a.bias != nullptr ? a.bias + b * a.bias_strides[0] : nullptr;
+  uint8_t* vo = a.valid_rows != nullptr ? a.valid_rows + b * a.row_stride : nullptr;
+  float* bo = a.bias_rows != nullptr ? a.bias_rows + b * a.row_stride : nullptr;
+  const bool v16 = a.valid_strides[1] == 1 && ((uintptr_t)vp & 15) == 0;
+  const bool b16 = a.bias_strides[1] == 1 && ((uintptr_t)bp & 15) == 0;
+  int last = 0;
+  for (int k0 = threadIdx.x * kKeysPerThread; k0 < width; k0 += kKeyThreads * kKeysPerThread) {
+    const bool whole = k0 + kKeysPerThread <= a.Sk;
+    uint32_t vw[4] = {0, 0, 0, 0};  // validity, one byte (0 or 1) per key
+    uint32_t bw[16];                // bias bits
+    if (vp != nullptr) {
+      if (v16 && whole) {
+        const u32x4 x = *(const u32x4*)(vp + k0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) vw[i >> 2] |= (((x[i >> 2] >> (8 * (i & 3))) & 0xffu) != 0 ? 1u : 0u) << (8 * (i & 3));
+      } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (k0 + i < a.Sk) vw[i >> 2] |= (vp[(k0 + i) * a.valid_strides[1]] != 0 ? 1u : 0u) << (8 * (i & 3));
+      }
+    }
+    if (bp != nullptr) {
+      if (b16 && whole) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const u32x4 x = *(const u32x4*)(bp + k0 + 4 * i);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) bw[4 * i + e] = x[e];
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          bw[i] = k0 + i < a.Sk ? ((const uint32_t*)bp)[(k0 + i) * a.bias_strides[1]] : kNegInfBits;
+      }
+    }
+    if (vo != nullptr) *(u32x4*)(vo + k0) = u32x4{vw[0], vw[1], vw[2], vw[3]};
+    if (bo != nullptr) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) *(u32x4*)(bo + k0 + 4 * i) = u32x4{bw[4 * i], bw[4 * i + 1], bw[4 * i + 2], bw[4 * i + 3]};
+    }
+    if (a.kv_len != nullptr) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        bool ok = k0 + i < a.Sk;
+        if (vp != nullptr) ok = ok && ((vw[i >> 2] >> (8 * (i & 3))) & 0xffu) != 0;
+        // above -inf: neither -inf nor NaN (tested on the bits)
+        if (bp != nullptr) ok = ok && bw[i] != kNegInfBits && (bw[i] & 0x7fffffffu) <= 0x7f800000u;
+        if (ok) last = k0 + i + 1;
+      }
+    }
+  }
+  if (a.kv_len == nullptr) return;
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) last = max(last, __shfl_xor(last, off, 64));
+  if ((threadIdx.x & 63) == 0) wave_last[threadIdx.x >> 6] = last;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int m = 0;
+    for (int w = 0; w < (int)blockDim.x / 64; ++w) m = max(m, wave_last[w]);
+    a.kv_len[b] = m;
+  }
+}
+
+// ---- full bias: rows of round_up(Sk, 64) fp32 values, one per (batch item,
+// head, query) of the broadcast extents, each bias + (mask ? 0 : -inf), the
+// padding 0 (no score there is used). One wave per row, 4 keys per lane and
+// pass; bound by the row stores (4 bytes per score), so nothing is gained by
+// wider loads of a mask byte.
+constexpr int kBiasWaves = 4;
+
+__global__ __launch_bounds__(kBiasWaves * 64) void full_bias_kernel(const FullBiasArgs a) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t rows = (int64_t)a.n[0] * a.n[1] * a.n[2];
+  const int width = (a.Sk + 63) & ~63;
+  for (int64_t r = (int64_t)blockIdx.x * kBiasWaves + wave; r < rows; r += (int64_t)gridDim.x * kBiasWaves) {
+    const int64_t bh = r / a.n[2];
+    const int q = (int)(r - bh * a.n[2]);
+    const int b = (int)(bh / a.n[1]), h = (int)(bh - (int64_t)b * a.n[1]);
+    const uint32_t* bp = a.bias != nullptr ? (const uint32_t*)a.bias + b * a.bias_strides[0] + h * a.bias_strides[1] +
+                                                 q * a.bias_strides[2]
+                                           : nullptr;
+    const uint8_t* mp =
+        a.mask != nullptr ? a.mask + b * a.mask_strides[0] + h * a.mask_strides[1] + q * a.mask_strides[2] : nullptr;
+    uint32_t* orow = (uint32_t*)a.out + r * width;
+    for (int k0 = lane * 4; k0 < width; k0 += 256) {
+      u32x4 o = {0, 0, 0, 0};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int k = k0 + e;
+        if (k < a.Sk) {
+          if (bp != nullptr) o[e] = bp[k * a.bias_strides[3]];
+          // x + -inf: -inf, or NaN where x is NaN or +inf
+          if (mp != nullptr && mp[k * a.mask_strides[3]] == 0)
+            o[e] = (o[e] & 0x7fffffffu) > 0x7f800000u || o[e] == 0x7f800000u ? kQuietNanBits : kNegInfBits;
+        }
+      }
+      *(u32x4*)(orow + k0) = o;
+    }
+  }
+}
+
+}  // namespace
+
+int launch_key_masks(const KeyMaskArgs& a, void* stream) {
+  const int need = (a.Sk + kKeysPerThread - 1) / kKeysPerThread;
+  const int threads = std::min(kKeyThreads, (need + 63) / 64 * 64);
+  hipLaunchKernelGGL(key_mask_kernel, dim3(a.B), dim3(threads), 0, (hipStream_t)stream, a);
+  return (int)hipGetLastError();
+}
+
+int launch_full_bias(const FullBiasArgs& a, void* stream) {
+  const int64_t rows = (int64_t)a.n[0] * a.n[1] * a.n[2];
+  const int64_t groups = std::min<int64_t>((rows + kBiasWaves - 1) / kBiasWaves, 8192);
+  hipLaunchKernelGGL(full_bias_kernel, dim3((unsigned)groups), dim3(kBiasWaves * 64), 0, (hipStream_t)stream, a);
+  return (int)hipGetLastError();
+}
+
+}  // namespace vx

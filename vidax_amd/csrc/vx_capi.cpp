@@ -574,6 +574,81 @@ int32_t vx_debug_clock_stamp(uint64_t* out, int32_t n_groups, int32_t* wall_cloc
 
 const char* vx_last_launch(void) { return g_last_launch; }
 
+int32_t vx_key_masks_fwd(const uint8_t* valid, const int64_t* valid_strides, const float* bias,
+                         const int64_t* bias_strides, int32_t batch, int32_t seq_k, int32_t* kv_len,
+                         uint8_t* valid_rows, float* bias_rows, int64_t row_stride, void* stream) {
+  if (valid == nullptr && bias == nullptr) return fail(VX_ERR_INVALID_ARGUMENT, "valid or bias must be non-NULL");
+  if (batch < 1 || seq_k < 1)
+    return fail(VX_ERR_INVALID_ARGUMENT, "batch (%d) and seq_k (%d) must be >= 1", batch, seq_k);
+  if ((valid_rows != nullptr && valid == nullptr) || (bias_rows != nullptr && bias == nullptr))
+    return fail(VX_ERR_INVALID_ARGUMENT, "a row output needs its input");
+  if (!aligned16(valid_rows) || !aligned16(bias_rows))
+    return fail(VX_ERR_INVALID_ARGUMENT, "valid_rows and bias_rows must be 16-byte aligned");
+  if ((reinterpret_cast<uintptr_t>(bias) & 3u) != 0 || (reinterpret_cast<uintptr_t>(kv_len) & 3u) != 0)
+    return fail(VX_ERR_INVALID_ARGUMENT, "bias and kv_len must be 4-byte aligned");
+  const int64_t need = ((int64_t)seq_k + 63) / 64 * 64;
+  if ((valid_rows != nullptr || bias_rows != nullptr) && (row_stride < need || row_stride % 64 != 0))
+    return fail(VX_ERR_INVALID_ARGUMENT,
+                "row_stride (%lld) must be a multiple of 64 and >= round_up(seq_k, 64) = %lld", (long long)row_stride,
+                (long long)need);
+  if ((valid != nullptr && valid_strides == nullptr) || (bias != nullptr && bias_strides == nullptr))
+    return fail(VX_ERR_INVALID_ARGUMENT, "strides must be given with valid and bias");
+  vx::KeyMaskArgs a{};
+  a.valid = valid;
+  a.bias = bias;
+  for (int i = 0; i < 2; ++i) {
+    a.valid_strides[i] = valid != nullptr ? valid_strides[i] : 0;
+    a.bias_strides[i] = bias != nullptr ? bias_strides[i] : 0;
+    if (a.valid_strides[i] < 0 || a.bias_strides[i] < 0)
+      return fail(VX_ERR_INVALID_ARGUMENT, "strides must be >= 0");
+  }
+  a.B = batch;
+  a.Sk = seq_k;
+  a.kv_len = kv_len;
+  a.valid_rows = valid_rows;
+  a.bias_rows = bias_rows;
+  a.row_stride = row_stride;
+  int32_t rc;
+  if ((rc = injected()) != VX_OK) return rc;
+  const int err = vx::launch_key_masks(a, stream);
+  if (err != 0) return fail(VX_ERR_LAUNCH, "key mask launch failed (hipError_t %d)", err);
+  return ok();
+}
+
+int32_t vx_full_bias_fwd(const float* bias, const int64_t* bias_strides, const uint8_t* mask,
+                         const int64_t* mask_strides, int32_t batch, int32_t num_heads, int32_t seq_q, int32_t seq_k,
+                         float* out, void* stream) {
+  if (bias == nullptr && mask == nullptr) return fail(VX_ERR_INVALID_ARGUMENT, "bias or mask must be non-NULL");
+  if (out == nullptr || !aligned16(out))
+    return fail(VX_ERR_INVALID_ARGUMENT, "out must be non-NULL and 16-byte aligned");
+  if ((reinterpret_cast<uintptr_t>(bias) & 3u) != 0)
+    return fail(VX_ERR_INVALID_ARGUMENT, "bias must be 4-byte aligned");
+  if (batch < 1 || num_heads < 1 || seq_q < 1 || seq_k < 1)
+    return fail(VX_ERR_INVALID_ARGUMENT, "batch (%d), num_heads (%d), seq_q (%d) and seq_k (%d) must be >= 1", batch,
+                num_heads, seq_q, seq_k);
+  if ((bias != nullptr && bias_strides == nullptr) || (mask != nullptr && mask_strides == nullptr))
+    return fail(VX_ERR_INVALID_ARGUMENT, "strides must be given with bias and mask");
+  vx::FullBiasArgs a{};
+  a.bias = bias;
+  a.mask = mask;
+  for (int i = 0; i < 4; ++i) {
+    a.bias_strides[i] = bias != nullptr ? bias_strides[i] : 0;
+    a.mask_strides[i] = mask != nullptr ? mask_strides[i] : 0;
+    if (a.bias_strides[i] < 0 || a.mask_strides[i] < 0)
+      return fail(VX_ERR_INVALID_ARGUMENT, "strides must be >= 0");
+  }
+  a.n[0] = batch;
+  a.n[1] = num_heads;
+  a.n[2] = seq_q;
+  a.Sk = seq_k;
+  a.out = out;
+  int32_t rc;
+  if ((rc = injected()) != VX_OK) return rc;
+  const int err = vx::launch_full_bias(a, stream);
+  if (err != 0) return fail(VX_ERR_LAUNCH, "full bias launch failed (hipError_t %d)", err);
+  return ok();
+}
+
 int32_t vx_flash_attn_split_plan(int32_t batch, int32_t seq_q, int32_t seq_k, int32_t num_heads, int32_t head_dim,
                                  int32_t num_cus, int32_t* split_items, int32_t* split_key,
                                  int64_t* workspace_bytes) {

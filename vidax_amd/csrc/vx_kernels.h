@@ -121,6 +121,34 @@ struct PrologueArgs {
   int64_t x_bstride, x_sstride, o_bstride, o_sstride, tab_stride;  // elements
 };
 
+// Key masks of the flash kernels: validity bytes (0 = masked) and biases of
+// Sk keys per batch item, at any element strides {batch, key} (0 for
+// broadcast dims), to rows of round_up(Sk, 64) keys row_stride apart. NULL
+// inputs and outputs are left out (a row output needs its input).
+struct KeyMaskArgs {
+  const uint8_t* valid;
+  const float* bias;
+  int64_t valid_strides[2], bias_strides[2];
+  int32_t B, Sk;
+  int32_t* kv_len;      // [B] last unmasked key + 1
+  uint8_t* valid_rows;  // 16-byte aligned, as bias_rows
+  float* bias_rows;
+  int64_t row_stride;   // elements, a multiple of 64
+};
+
+// Full bias of the flash kernels: out[b, h, q, k] = bias + (mask ? 0 : -inf)
+// over the extents n = {batch, head, query}, contiguous rows of
+// round_up(Sk, 64) values (padding 0). Strides {batch, head, query, key} in
+// elements, 0 for broadcast dims; bias or mask may be NULL.
+struct FullBiasArgs {
+  const float* bias;
+  const uint8_t* mask;
+  int64_t bias_strides[4], mask_strides[4];
+  int32_t n[3];
+  int32_t Sk;
+  float* out;
+};
+
 // Compute units of the current device (0 if unknown), cached per device.
 int device_cu_count();
 
@@ -134,6 +162,8 @@ int noalloc_scratch(void** ptr, int64_t* bytes);
 int launch_flash_fwd(const FlashArgs& a, void* stream, const char** launched);
 int launch_na3d_fwd(const Na3dArgs& a, void* stream, const char** launched);
 int launch_qk_prologue(const PrologueArgs& a, void* stream, const char** launched);
+int launch_key_masks(const KeyMaskArgs& a, void* stream);    // (no kernel name)
+int launch_full_bias(const FullBiasArgs& a, void* stream);
 
 // Measurement only: n_groups one-wave workgroups each store (XCD id, HW_ID,
 // shader clock counter, real-time counter) as four uint64 at out + 4 * group;
