@@ -316,3 +316,28 @@ def test_na3d_quad_waves(gpu, shape, ks, seed):
     ref = O.na3d(*(x.float().cpu().numpy() for x in few), ks)
     _check(out[..., heads, :].float().cpu().numpy(), ref, "2 x 2 waves vs oracle")
     _check(out_few.float().cpu().numpy(), ref, "8 y x 4 x waves vs oracle")
+
+
+@pytest.mark.parametrize("T,H,W,D,window,few,many", [
+    (3, 11, 20, 64, (3, 7, 7), 56, 58),     # 1 x 4 x 32 bricks: 504 and 522 workgroups
+    (2, 9, 33, 64, (1, 5, 9), 40, 48),      # one-plane windows, ragged x: 480 and 576
+    (4, 10, 33, 128, (3, 7, 7), 28, 29),    # t-stacked: 504 and 522
+    (3, 7, 17, 128, (2, 5, 9), 64, 66),     # an odd t plane, idle waves: 512 and 528
+])
+def test_na3d_few_and_many_workgroups(gpu, T, H, W, D, window, few, many):
+    """Grids that two workgroups per CU hold run pipelined steps, larger ones
+    block steps. Both score the same keys; the heads of the larger grid repeat
+    those of the smaller one, so each output may differ by the order of fp32
+    sums and one bf16 rounding (2^-7 of a value's binade)."""
+    from vidax_amd import neighborhood_attention_3d
+    print(f"[case] na3d few/many {T}x{H}x{W} D={D} {window} NH={few}/{many}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(11)
+    x = [torch.randn((1, T, H, W, few, D), generator=g, device=gpu).to(torch.bfloat16) for _ in range(3)]
+    x[0] = x[0] * D ** -0.5
+    heads = torch.arange(many, device=gpu) % few
+    a = neighborhood_attention_3d(*x, window)
+    b = neighborhood_attention_3d(*[t[..., heads, :].contiguous() for t in x], window)
+    torch.cuda.synchronize()
+    a = a[..., heads, :].float()
+    d = (a - b.float()).abs()
+    assert (d <= 2.0 ** -7 * a.abs() + 1e-5).all(), d.max().item()

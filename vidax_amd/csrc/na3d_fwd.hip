@@ -431,9 +431,13 @@ void na3d_wave_kernel(const Na3dArgs a, int n_yb, int n_xb, int n_xg) {
 // query against 672 for 8 y x 4 x waves, and a row is staged in 24 slots
 // instead of 32. The steps are as many, so it pays once the grid keeps the
 // CUs busy (kNaQuadMinGroups).
-template <int SEG, int D, bool TALL = false, bool WIDE = false, bool DEEP = false, bool TSTACK = false, bool QUAD = false>
+// FEW: the pipelined form for the 1 x 4 x 32 bricks at head dim 64 and the
+// t-stacked bricks too, for grids that two workgroups per CU hold
+// (kNaFewGroups): a wave then has no others to overlap with.
+template <int SEG, int D, bool TALL = false, bool WIDE = false, bool DEEP = false, bool TSTACK = false, bool QUAD = false,
+          bool FEW = false>
 struct PipeCfg {
-  static constexpr bool kBlock = (D == 64 && SEG == 16) || TSTACK;  // block form of the step
+  static constexpr bool kBlock = ((D == 64 && SEG == 16) || TSTACK) && !FEW;  // block form of the step
   static constexpr bool kHalfStep = WIDE;                           // the two waves of a SIMD half a step apart
   static constexpr bool kSkip = TSTACK || QUAD;                     // a wave skips chunks outside its t (y) window
   // block form: row sums of the unrounded probabilities (their x window a
@@ -478,9 +482,10 @@ struct PipeCfg {
   static_assert(kNS % kKeysPerCopy == 0 && kHalfL % 256 == 0, "whole copies per row, bank-aligned planes");
 };
 
-template <int SEG, int D, bool TALL, bool WIDE = false, bool DEEP = false, bool TSTACK = false, bool QUAD = false>
+template <int SEG, int D, bool TALL, bool WIDE = false, bool DEEP = false, bool TSTACK = false, bool QUAD = false,
+          bool FEW = false>
 __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int n_xb, unsigned char* smem) {
-  using C = PipeCfg<SEG, D, TALL, WIDE, DEEP, TSTACK, QUAD>;
+  using C = PipeCfg<SEG, D, TALL, WIDE, DEEP, TSTACK, QUAD, FEW>;
   static_assert(C::kQY * (QUAD ? 2 : 1) == C::kBrickY, "the waves of a brick cover its y rows");
   static_assert(C::kBrickX - C::kQX + SEG <= C::kNS, "a wave's segment stays inside the LDS row");
   VX_LDS unsigned char* const lds = (VX_LDS unsigned char*)smem;
@@ -624,13 +629,23 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
   }
   // Box rows are walked with a cursor (its y and plane in the box, its row
   // t * Hs + y of the grid) that advances one row at a time, so no step
-  // divides by NY. Past the last row it wraps to the box's first plane: those
-  // rows are copied but masked (their index is not below nrows).
+  // divides by NY. The rows past the last one are copied but masked (their
+  // index is not below nrows): at head dim 128 the cursor stays on the last
+  // row, whose lines are in the CU's cache (7x33x60 NH=12 (1,7,7), whose
+  // bricks walk 10 rows and copy 4 more, 59.5 -> 53.9 us; t-stacked bricks
+  // 21x45x80 NH=24 (3,7,7) 754 -> 742 us); at head dim 64, half the bytes a
+  // row, it wraps to the box's first plane, which spares the scalar unit the
+  // count (5x22x40 NH=16 (3,7,7) 24.5 -> 23.7 us, 33x88x160 NH=4 (11,11,11)
+  // 1.510 -> 1.482 ms).
+  constexpr bool kStay = D == 128 || FEW;
+  using Row = std::conditional_t<C::kBlock, int, int64_t>;  // block form: row number; pipelined: its byte offset
   struct Cursor {
-    int yr, tr, row;
+    int yr, tr, left;  // left (kStay): rows of the box after this one
+    Row row;
   };
   const uint32_t row_bytes = (uint32_t)((int64_t)W * tok_stride * 2);  // below 2^31 (checked on the host)
-  const int row0 = t_lo * Hs + Y_lo;                                   // the box's first row
+  const Row row_unit = C::kBlock ? (Row)1 : (Row)row_bytes;
+  const Row row0 = (Row)(t_lo * Hs + Y_lo) * row_unit;                 // the box's first row
   // Deep t windows (the t-plane-first brick order) walk their box planes
   // from the one whose t is a multiple of NT, wrapping round: bricks whose
   // boxes share a plane then read it in the same phase of their walks, while
@@ -639,26 +654,42 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
   // (3,7,7) window, in the launch order, 2 % slower, so the others walk
   // their planes in order).
   const int p0 = a.order == kNaOrderTColumns ? uni((NT - t_lo % NT) % NT) : 0;
-  // The cursor is wave-uniform; moving it through readfirstlane keeps its
-  // arithmetic on the scalar unit (left to itself the compiler walked it in
-  // 64-bit vector registers: ~60 VALU instructions per step).
-  const int plane_step = Hs - NY + 1;  // last y of a plane -> first y of the next
+  // (branches: nested selects cost more scalar instructions per step, and the
+  // scalar unit is shared by the CU's 8-16 waves: same box, 33x88x160 NH=4
+  // D=64 (11,11,11) 1.470 -> 1.443 ms, 21x45x80 NH=24 D=128 (3,7,7) 737 -> 725
+  // us, 5x11x20 NH=32 D=64 (3,7,7) 14.3 -> 13.2 us)
+  const Row plane_jump = (Row)(Hs - NY) * row_unit;  // last y of a plane -> last y before the next one's first
   auto advance = [&](Cursor& c) {
-    const bool last_y = c.yr + 1 == NY, wrap = last_y && c.tr + 1 == NT;
-    c.row = wrap ? row0 : c.row + (last_y ? plane_step : 1);
-    c.tr = wrap ? 0 : c.tr + (last_y ? 1 : 0);
-    c.yr = last_y ? 0 : c.yr + 1;
-    c.yr = __builtin_amdgcn_readfirstlane(c.yr);
-    c.tr = __builtin_amdgcn_readfirstlane(c.tr);
-    c.row = __builtin_amdgcn_readfirstlane(c.row);
+    if (!kStay || c.left > 0) {
+      if (kStay) --c.left;
+      c.row += row_unit;
+      if (++c.yr == NY) {
+        c.yr = 0;
+        if (c.tr + 1 == NT) {  // (the wrap to the box's first plane)
+          c.tr = 0;
+          c.row = row0;
+        } else {
+          ++c.tr;
+          c.row += plane_jump;
+        }
+      }
+    }
+    // moving the cursor through readfirstlane keeps its arithmetic on the
+    // scalar unit (left to itself the compiler walked it in 64-bit vector
+    // registers: ~60 VALU instructions per step)
+    if (kStay) c.left = __builtin_amdgcn_readfirstlane(c.left);
+    if constexpr (C::kBlock)
+      c.row = __builtin_amdgcn_readfirstlane(c.row);
+    else
+      c.row = (Row)uniform_u64((uint64_t)c.row);
   };
-  const Cursor first = {0, p0, row0 + p0 * Hs};
+  const Cursor first = {0, p0, nrows - 1, row0 + (Row)(p0 * Hs) * row_unit};
   // The key rows of one step (their grid rows and places in the box), taken
   // from the cursor, which moves on by kRows rows. K walks the rows; V and
   // the window mask use each step's record in later steps, so only one
   // cursor runs (the scalar unit is shared by the CU's 8-16 waves).
   struct StepRows {
-    int row0, row1;
+    Row row0, row1;
     int yr0, yr1;
     int tr0, tr1;  // (deep bricks: the rows' planes in the box)
   };
@@ -683,8 +714,8 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
   const bool copier = C::kCopyWaves == C::kWaves || wave < C::kCopyWaves;      // wave-uniform
   auto copy_row = [&](uint64_t base, int slot_off, const StepRows& rr, int p) __attribute__((always_inline)) {
     if (kExtraWaves == 0 || p + 1 < C::kCopiesPerWave || extra) {
-      const uint32_t row = (uint32_t)(dma_row[p] ? rr.row1 : rr.row0);
-      lds_dma16_buf(raw_rsrc_u64(base + (uint64_t)row * row_bytes), dma_voff[p], lds_base + slot_off + dma_dst[p]);
+      const Row row = dma_row[p] ? rr.row1 : rr.row0;
+      lds_dma16_buf(raw_rsrc_u64(base + (C::kBlock ? (uint64_t)(uint32_t)row * row_bytes : (uint64_t)row)), dma_voff[p], lds_base + slot_off + dma_dst[p]);
     }
   };
   auto issue = [&](uint64_t base, int slot_off, const StepRows& rr) {
@@ -764,15 +795,33 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
   for (int ds = 0; ds < C::kQK; ++ds) S = mfma32x32x16(kfrag(lds + C::kK, ds), qr[ds], S);
   bf16x8 Pp[2] = {bf16x8{}, bf16x8{}};
 
+  // Whether some row of chunk c (rows r) lies in this wave's t window
+  // (t-stacked bricks: st is the wave's first plane in the box, its lanes
+  // share one t plane) or in the union of its y windows (quad bricks).
+  const int st_w = TSTACK ? uni(st) : 0;
+  const int sy_w = QUAD ? uni(window_start(min(yw, Hs - 1), Hs, kh) - Y_lo) : 0;
+  const int ny_w = QUAD ? uni(window_start(min(yw + C::kQY - 1, Hs - 1), Hs, kh) - Y_lo) + kh - sy_w : 0;
+  auto chunk_active = [&](const StepRows& r, int c) -> bool {
+    if constexpr (!C::kSkip) return true;
+    const int r0 = c * C::kRows;
+    const bool in0 = QUAD ? (unsigned)(r.yr0 - sy_w) < (unsigned)ny_w : (unsigned)(r.tr0 - st_w) < (unsigned)kt;
+    const bool in1 = QUAD ? (unsigned)(r.yr1 - sy_w) < (unsigned)ny_w : (unsigned)(r.tr1 - st_w) < (unsigned)kt;
+    return (r0 < nrows && in0) || (r0 + 1 < nrows && in1);
+  };
+
   // One pipelined step: consumes S (scores of chunk s) and Pp (probabilities
   // of chunk s-1), produces Sn (scores of chunk s+1) and P (probabilities of
   // chunk s). rr: the rows of step s on entry (their K was issued two steps
   // ago), the rows of step s + 2 on return. IN (compile-time, so that the loop
   // carries no per-step test of it): some query of this wave lies inside the
   // grid.
+  // rn: the rows of step s + 1; act_prev (t-stacked bricks): chunk s-1 had a
+  // row in this wave's t window.
   auto step = [&](auto in_tag, const int s, f32x16& S, f32x16& Sn, const bf16x8 (&Pp)[2], bf16x8 (&P)[2],
-                  StepRows& rr) __attribute__((always_inline)) {
+                  StepRows& rr, const StepRows& rn, bool& act_prev) __attribute__((always_inline)) {
     constexpr bool IN = decltype(in_tag)::value;
+    const bool act_cur = chunk_active(rr, s), act_next = chunk_active(rn, s + 1);
+    const bool idle = C::kSkip && !act_prev && !act_cur && !act_next;
     // The previous step's copies (K of s+1, V of s-1) have landed once this
     // wave has none outstanding; the barrier publishes everyone's and frees
     // K slot s%2 (K of s, read last step) and V slot s%2 (V of s-2).
@@ -807,9 +856,13 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
     // (IN is the tag's value; the 1 x 4 x 32 bricks pass the runtime flag
     // instead, one loop for all waves: their two loops measured ~1 % slower
     // at the (3,7,7) config, whose x edge holds waves without queries)
-    if (!(IN && (TALL || wave_in))) {
-      // no query of this wave is inside the grid (the ragged x or y edge): it
-      // only copies its share of the rows
+    if (!(IN && (TALL || wave_in)) || idle) {
+      // no query of this wave is inside the grid (the ragged x or y edge), or
+      // none of chunks s-1, s, s+1 has a row in its t window: it only copies
+      // its share of the rows. An idle step's chunk s+1 scores start from the
+      // x window alone (no row of it counts).
+      if (idle) Sn = s_init;
+      act_prev = act_cur;
 #pragma unroll
       for (int j = 0; j < kStepCopies; ++j) copy(j);
       P[0] = bf16x8{};
@@ -888,22 +941,10 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
       l_tile = sum16(pf);
     }
     l_run += l_tile;
+    act_prev = act_cur;
   };
 
   // ---- block form.
-  // Whether some row of chunk c (rows r) lies in this wave's t window
-  // (t-stacked bricks: st is the wave's first plane in the box, its lanes
-  // share one t plane) or in the union of its y windows (quad bricks).
-  const int st_w = TSTACK ? uni(st) : 0;
-  const int sy_w = QUAD ? uni(window_start(min(yw, Hs - 1), Hs, kh) - Y_lo) : 0;
-  const int ny_w = QUAD ? uni(window_start(min(yw + C::kQY - 1, Hs - 1), Hs, kh) - Y_lo) + kh - sy_w : 0;
-  auto chunk_active = [&](const StepRows& r, int c) -> bool {
-    if constexpr (!C::kSkip) return true;
-    const int r0 = c * C::kRows;
-    const bool in0 = QUAD ? (unsigned)(r.yr0 - sy_w) < (unsigned)ny_w : (unsigned)(r.tr0 - st_w) < (unsigned)kt;
-    const bool in1 = QUAD ? (unsigned)(r.yr1 - sy_w) < (unsigned)ny_w : (unsigned)(r.tr1 - st_w) < (unsigned)kt;
-    return (r0 < nrows && in0) || (r0 + 1 < nrows && in1);
-  };
   // The probabilities of the chunk in S against the exponent offsets m0, m1 of
   // its two key rows (-m_run, or -inf for a row outside the lane's y or t
   // window): exponent, x window, bf16 packing into Pp; returns their sum.
@@ -1062,14 +1103,15 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
   } else {
     f32x16 S2;
     bf16x8 P2[2];
+    bool act_prev = false;  // chunk -1 (none)
     auto key_loop = [&](auto in_tag) __attribute__((always_inline)) {
       int s = 0;
       for (; s + 1 < n_steps; s += 2) {
-        step(in_tag, s, S, S2, Pp, P2, rows_even);
-        step(in_tag, s + 1, S2, S, P2, Pp, rows_odd);
+        step(in_tag, s, S, S2, Pp, P2, rows_even, rows_odd, act_prev);
+        step(in_tag, s + 1, S2, S, P2, Pp, rows_odd, rows_even, act_prev);
       }
       if (s < n_steps) {
-        step(in_tag, s, S, S2, Pp, P2, rows_even);
+        step(in_tag, s, S, S2, Pp, P2, rows_even, rows_odd, act_prev);
         Pp[0] = P2[0];
         Pp[1] = P2[1];
       }
@@ -1100,6 +1142,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? (
 void na3d_pipe_kernel(const Na3dArgs a, int n_yb, int n_xb) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[PipeCfg<SEG, D>::kSmem];
   na3d_pipe_body<SEG, D, false>(a, n_yb, n_xb, smem);
+}
+
+// The same bricks for few workgroups (head dim 64): pipelined steps, two
+// waves per SIMD.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void na3d_pipe_few_kernel(const Na3dArgs a, int n_yb, int n_xb) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem[PipeCfg<16, 64>::kSmem];
+  na3d_pipe_body<16, 64, false, false, false, false, false, true>(a, n_yb, n_xb, smem);
 }
 
 // Head dim 64: four waves per SIMD (at most 128 VGPRs; the workgroup's 32 KiB
@@ -1147,11 +1197,23 @@ void na3d_tstack_kernel(const Na3dArgs a, int n_yb, int n_xb) {
   na3d_pipe_body<16, D, false, false, false, true>(a, n_yb, n_xb, smem);
 }
 
+// The same bricks for few workgroups: pipelined steps, two waves per SIMD.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void na3d_tstack_few_kernel(const Na3dArgs a, int n_yb, int n_xb) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem[PipeCfg<16, 128, false, false, false, true>::kSmem];
+  na3d_pipe_body<16, 128, false, false, false, true, false, true>(a, n_yb, n_xb, smem);
+}
+
 // Workgroups from which the tall bricks at head dim 64 with kw' <= 9 take the
 // 2 x 2 waves (12 per CU). Same box, (3,7,7) windows, 8 x 4 -> 4 x 8 waves:
 // 720 workgroups 24.1 -> 24.8 us, 1296 37.3 -> 39.6, 1680 46.2 -> 47.0, 2592
 // 68.2 -> 68.2, 15120 458 -> 425; 4080 at (5,9,9) 182 -> 170.
 constexpr int64_t kNaQuadMinGroups = 3072;
+// Workgroups up to which the 1 x 4 x 32 bricks at head dim 64 run pipelined
+// steps: two per CU. Same box, block -> pipelined, 11 x 20 planes: 240
+// workgroups at (3,7,7) 12.5 -> 11.2 us, 480 15.1 -> 13.5, 600 17.7 -> 22.0,
+// 960 25.7 -> 27.6; 432 at (5,7,7) 22.2 -> 19.5, 648 26.4 -> 31.8.
+constexpr int64_t kNaFewGroups = 512;
 
 }  // namespace
 
@@ -1196,7 +1258,10 @@ int launch_na3d_fwd(const Na3dArgs& a, void* stream, const char** launched) {
       const int n_yb = (a.Hs + 3) / 4;
       const int n_xb = (a.W + 15) / 16;
       dim3 grid((unsigned)((a.T + 1) / 2) * n_yb * n_xb, a.NH, a.B);
-      hipLaunchKernelGGL((na3d_tstack_kernel<128>), grid, dim3(256), 0, st, a, n_yb, n_xb);
+      if ((int64_t)grid.x * grid.y * grid.z <= kNaFewGroups)
+        hipLaunchKernelGGL(na3d_tstack_few_kernel, grid, dim3(256), 0, st, a, n_yb, n_xb);
+      else
+        hipLaunchKernelGGL((na3d_tstack_kernel<128>), grid, dim3(256), 0, st, a, n_yb, n_xb);
       *launched = "na3d_tstack_kernel<128>";
       return (int)hipGetLastError();
     }
@@ -1212,7 +1277,11 @@ int launch_na3d_fwd(const Na3dArgs& a, void* stream, const char** launched) {
         hipLaunchKernelGGL((na3d_pipe_kernel<32, 128>), grid, dim3(256), 0, st, a, n_yb, n_xb);
         *launched = "na3d_pipe_kernel<32, 128>";
       } else if (a.variant == kNaPipe16) {
-        hipLaunchKernelGGL((na3d_pipe_kernel<16, 64>), grid, dim3(256), 0, st, a, n_yb, n_xb);
+        // (one name for both: the host-side plan does not know the grid)
+        if ((int64_t)grid.x * grid.y * grid.z <= kNaFewGroups)
+          hipLaunchKernelGGL(na3d_pipe_few_kernel, grid, dim3(256), 0, st, a, n_yb, n_xb);
+        else
+          hipLaunchKernelGGL((na3d_pipe_kernel<16, 64>), grid, dim3(256), 0, st, a, n_yb, n_xb);
         *launched = "na3d_pipe_kernel<16, 64>";
       } else {
         hipLaunchKernelGGL((na3d_pipe_kernel<32, 64>), grid, dim3(256), 0, st, a, n_yb, n_xb);
