@@ -321,7 +321,8 @@ int32_t vx_na3d_qprep_axes_check(const void* q, const void* k, const void* v, co
  *                       with the mean over the whole row (per_head_norm = 0,
  *                       Wan's q/k norm over the projected dim) or over each
  *                       head (per_head_norm = 1); fp32 statistics; weight is
- *                       fp32[num_heads * head_dim]
+ *                       fp32[num_heads * head_dim], or fp32[head_dim] for the
+ *                       per-head norm (the same for every head)
  *   else                y = x
  *   if rope_cos != NULL: every head's adjacent pairs (y[2j], y[2j+1]) are
  *                       rotated by (rope_cos[s*rope_stride + j],

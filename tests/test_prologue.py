@@ -454,3 +454,20 @@ def test_na3d_block_attention_fused_q(gpu, B, grid, NH, HD, ks, norm, rope):
     d = np.abs(o - ref)
     print(f"  vs oracle: max_abs={d.max():.3e} mean_abs={d.mean():.3e}", flush=True)
     assert d.max() <= 2e-2 and d.mean() <= 2e-3
+
+
+@pytest.mark.gpu
+def test_per_head_norm_takes_any_weight_view(gpu):
+    """The kernel reads the head_dim weights of a per-head norm in place: a
+    view at an address that is not 16-byte aligned, a strided one and another
+    dtype give the results of the plain vector."""
+    from vidax_amd import na3d_qk_norm_rope, rms_norm
+    print("[case] per-head norm weight views", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(3)
+    x = torch.randn((1, 2, 3, 5, 3, 64), generator=g, device=gpu).to(torch.bfloat16)
+    buf = torch.randn(129, generator=g, device=gpu).to(torch.bfloat16).float()
+    for w in (buf[1:65], buf[::2][:64], buf[:64].to(torch.bfloat16)):
+        plain = w.float().contiguous().clone()
+        assert torch.equal(na3d_qk_norm_rope(x, w, None), na3d_qk_norm_rope(x, plain, None))
+        y = x.reshape(1, -1, 3, 64)
+        assert torch.equal(rms_norm(y, w), rms_norm(y, plain))

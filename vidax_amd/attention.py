@@ -11,6 +11,7 @@ request raises instead of silently running something else.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 from typing import Optional, Tuple
 
@@ -29,6 +30,11 @@ __all__ = [
 
 
 def _check_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
+    if (isinstance(q, torch.Tensor) and isinstance(k, torch.Tensor) and isinstance(v, torch.Tensor) and
+            q.dim() == k.dim() == v.dim() == 4 and q.dtype == k.dtype == v.dtype == torch.bfloat16 and
+            q.is_cuda and q.device == k.device == v.device and q.stride(3) == k.stride(3) == v.stride(3) == 1 and
+            k.shape == v.shape and q.shape[0] == k.shape[0] and q.shape[2:] == k.shape[2:]):
+        return  # (the checks below say what is wrong)
     for name, t in (("q", q), ("k", k), ("v", v)):
         if not isinstance(t, torch.Tensor):
             raise TypeError(f"{name} must be a torch.Tensor")
@@ -53,10 +59,20 @@ def _check_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
 _MAX_KV_SEQ_STRIDE = 1 << 24
 
 
+def _strides3(t: torch.Tensor):
+    """The C ABI's {batch, seq, head} strides of a (B, S, H, D) tensor: None
+    (NULL) for the contiguous ones."""
+    _, S, H, D = t.shape
+    st = t.stride()
+    return None if st == (S * H * D, H * D, D, 1) else _lib.strides3(st[:3])
+
+
 def _aligned(t: torch.Tensor, max_seq_stride: Optional[int] = None) -> torch.Tensor:
     """Tensor usable by the kernels: 16-byte aligned with strides in multiples
     of 8 (and, for k and v, a sequence stride within the kernel's limit);
     otherwise a contiguous copy."""
+    if t.data_ptr() % 16 == 0 and _strides3(t) is None and t.shape[3] % 8 == 0:
+        return t
     ok = t.data_ptr() % 16 == 0 and all(s % 8 == 0 for s in t.stride()[:3])
     if max_seq_stride is not None and t.stride(1) > max_seq_stride:
         ok = False
@@ -66,10 +82,6 @@ def _aligned(t: torch.Tensor, max_seq_stride: Optional[int] = None) -> torch.Ten
 def _strides(x: torch.Tensor, dims) -> ctypes.Array:
     """Element strides of x's dims, 0 where the extent is 1 (broadcast)."""
     return (ctypes.c_int64 * len(dims))(*[0 if x.shape[d] == 1 else x.stride(d) for d in dims])
-
-
-def _stream(dev) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
 
 
 class _KeyMasks:
@@ -93,11 +105,12 @@ class _KeyMasks:
         self.kv_len = base if want_len else None
         self.bias = base + self.bias_off if want_rows and bias is not None else None
         self.valid = base + self.valid_off if want_rows and valid is not None else None
-        with torch.cuda.device(dev):
-            _lib.raise_for(_lib.lib().vx_key_masks_fwd(
-                valid.data_ptr() if valid is not None else None, _strides(valid, (0, 1)) if valid is not None else None,
-                bias.data_ptr() if bias is not None else None, _strides(bias, (0, 1)) if bias is not None else None,
-                B, Sk, self.kv_len, self.valid, self.bias, self.stride, _stream(dev)))
+        _lib.launch(dev, _lib.lib().vx_key_masks_fwd,
+                    valid.data_ptr() if valid is not None else None,
+                    _strides(valid, (0, 1)) if valid is not None else None,
+                    bias.data_ptr() if bias is not None else None,
+                    _strides(bias, (0, 1)) if bias is not None else None,
+                    B, Sk, self.kv_len, self.valid, self.bias, self.stride)
 
 
 def _mask_rows(x: torch.Tensor, sk: int, dtype: torch.dtype, fill) -> torch.Tensor:
@@ -145,11 +158,10 @@ def _full_bias(bias, B: int, H: int, Sq: int, Sk: int, dev, mask=None) -> Tuple[
         out[..., :Sk] = x if m is None else x.masked_fill(~m, float("-inf"))
     else:
         out = torch.empty(lead + [width], dtype=torch.float32, device=dev)
-        with torch.cuda.device(out.device):
-            _lib.raise_for(_lib.lib().vx_full_bias_fwd(
-                x.data_ptr() if x is not None else None, _strides(x, range(4)) if x is not None else None,
-                m.data_ptr() if m is not None else None, _strides(m, range(4)) if m is not None else None,
-                lead[0], lead[1], lead[2], Sk, out.data_ptr(), _stream(out.device)))
+        _lib.launch(out.device, _lib.lib().vx_full_bias_fwd,
+                    x.data_ptr() if x is not None else None, _strides(x, range(4)) if x is not None else None,
+                    m.data_ptr() if m is not None else None, _strides(m, range(4)) if m is not None else None,
+                    lead[0], lead[1], lead[2], Sk, out.data_ptr())
     return out, tuple(0 if lead[i] == 1 else out.stride(i) for i in range(3))
 
 
@@ -165,7 +177,20 @@ def flash_supported(batch: int, seq_q: int, seq_k: int, num_heads: int, head_dim
     return _lib.flash_shape_check(batch, seq_q, seq_k, num_heads, head_dim)[0] == _lib.VX_OK
 
 
+@functools.lru_cache(maxsize=1024)
+def _shape_ok(B: int, Sq: int, Sk: int, H: int, D: int) -> bool:
+    return _lib.flash_shape_check(B, Sq, Sk, H, D)[0] == _lib.VX_OK
+
+
+@functools.lru_cache(maxsize=1024)
+def _workspace_bytes(device_index: int, B: int, Sq: int, Sk: int, H: int, D: int) -> int:
+    with torch.cuda.device(device_index):
+        return int(_lib.lib().vx_flash_attn_workspace_size(B, Sq, Sk, H, D))
+
+
 def _require_supported(B: int, Sq: int, Sk: int, H: int, D: int) -> None:
+    if _shape_ok(B, Sq, Sk, H, D):
+        return
     rc, msg = _lib.flash_shape_check(B, Sq, Sk, H, D)
     if rc == _lib.VX_ERR_UNSUPPORTED:
         raise NotImplementedError(
@@ -204,9 +229,9 @@ def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *,
     if kv_len is not None:
         kv_len_t = torch.as_tensor(kv_len, device=dev).to(torch.int32).reshape(B).contiguous()
     if key_valid is not None:
-        kvd = torch.as_tensor(key_valid, device=dev).reshape(B, Sk).to(torch.bool)
+        kvd = _lib.as_dtype(key_valid, dev, torch.bool).reshape(B, Sk)
     if key_bias is not None:
-        kbd = torch.as_tensor(key_bias, device=dev).reshape(B, Sk).to(torch.float32)
+        kbd = _lib.as_dtype(key_bias, dev, torch.float32).reshape(B, Sk)
     if kvd is not None or kbd is not None:
         masks = _KeyMasks(kvd, kbd, want_len=False)
     return _flash(q, k, v, scale, kv_len_t.data_ptr() if kv_len_t is not None else None, masks, bias, None, out)
@@ -231,32 +256,21 @@ def _flash(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional[fl
         raise ValueError("out must be a (B, Sq, H, D) bf16 tensor with a contiguous head dim, on q's device")
     key_valid, key_bias, stride = (masks.valid, masks.bias, masks.stride) if masks is not None else (None, None, 0)
     L = _lib.lib()
-    stream = _stream(dev)
+    ptrs = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), kv_len, key_valid, key_bias, stride)
+    strides = (_strides3(q), _strides3(k), _strides3(v), _strides3(out))
     if bias is not None or mask is not None:
         fb, fbs = _full_bias(bias, B, H, Sq, Sk, dev, mask)
-        with torch.cuda.device(dev):
-            rc = L.vx_flash_attn_bias_fwd(
-                q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), kv_len, key_valid, key_bias,
-                stride, fb.data_ptr(), _lib.strides3(fbs), B, Sq, Sk, H, D,
-                _lib.strides3(q.stride()[:3]), _lib.strides3(k.stride()[:3]),
-                _lib.strides3(v.stride()[:3]), _lib.strides3(out.stride()[:3]),
-                ctypes.c_float(scale), stream)
-        _lib.raise_for(rc)
+        _lib.launch(dev, L.vx_flash_attn_bias_fwd, *ptrs, fb.data_ptr(), _lib.strides3(fbs), B, Sq, Sk, H, D,
+                    *strides, scale)
         return out
-    with torch.cuda.device(dev):
-        # grids whose last round would leave the device mostly idle split
-        # that round's query tiles over two key halves (fp32 partials in a
-        # workspace from torch's caching allocator)
-        # (calls with a key bias never split: no workspace)
-        ws_bytes = 0 if key_bias is not None else int(L.vx_flash_attn_workspace_size(B, Sq, Sk, H, D))
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
-        rc = L.vx_flash_attn_ws_fwd(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), kv_len, key_valid, key_bias,
-            stride, B, Sq, Sk, H, D,
-            _lib.strides3(q.stride()[:3]), _lib.strides3(k.stride()[:3]),
-            _lib.strides3(v.stride()[:3]), _lib.strides3(out.stride()[:3]),
-            ctypes.c_float(scale), ws.data_ptr() if ws is not None else None, ws_bytes, stream)
-    _lib.raise_for(rc)
+    # grids whose last round would leave the device mostly idle split
+    # that round's query tiles over two key halves (fp32 partials in a
+    # workspace from torch's caching allocator)
+    # (calls with a key bias never split: no workspace)
+    ws_bytes = 0 if key_bias is not None else _workspace_bytes(dev.index, B, Sq, Sk, H, D)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
+    _lib.launch(dev, L.vx_flash_attn_ws_fwd, *ptrs, B, Sq, Sk, H, D, *strides, scale,
+                ws.data_ptr() if ws is not None else None, ws_bytes)
     return out
 
 
@@ -383,7 +397,7 @@ def masked_self_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     if key_valid is None:
         out = flash_attention(q, k, v, scale=scale)
     else:
-        kv = torch.as_tensor(key_valid, device=q.device).reshape(b, k.shape[1]).to(torch.bool)
+        kv = _lib.as_dtype(key_valid, q.device, torch.bool).reshape(b, k.shape[1])
         _require_supported(b, s, k.shape[1], h, d)
         masks = _KeyMasks(kv, None, want_len=True)
         out = _flash(q, k, v, scale, masks.kv_len, masks, None, None)

@@ -111,7 +111,7 @@ constexpr int32_t kNaTColumnsMinKt = 5;
 struct PrologueArgs {
   const void* x;        // bf16 rows of H * D
   void* out;            // bf16, same row layout
-  const float* weight;  // H * D (whole-row norm) or H * D (per-head norm, per channel); NULL = no norm
+  const float* weight;  // H * D (whole-row norm) or D (per-head norm); NULL = no norm
   const float* cos;     // (S, >= D/2) rows at tab_stride; NULL = no rotation
   const float* sin;
   float eps;

@@ -13,6 +13,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
+from .prologue import AbsRope3dAxes, _tables
 
 __all__ = ["neighborhood_attention_3d", "na3d_attention", "na3d_kernel_name", "na3d_block_attention"]
 
@@ -82,13 +83,8 @@ def na3d_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     elif (out.shape != q.shape or out.dtype != q.dtype or not out.is_contiguous() or
           out.device != q.device or out.data_ptr() % 16 != 0):
         raise ValueError("out must be a contiguous, 16-byte aligned bf16 tensor shaped like q, on q's device")
-    stream = torch.cuda.current_stream(q.device).cuda_stream
-    with torch.cuda.device(q.device):
-        rc = _lib.lib().vx_na3d_fwd(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-            B, T, H, W, NH, HD, int(kernel_size[0]), int(kernel_size[1]), int(kernel_size[2]),
-            ctypes.c_float(scale), ctypes.c_void_p(stream))
-    _lib.raise_for(rc)
+    _lib.launch(q.device, _lib.lib().vx_na3d_fwd, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+                B, T, H, W, NH, HD, int(kernel_size[0]), int(kernel_size[1]), int(kernel_size[2]), scale)
     return out
 
 
@@ -126,15 +122,13 @@ def na3d_block_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         q_post_scale = HD ** -0.5
     weight = None
     if q_norm_weight is not None:
-        weight = torch.as_tensor(q_norm_weight, device=q.device).to(torch.float32).reshape(-1).contiguous()
+        weight = _lib.as_dtype(q_norm_weight, q.device, torch.float32).reshape(-1).contiguous()
         if weight.numel() != HD:
             raise ValueError(f"q_norm_weight has {weight.numel()} entries, head_dim is {HD}")
-    from .prologue import AbsRope3dAxes
     axes = isinstance(freqs, AbsRope3dAxes)
     cos_t = sin_t = None
     stride = 0
     if freqs is not None and not axes:
-        from .prologue import _tables
         cos_t, sin_t, stride = _tables(freqs, T * H * W, HD // 2, q.device)
     if axes:
         # one fp32 table each of T + H + W rows (t axis, h axis, w axis)
@@ -159,22 +153,13 @@ def na3d_block_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     elif (out.shape != q.shape or out.dtype != q.dtype or not out.is_contiguous() or
           out.device != q.device or out.data_ptr() % 16 != 0):
         raise ValueError("out must be a contiguous, 16-byte aligned bf16 tensor shaped like q, on q's device")
-    stream = torch.cuda.current_stream(q.device).cuda_stream
-    with torch.cuda.device(q.device):
-        if axes:
-            rc = _lib.lib().vx_na3d_qprep_axes_fwd(
-                q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-                B, T, H, W, NH, HD, int(kernel_size[0]), int(kernel_size[1]), int(kernel_size[2]),
-                weight.data_ptr() if weight is not None else None, ctypes.c_float(eps),
-                ctypes.c_float(q_post_scale),
-                ax_c.data_ptr(), ax_s.data_ptr(), int(ax_c.stride(0)), ax_split, ctypes.c_void_p(stream))
-        else:
-            rc = _lib.lib().vx_na3d_qprep_fwd(
-                q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-                B, T, H, W, NH, HD, int(kernel_size[0]), int(kernel_size[1]), int(kernel_size[2]),
-                weight.data_ptr() if weight is not None else None, ctypes.c_float(eps),
-                ctypes.c_float(q_post_scale),
-                cos_t.data_ptr() if cos_t is not None else None,
-                sin_t.data_ptr() if sin_t is not None else None, stride, ctypes.c_void_p(stream))
-    _lib.raise_for(rc)
+    args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, T, H, W, NH, HD, int(kernel_size[0]),
+            int(kernel_size[1]), int(kernel_size[2]), weight.data_ptr() if weight is not None else None, eps,
+            q_post_scale)
+    if axes:
+        _lib.launch(q.device, _lib.lib().vx_na3d_qprep_axes_fwd, *args, ax_c.data_ptr(), ax_s.data_ptr(),
+                    int(ax_c.stride(0)), ax_split)
+    else:
+        _lib.launch(q.device, _lib.lib().vx_na3d_qprep_fwd, *args, cos_t.data_ptr() if cos_t is not None else None,
+                    sin_t.data_ptr() if sin_t is not None else None, stride)
     return out

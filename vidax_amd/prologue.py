@@ -13,7 +13,6 @@ reference's norm -> (scale) -> rope sequences.
 """
 from __future__ import annotations
 
-import ctypes
 from typing import NamedTuple, Optional, Tuple
 
 import torch
@@ -67,6 +66,9 @@ def _check_x(x: torch.Tensor, name: str = "x") -> None:
 
 def _tables(freqs, seq: int, half: int, device) -> Tuple[torch.Tensor, torch.Tensor, int]:
     cos, sin = freqs
+    if half % 4 == 0 and all(isinstance(t, torch.Tensor) and t.dtype == torch.float32 and t.device == device and
+                             t.is_contiguous() and t.numel() == seq * half for t in (cos, sin)):
+        return cos, sin, half
     cos = torch.as_tensor(cos, device=device).to(torch.float32).reshape(-1, half)
     sin = torch.as_tensor(sin, device=device).to(torch.float32).reshape(-1, half)
     if cos.shape[0] != seq or sin.shape[0] != seq:
@@ -87,16 +89,17 @@ def _run(x4: torch.Tensor, out4: torch.Tensor, weight: Optional[torch.Tensor], e
     stride = 0
     if tables is not None:
         cos_t, sin_t, stride = tables
-    xs = _lib.strides2((x4.stride(0), x4.stride(1)))
-    os_ = _lib.strides2((out4.stride(0), out4.stride(1)))
-    stream = torch.cuda.current_stream(x4.device).cuda_stream
-    with torch.cuda.device(x4.device):
-        rc = _lib.lib().vx_rmsnorm_scale_rope_fwd(
-            x4.data_ptr(), out4.data_ptr(),
-            weight.data_ptr() if weight is not None else None, ctypes.c_float(eps), int(per_head),
-            ctypes.c_float(post_scale), cos_t.data_ptr() if cos_t is not None else None, sin_t.data_ptr() if sin_t is not None else None,
-            stride, B, S, H, D, xs, os_, ctypes.c_void_p(stream))
-    _lib.raise_for(rc)
+    _lib.launch(x4.device, _lib.lib().vx_rmsnorm_scale_rope_fwd, x4.data_ptr(), out4.data_ptr(),
+                weight.data_ptr() if weight is not None else None, eps, int(per_head), post_scale,
+                cos_t.data_ptr() if cos_t is not None else None, sin_t.data_ptr() if sin_t is not None else None,
+                stride, B, S, H, D, _lib.strides2(x4.stride()[:2]), _lib.strides2(out4.stride()[:2]))
+
+
+def _head_weight(w: torch.Tensor) -> torch.Tensor:
+    """A per-head norm's weight as the kernel reads it: contiguous and 16-byte
+    aligned."""
+    w = w.contiguous()
+    return w if w.data_ptr() % 16 == 0 else w.clone()
 
 
 def _head_dim_for(length: int) -> int:
@@ -125,14 +128,14 @@ def rms_norm(x: torch.Tensor, scale: torch.Tensor, eps: float = 1e-6) -> torch.T
     (..., L) bf16 with L a multiple of 64 (the projected q/k) or (B, S, H, D)
     with the norm over each head's D."""
     _check_x(x)
-    scale = torch.as_tensor(scale, device=x.device).to(torch.float32).reshape(-1)
+    scale = _lib.as_dtype(scale, x.device, torch.float32).reshape(-1)
     L = x.shape[-1]
     if scale.numel() != L:
         raise ValueError(f"scale has {scale.numel()} entries, x's last axis {L}")
     if x.dim() == 4:
         B, S, H, D = x.shape
         x4 = x.contiguous()
-        weight = scale.repeat(H).contiguous()
+        weight = _head_weight(scale)
         per_head = True
     else:
         lead = x.shape[:-1]
@@ -162,7 +165,7 @@ def qk_norm_rope(x: torch.Tensor, scale: Optional[torch.Tensor], freqs, num_head
     out4 = torch.empty((B, S, num_heads, D), dtype=x.dtype, device=x.device)
     weight = None
     if scale is not None:
-        weight = torch.as_tensor(scale, device=x.device).to(torch.float32).reshape(-1).contiguous()
+        weight = _lib.as_dtype(scale, x.device, torch.float32).reshape(-1).contiguous()
         if weight.numel() != L:
             raise ValueError(f"scale has {weight.numel()} entries, rows have {L}")
     tables = _tables(freqs, S, D // 2, x.device) if freqs is not None else None
@@ -289,10 +292,9 @@ def na3d_qk_norm_rope(x: torch.Tensor, scale: Optional[torch.Tensor], freqs, eps
     out4 = torch.empty_like(x4)
     weight = None
     if scale is not None:
-        w = torch.as_tensor(scale, device=x.device).to(torch.float32).reshape(-1)
-        if w.numel() != HD:
-            raise ValueError(f"scale has {w.numel()} entries, head_dim is {HD}")
-        weight = w.repeat(NH).contiguous()
+        weight = _head_weight(_lib.as_dtype(scale, x.device, torch.float32).reshape(-1))
+        if weight.numel() != HD:
+            raise ValueError(f"scale has {weight.numel()} entries, head_dim is {HD}")
     tables = _tables(freqs, T * H * W, HD // 2, x.device) if freqs is not None else None
     _run(x4, out4, weight, float(eps), True, tables, float(post_scale))
     return out4.reshape(x.shape)
