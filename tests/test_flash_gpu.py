@@ -851,3 +851,52 @@ def test_dot_product_attention_key_bias_forms(gpu, form):
         print(f"  key bias vs validity mask: equal={torch.equal(out, as_mask)} max {d.max().item():.3e}",
               flush=True)
         assert d.max().item() <= 1e-2 and d.mean().item() <= 1e-4, (d.max().item(), d.mean().item())
+
+
+# ------------------------------------- two groups of waves per query tile (pairs)
+PAIR_CASES = [
+    # B, Sq, Sk, H, D, mask (grids of at most one workgroup per CU)
+    (1, 130, 384, 2, 64, None),                       # 6 tiles: the first pair at head dim 64
+    (1, 70, 320, 2, 64, None),                        # 5 tiles: one group
+    (2, 129, 449, 3, 64, ("kv_len", 449, 1)),         # an odd tile count; one key: group 1 without tiles
+    (2, 33, 640, 2, 128, ("kv_len", 0, 129)),         # no key; three tiles, two and one
+    (1, 128, 640, 2, 128, None),                      # 10 tiles: the first pair at head dim 128
+    (1, 200, 705, 2, 128, ("tail_pad", 200)),         # 12 tiles, key validity with an empty tail
+    (1, 140, 1537, 2, 128, None),                     # 25 tiles: key halves on two pairs
+    (2, 140, 1537, 2, 64, ("kv_len", 1000, 700)),     # the second key half empty for one item
+]
+
+
+@pytest.mark.parametrize("B,Sq,Sk,H,D,mask", PAIR_CASES)
+@pytest.mark.parametrize("kind", ["plain", "key_bias", "full_bias"])
+def test_flash_pairs(gpu, B, Sq, Sk, H, D, mask, kind):
+    """Grids that leave CUs idle run two groups of four waves per query tile,
+    each over half of the key tiles, merged in LDS: against the oracle at the
+    edges of the rule and of the halves, with every mask form that runs pairs."""
+    from vidax_amd import flash_attention
+    _say(f"flash pairs B={B} Sq={Sq} Sk={Sk} H={H} D={D} mask={mask} {kind}")
+    q, k, v, extra = O.make_flash_inputs(B, Sq, Sk, H, D, 190)
+    rng = np.random.default_rng(191)
+    if mask is not None and mask[0] == "kv_len":
+        extra["kv_len"] = np.array(mask[1:], np.int32)
+    elif mask is not None:
+        extra["key_valid"] = np.broadcast_to(np.arange(Sk) < Sk - mask[1], (B, Sk)).copy()
+    if kind == "key_bias":
+        if "key_valid" in extra:
+            pytest.skip("validity together with a key bias runs one group")
+        extra["key_bias"] = rng.standard_normal((B, Sk)).astype(np.float32)
+        extra["key_bias"][:, Sk // 3:Sk // 3 + 70] = -np.inf
+        extra["key_bias"][:, 0] = 0.0
+    if kind == "full_bias":
+        extra["bias"] = rng.standard_normal((1, H, Sq, Sk)).astype(np.float32)
+        extra["bias"][..., 1::7] = -np.inf
+    out = flash_attention(_t(q, gpu), _t(k, gpu), _t(v, gpu),
+                          **{n: torch.from_numpy(x).to(gpu) for n, x in extra.items()})
+    torch.cuda.synchronize()
+    if "bias" in extra:
+        extra["bias"] = np.broadcast_to(extra["bias"], (B, H, Sq, Sk))
+    ref = O.attention(q, k, v, **extra)
+    if "kv_len" in extra and (extra["kv_len"] == 0).any():
+        assert (out[0] == 0).all()
+        out, ref = out[1:], ref[1:]
+    _check(out, ref, "oracle")

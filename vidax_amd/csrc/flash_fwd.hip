@@ -127,7 +127,11 @@ __device__ __forceinline__ void store_out_lines(const f32x16 (&O)[kDB], float in
 // normalised bf16 output rows; part >= 0 writes the unnormalised fp32
 // accumulators, the reference point and the row sums to partial slot `part`
 // of a.ws (a key-split item, merged by flash_combine_kernel).
-template <int MASK, int D, int WAVES>
+//
+// PAIR: a workgroup of two groups of WAVES waves on the same query tile, each
+// with its own LDS rings and half of the key tiles; group 0 issues both
+// groups' copies and takes group 1's accumulators from LDS at the end.
+template <int MASK, int D, int WAVES, bool PAIR = false>
 __device__ __forceinline__ void flash_tile(const FlashArgs& a, const int qtile, const int head, const int b,
                                            const int k_lo, const int k_hi, const int part) {
   using C = FCfg<D, WAVES>;
@@ -139,11 +143,18 @@ __device__ __forceinline__ void flash_tile(const FlashArgs& a, const int qtile, 
   constexpr bool MASKED = MASK != kMaskNone;
   constexpr int kMaskCopies = (MASK & kMaskValid ? 1 : 0) + (MASK & kMaskBias ? 1 : 0);
   constexpr bool kFull = (MASK & kMaskFull) != 0;
-  __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytes + (MASKED ? kMaskRing * kMaskSlot : 0)];
-  lds_u8* const lds = (lds_u8*)smem;
+  constexpr int kGroupBytes = kSmemBytes + (MASKED ? kMaskRing * kMaskSlot : 0);
+  static_assert(kGroupBytes % 256 == 0, "the second group's rings start on a bank boundary");
+  static_assert(!PAIR || kSmemBytes >= WAVES * 64 * kDB * 64, "group 1's accumulators fit its rings");
+  // (a pair: both groups' rings, then group 1's reference points and row sums)
+  __shared__ __attribute__((aligned(16))) unsigned char smem[PAIR ? 2 * kGroupBytes + kThreads * 8 : kGroupBytes];
 
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
+  const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
+  const int group = PAIR ? wave_all / kWaves : 0;
+  const int wave = PAIR ? wave_all % kWaves : wave_all;
+  const int tid = wave * 64 + lane;
+  lds_u8* const lds = (lds_u8*)smem + group * kGroupBytes;
   const int hf = lane >> 5;   // which half of the wave
   const int col = lane & 31;  // query column within the wave's 32
   const int qw0 = (qtile * kWaves + wave) * 32;
@@ -155,8 +166,19 @@ __device__ __forceinline__ void flash_tile(const FlashArgs& a, const int qtile, 
   int kv_end = k_hi;
   if (a.kv_len != nullptr) kv_end = min(max(a.kv_len[b], 0), k_hi);
   kv_end = __builtin_amdgcn_readfirstlane(kv_end);  // uniform: scalar loop control
-  const int t_begin = k_lo / kBN;                   // first key tile of the range
-  const int n_tiles = (kv_end + kBN - 1) / kBN;     // one past the last key tile
+  int t_begin = k_lo / kBN;                         // first key tile of the range
+  int n_tiles = (kv_end + kBN - 1) / kBN;           // one past the last key tile
+  // a pair's key tiles: group 0 takes the first half (one more of an odd
+  // number); its tile t goes with group 1's tile t + pair_ofs
+  const int n_pair = PAIR ? max(n_tiles - t_begin, 0) : 0;
+  const int pair_ofs = (n_pair + 1) / 2, pair_last = n_tiles - 1;
+  if (PAIR) {
+    const int mid = t_begin + (n_pair + 1) / 2;
+    if (group == 0)
+      n_tiles = min(n_tiles, mid);
+    else
+      t_begin = mid;
+  }
   const float c = a.scale * kLog2e;
 
   // ---- Q (B operand of S^T = K Q^T), resident for the whole key loop.
@@ -354,9 +376,9 @@ __device__ __forceinline__ void flash_tile(const FlashArgs& a, const int qtile, 
   // per-lane part of the source is a small constant offset)
   const uint64_t vrow_addr = uniform_u64((uint64_t)(uintptr_t)vrow);
   const uint64_t brow_addr = uniform_u64((uint64_t)(uintptr_t)brow);
-  auto stage_mask = [&](int j) {
+  auto stage_mask_at = [&](int j, uint32_t base) {
     if (!MASKED || wave != 0) return;
-    const uint32_t slot = lds_base + kMaskBuf + (j & (kMaskRing - 1)) * kMaskSlot;
+    const uint32_t slot = base + kMaskBuf + (j & (kMaskRing - 1)) * kMaskSlot;
     if (MASK & kMaskValid) {
       if (lane < 4) lds_dma16_buf(raw_rsrc_u64(vrow_addr + (uint64_t)j * kBN), lane * 16, slot);
     }
@@ -364,10 +386,26 @@ __device__ __forceinline__ void flash_tile(const FlashArgs& a, const int qtile, 
       if (lane < 16) lds_dma16_buf(raw_rsrc_u64(brow_addr + (uint64_t)j * kBN * 4), lane * 16, slot + 64);
     }
   };
+  auto stage_mask = [&](int j) {
+    stage_mask_at(min(j, n_tiles - 1), lds_base);
+    if (PAIR) stage_mask_at(min(j + pair_ofs, pair_last), lds_base + kGroupBytes);
+  };
+  // the copies of tile j of a group's walk (the last tile again past its end)
+  // into its buffer at buf_off, for both groups of a pair
+  auto copy_k = [&](const Lanes& ln, int j, int buf_off) __attribute__((always_inline)) {
+    stage_k(ln, min(j, n_tiles - 1), buf_off);
+    if (PAIR) stage_k(ln, min(j + pair_ofs, pair_last), buf_off + kGroupBytes);
+  };
+  auto copy_v = [&](const Lanes& ln, int j, int buf_off) __attribute__((always_inline)) {
+    stage_v(ln, min(j, n_tiles - 1), buf_off);
+    if (PAIR) stage_v(ln, min(j + pair_ofs, pair_last), buf_off + kGroupBytes);
+  };
+  constexpr int kCopyGroups = PAIR ? 2 : 1;
   // At the top of iteration t: the tiles it reads (K_{t+1}, V_{t-1}) were
   // issued kNB - 1 iterations earlier; the copies of the last kNB - 2
   // iterations may still be in flight.
   auto wait_prev = [&]() {
+    static_assert(!PAIR || kNB == 2, "a pair waits for all its copies");
     if (MASKED && wave == 0)
       wait_vmem<(kNB - 2) * (2 * kLoadsPerWave + kMaskCopies)>();
     else
@@ -382,26 +420,26 @@ __device__ __forceinline__ void flash_tile(const FlashArgs& a, const int qtile, 
     // finished reading; the prologue issues the first mask and then the same
     // groups for t = -kNB .. -1, so that every wait below counts whole
     // groups (the first mask is older than all of them).
-    if (wave < kCopyWaves) {
+    if (wave < kCopyWaves && group == 0) {
       const Lanes ln = make_lanes();
       stage_mask(t_begin);  // (masks run one tile ahead of K: the first one on its own)
 #pragma unroll
       for (int j = 0; j < kNB; ++j) {
-        stage_k(ln, min(t_begin + j, n_tiles - 1), kKBuf + j * kTileBytes);
-        stage_mask(min(t_begin + j + 1, n_tiles - 1));
-        if (j >= 2) stage_v(ln, min(t_begin + j - 2, n_tiles - 1), kVBuf + (j - 2) * kTileBytes);
+        copy_k(ln, t_begin + j, kKBuf + j * kTileBytes);
+        stage_mask(t_begin + j + 1);
+        if (j >= 2) copy_v(ln, t_begin + j - 2, kVBuf + (j - 2) * kTileBytes);
       }
     }
 #pragma unroll
     for (int p = 0; p < kTileBytes / (kThreads * 16); ++p)
-      *(VX_LDS u32x4*)(lds + kVBuf + (kNB - 1) * kTileBytes + (p * kThreads + threadIdx.x) * 16) = u32x4{0, 0, 0, 0};
+      *(VX_LDS u32x4*)(lds + kVBuf + (kNB - 1) * kTileBytes + (p * kThreads + tid) * 16) = u32x4{0, 0, 0, 0};
     // K_0 has landed (with two tiles per ring, K_1 may still be in flight;
     // with more, K_1 has landed too)
     if (kNB == 2) {
       if (MASKED && wave == 0)
-        wait_vmem<kLoadsPerWave + kMaskCopies>();
+        wait_vmem<kCopyGroups * (kLoadsPerWave + kMaskCopies)>();
       else
-        wait_vmem<kLoadsPerWave>();
+        wait_vmem<kCopyGroups * kLoadsPerWave>();
     } else {
       wait_prev();
     }
@@ -424,12 +462,14 @@ __device__ __forceinline__ void flash_tile(const FlashArgs& a, const int qtile, 
     // tile t-1), produces Sn (scores of tile t+1) and P (probabilities of
     // tile t). The loop below calls it twice per trip with the two register
     // sets swapped, so no copies are needed between tiles.
-    // COPY (a compile-time tag): this wave issues tile copies. The 8-wave
-    // workgroups run two copies of the loop, one for the copying waves and
-    // one for the others, so that neither carries the other's branches.
+    // copy_tag (compile-time): 1, this wave issues tile copies (COPY); 2, its
+    // softmax follows its MFMAs (LATE). The 8-wave workgroups run two copies
+    // of the loop, one for the copying waves and one for the others, so that
+    // neither carries the other's branches; so do the groups of a pair.
     auto step = [&](auto copy_tag, const Lanes& ln, const int t, f32x16 (&S)[2], f32x16 (&Sn)[2],
                     const bf16x8 (&Pp)[2][2], bf16x8 (&P)[2][2]) __attribute__((always_inline)) {
-      constexpr bool COPY = decltype(copy_tag)::value;
+      constexpr bool COPY = (decltype(copy_tag)::value & 1) != 0;
+      constexpr bool LATE = (decltype(copy_tag)::value & 2) != 0;
       // K_{t+1} and V_{t-1} have landed once wait_prev returns; the barrier
       // then publishes them, and it also frees K buffer t % kNB (K_t, read by
       // QK(t) last iteration) and V buffer (t+kNB-2) % kNB (V_{t-2}) for this
@@ -461,9 +501,9 @@ __device__ __forceinline__ void flash_tile(const FlashArgs& a, const int qtile, 
       if (MASK & kMaskFull) slow = true;
       // this iteration's copies: K_{t+kNB}, the mask of tile t+kNB+1 and V_{t+kNB-2}
       if (COPY) {
-        stage_k(ln, min(t + kNB, n_tiles - 1), kKBuf + kb_next * kTileBytes);
-        stage_mask(min(t + kNB + 1, n_tiles - 1));
-        stage_v(ln, min(t + kNB - 2, n_tiles - 1), kVBuf + vb_next * kTileBytes);
+        copy_k(ln, t + kNB, kKBuf + kb_next * kTileBytes);
+        stage_mask(t + kNB + 1);
+        copy_v(ln, t + kNB - 2, kVBuf + vb_next * kTileBytes);
       }
       float cc = c;
       if (slow) {
@@ -503,8 +543,9 @@ __device__ __forceinline__ void flash_tile(const FlashArgs& a, const int qtile, 
       // waves per SIMD, one wave's MFMA block overlaps the other wave's VALU
       // block, which measured 1.5 % faster at L=32760 than interleaving one
       // score's exp into every slot (and no slower with 4 waves). In 8-wave
-      // workgroups the VALU block follows the MFMAs, in 4-wave workgroups it
-      // precedes them.
+      // workgroups the VALU block follows the MFMAs of the waves that do not
+      // copy, in 4-wave workgroups it precedes them, and in a pair it follows
+      // them in group 1.
       float l_tile = 0.f;
       {
         const lds_u8* kb0 = lds + kKBuf + kb_cur * kTileBytes;
@@ -530,8 +571,8 @@ __device__ __forceinline__ void flash_tile(const FlashArgs& a, const int qtile, 
         // fill the gaps they leave: +0.7 %), with 4 waves (two workgroups per
         // CU) for every wave, ahead of the other workgroup's wave while that
         // one copies, waits or starts (+2-4 % at 512 keys).
-        constexpr bool kAllPrio = WAVES == 4;
-        if (kAllPrio || !COPY) __builtin_amdgcn_s_setprio(1);
+        constexpr bool kPrio = (WAVES == 4 && !PAIR) || !COPY;
+        if (kPrio) __builtin_amdgcn_s_setprio(1);
         bf16x8 fr[kSlots];
         float pf[32];
         bf16x2 pk[16];
@@ -557,7 +598,7 @@ __device__ __forceinline__ void flash_tile(const FlashArgs& a, const int qtile, 
           for (int i = 0; i < 16; ++i) l_tile = __builtin_amdgcn_fdot2_f32_bf16(pk[i], one2, l_tile, false);
           __builtin_amdgcn_sched_barrier(0);
         };
-        if (WAVES == 4 || COPY) softmax_block();
+        if (!LATE) softmax_block();
         // read by the QK^T slots (16 and on)
         Sn[0] = f32x16{};
         Sn[1] = f32x16{};
@@ -573,9 +614,9 @@ __device__ __forceinline__ void flash_tile(const FlashArgs& a, const int qtile, 
           }
           __builtin_amdgcn_sched_barrier(0);
         }
-        if (kAllPrio || !COPY) __builtin_amdgcn_s_setprio(0);
+        if (kPrio) __builtin_amdgcn_s_setprio(0);
         __builtin_amdgcn_sched_barrier(0);
-        if (WAVES == 8 && !COPY) softmax_block();
+        if (LATE) softmax_block();
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -614,7 +655,7 @@ __device__ __forceinline__ void flash_tile(const FlashArgs& a, const int qtile, 
     bf16x8 P2[2][2];
     auto key_loop = [&](auto copy_tag) __attribute__((always_inline)) {
       Lanes ln{};
-      if constexpr (decltype(copy_tag)::value) ln = make_lanes();
+      if constexpr (decltype(copy_tag)::value & 1) ln = make_lanes();
       int t = t_begin;
       for (; t + 1 < n_tiles; t += 2) {
         step(copy_tag, ln, t, S, S2, Pp, P2);
@@ -628,14 +669,51 @@ __device__ __forceinline__ void flash_tile(const FlashArgs& a, const int qtile, 
           for (int j = 0; j < 2; ++j) Pp[kb][j] = P2[kb][j];
       }
     };
-    if (kCopyWaves == kWaves || wave < kCopyWaves)
-      key_loop(std::integral_constant<bool, true>{});
+    using Early = std::integral_constant<int, 1>;
+    using Late = std::integral_constant<int, !PAIR && kCopyWaves == kWaves ? 1 : 2>;
+    if (PAIR ? group == 0 : kCopyWaves == kWaves || wave < kCopyWaves)
+      key_loop(Early{});
     else
-      key_loop(std::integral_constant<bool, kCopyWaves == kWaves>{});
+      key_loop(Late{});
     // ---- PV of the last tile (V_{n-1} sits in V buffer vb_prev now).
     wait_vmem<0>();
     __syncthreads();
     pv(kVBuf + vb_prev * kTileBytes, Pp, O);
+  }
+
+  // ---- pair: group 1's accumulators through its rings
+  if constexpr (PAIR) {
+    // (a group of c > 0 tiles passes c + 2 barriers, one without tiles none:
+    // group 1 makes up for its fewer ones)
+    const int c0 = (n_pair + 1) / 2, c1 = n_pair / 2;
+    if (group == 1)
+      for (int i = c0 + (c0 > 0 ? 2 : 0) - c1 - (c1 > 0 ? 2 : 0); i > 0; --i) __syncthreads();
+    __syncthreads();  // group 1 has read its last V tile
+    VX_LDS f32x4* const xo = (VX_LDS f32x4*)((lds_u8*)smem + kGroupBytes) + wave * (kDB * 4) * 64 + lane;
+    VX_LDS float* const xm = (VX_LDS float*)((lds_u8*)smem + 2 * kGroupBytes) + 2 * tid;
+    if (group == 1) {
+#pragma unroll
+      for (int db = 0; db < kDB; ++db)
+#pragma unroll
+        for (int k4 = 0; k4 < 4; ++k4)
+          xo[(db * 4 + k4) * 64] = f32x4{O[db][4 * k4], O[db][4 * k4 + 1], O[db][4 * k4 + 2], O[db][4 * k4 + 3]};
+      xm[0] = m_run;
+      xm[1] = l_run;
+    }
+    __syncthreads();
+    if (group == 1) return;
+    const float m1 = xm[0], l1 = xm[1], M = fmaxf(m_run, m1);
+    const float a0 = fast_exp2(m_run - M), a1 = fast_exp2(m1 - M);
+    m_run = M;
+    l_run = l_run * a0 + l1 * a1;
+#pragma unroll
+    for (int db = 0; db < kDB; ++db)
+#pragma unroll
+      for (int k4 = 0; k4 < 4; ++k4) {
+        const f32x4 x = xo[(db * 4 + k4) * 64];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) O[db][4 * k4 + e] = O[db][4 * k4 + e] * a0 + x[e] * a1;
+      }
   }
 
   // ---- key-split item: the unnormalised accumulators, the reference point
@@ -686,6 +764,28 @@ void flash_fwd_split_kernel(const FlashArgs a, int n_full, int n_qt) {
   }
   const int qt = item % n_qt, bh = item / n_qt;
   flash_tile<MASK, D, WAVES>(a, qt, bh % a.H, bh / a.H, k_lo, k_hi, part);
+}
+
+// Two groups of four waves per 128-query tile (flash_tile's PAIR), for grids
+// that leave a CU to each workgroup: the same two waves per SIMD that two
+// workgroups per CU give larger grids, with half the key tiles each, merged in
+// LDS. One workgroup per item, or per half of its keys (a.split_items > 0,
+// every item split).
+template <int MASK, int D>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void flash_pair_kernel(const FlashArgs a, int n_qt) {
+  const int w = blockIdx.x;
+  int item = w, k_lo = 0, k_hi = a.Sk, part = -1;
+  if (a.split_items > 0) {
+    part = w;
+    item = w >> 1;
+    if (part & 1)
+      k_lo = a.k_mid;
+    else
+      k_hi = a.k_mid;
+  }
+  const int qt = item % n_qt, bh = item / n_qt;
+  flash_tile<MASK, D, 4, true>(a, qt, bh % a.H, bh / a.H, k_lo, k_hi, part);
 }
 
 // Merges the two key halves of each split item: with M the larger reference
@@ -1334,9 +1434,48 @@ const char* flash_split_kernel_name() {
   return name.c_str();
 }
 
+// Key tiles from which a grid of at most one workgroup per CU runs pairs: a
+// pair's second start and its merge cost 1.5-2 us (64 KiB through LDS), and it
+// takes two tiles in the time of 1.5 (with the full bias at head dim 128,
+// whose loads bound it, less). Same box, B=1 H=12, one group -> pair: head dim
+// 128 8 tiles 13.2 -> 13.5 us, 10 15.5 -> 14.9, 16 21.8 -> 20.8, key validity
+// 10 tiles 21.0 -> 19.4, full bias 12 34.3 -> 34.8, 16 44.2 -> 43.5; head dim
+// 64 4 tiles 6.6 -> 7.2, 6 8.1 -> 8.0, 8 9.6 -> 9.2, 16 16.7 -> 13.3, full
+// bias 8 17.5 -> 16.0. 25 tiles at head dim 128 (two key halves on two
+// workgroups before) 33.7 -> 28.7.
+template <int MASK, int D>
+constexpr int kPairMinTiles = D == 64 ? 6 : (MASK & kMaskFull) ? 16 : 10;
+// The rare mask pairs with a key bias keep one group.
+template <int MASK>
+constexpr bool kPairMask = MASK != (kMaskValid | kMaskBias) && !((MASK & kMaskFull) && (MASK & kMaskBias));
+// Key tiles from which such a grid, where it fills at most half the CUs, runs
+// the key halves of its items as two pairs: the partials and the merging
+// launch cost ~10 us (one pair -> two: head dim 64 16 tiles 13.3 -> 15.9 us,
+// head dim 128 16 21.3 -> 22.2, 25 27.3 -> 25.3).
+constexpr int kPairSplitMinTiles = 24;
+
 template <int MASK, int WAVES, int D>
 int launch_one(const FlashArgs& a, hipStream_t stream, const char** launched) {
   const int n_qt = (a.Sq + WAVES * 32 - 1) / (WAVES * 32);
+  if constexpr (WAVES == 4 && kPairMask<MASK>) {
+    // (launched under the planned kernel's name: the host-side plan does not
+    // know the device)
+    const int64_t n = (int64_t)n_qt * a.H * a.B, cus = device_cu_count();
+    const int tiles = (a.Sk + kBN - 1) / kBN;
+    if (n <= cus && tiles >= kPairMinTiles<MASK, D>) {
+      FlashArgs p = a;
+      if (p.split_items != n || 2 * n > cus || tiles < kPairSplitMinTiles) p.split_items = 0;
+      hipLaunchKernelGGL((flash_pair_kernel<MASK, D>), dim3((unsigned)(p.split_items > 0 ? 2 * n : n)), dim3(512), 0,
+                         stream, p, n_qt);
+      if constexpr (!(MASK & (kMaskFull | kMaskBias))) {
+        if (p.split_items > 0)
+          hipLaunchKernelGGL((flash_combine_kernel<D, WAVES>), dim3(p.split_items), dim3(WAVES * 64), 0, stream, p, 0,
+                             n_qt);
+      }
+      *launched = a.split_items > 0 ? flash_split_kernel_name<MASK, D, WAVES>() : flash_kernel_name<MASK, D, WAVES>();
+      return (int)hipGetLastError();
+    }
+  }
   if constexpr (!(MASK & (kMaskFull | kMaskBias))) {  // bias paths are not split
     if (a.split_items > 0) {
     const int n_items = n_qt * a.H * a.B;
