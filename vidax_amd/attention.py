@@ -142,7 +142,7 @@ def _full_bias(bias, B: int, H: int, Sq: int, Sk: int, dev, mask=None) -> Tuple[
         while x.dim() < 4:
             x = x.unsqueeze(0)
         if x.dim() != 4 or any(x.shape[i] not in (1, n) for i, n in enumerate((B, H, Sq, Sk))):
-            raise ValueError(f"{what} of shape {tuple(t.shape)} is not broadcastable to (B, H, Sq, Sk) = "
+            raise ValueError(f"{what} of shape {tuple(x.shape)} is not broadcastable to (B, H, Sq, Sk) = "
                              f"({B}, {H}, {Sq}, {Sk})")
         return x
 
