@@ -471,3 +471,24 @@ def test_per_head_norm_takes_any_weight_view(gpu):
         assert torch.equal(na3d_qk_norm_rope(x, w, None), na3d_qk_norm_rope(x, plain, None))
         y = x.reshape(1, -1, 3, 64)
         assert torch.equal(rms_norm(y, w), rms_norm(y, plain))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,D", [(1, 64), (3, 64), (4, 64), (3, 128), (30, 64)])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (2, 1, 3, 7), (1, 3, 17, 29)])
+@pytest.mark.parametrize("rope,post", [(True, 1.0), (False, 0.125), (True, 0.125)])
+def test_per_head_norm_of_ragged_rows(gpu, H, D, shape, rope, post):
+    """Rows that are no multiple of 512 values run one chunk per lane over all
+    rows; the same heads inside rows that are (the one-wave-per-row kernel) must
+    give the same bits."""
+    from vidax_amd import create_abs_rope3d_freqs, na3d_qk_norm_rope
+    print(f"[case] ragged rows H={H} D={D} {shape} rope={rope} post={post}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(4)
+    H2 = -(-H * D // 512) * 512 // D
+    wide = torch.randn((*shape, H2, D), generator=g, device=gpu).to(torch.bfloat16)
+    w = 1.0 + 0.3 * torch.randn(D, generator=g, device=gpu)
+    freqs = create_abs_rope3d_freqs(*shape[1:], D, device=gpu) if rope else None
+    a = na3d_qk_norm_rope(wide[..., :H, :].contiguous(), w, freqs, post_scale=post)
+    b = na3d_qk_norm_rope(wide, w, freqs, post_scale=post)
+    torch.cuda.synchronize()
+    assert torch.equal(a, b[..., :H, :])

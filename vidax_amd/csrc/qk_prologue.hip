@@ -184,6 +184,60 @@ __global__ __launch_bounds__(kWavesPerBlock * 64) void qk_prologue_kernel(const 
   }
 }
 
+// The per-head norm of rows that are no whole number of 1 KiB wave accesses
+// (num_heads * head_dim not a multiple of 512): one 16-byte chunk per lane over
+// the chunks of all rows in order, so that no lane idles (a wave per row left
+// half of them idle at 256 values: the block at 33x88x160 NH=4 D=64 (11,11,11)
+// 1664 -> 1599 us). A head's head_dim / 8 lanes stay an aligned
+// group, as rows hold whole heads. Memory-bound: kFlat chunks per lane in
+// flight, a grid's width apart. Needs rows * chunks per row < 2^31 - 2^24.
+constexpr int kFlat = 4;
+__global__ __launch_bounds__(256) void qk_prologue_flat_kernel(const PrologueArgs a) {
+  const uint32_t n_chunks = (uint32_t)(a.H * a.D / 8);
+  const uint32_t total = (uint32_t)a.B * (uint32_t)a.S * n_chunks;
+  const uint32_t stride = gridDim.x * 256;
+  const float ps = (float)to_bf16(a.post_scale);
+  const int hpos = (int)((threadIdx.x * 8) % (uint32_t)a.D);  // (256 chunks are a whole number of heads)
+  bf16x8 wb;
+  {
+    const f32x4 w0 = *(const f32x4*)(a.weight + hpos), w1 = *(const f32x4*)(a.weight + hpos + 4);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) wb[e] = to_bf16(e < 4 ? w0[e] : w1[e - 4]);
+  }
+  for (uint32_t g0 = blockIdx.x * 256 + threadIdx.x; g0 - threadIdx.x % 64 < total; g0 += kFlat * stride) {
+    bf16x8 v[kFlat];
+    f32x4 cs[kFlat], sn[kFlat];
+    int64_t out[kFlat];
+#pragma unroll
+    for (int u = 0; u < kFlat; ++u) {
+      const uint32_t g = min(g0 + u * stride, total - 1);  // (past the end: the last chunk, not stored)
+      const uint32_t row = g / n_chunks, c = g - row * n_chunks;
+      const uint32_t b = row / (uint32_t)a.S, s = row - b * (uint32_t)a.S;
+      v[u] = __builtin_nontemporal_load((const bf16x8*)((const bf16*)a.x + b * a.x_bstride + s * a.x_sstride + c * 8));
+      out[u] = b * a.o_bstride + s * a.o_sstride + c * 8;
+      if (a.cos != nullptr) {
+        cs[u] = *(const f32x4*)(a.cos + s * a.tab_stride + hpos / 2);
+        sn[u] = *(const f32x4*)(a.sin + s * a.tab_stride + hpos / 2);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kFlat; ++u) {
+      const float rinv = rms_inv(group_sum(sum_sq8(v[u]), a.D / 8), a.D, a.eps);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[u][e] = rms_elem((float)v[u][e], rinv, (float)wb[e]);
+      if (a.post_scale != 1.0f) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[u][e] = scale_elem((float)v[u][e], ps);
+      }
+      if (a.cos != nullptr) {
+#pragma unroll
+        for (int p = 0; p < 4; ++p) rope_pair(v[u], p, cs[u][p], sn[u][p]);
+      }
+      if (g0 + u * stride < total) __builtin_nontemporal_store(v[u], (bf16x8*)((bf16*)a.out + out[u]));
+    }
+  }
+}
+
 template <int NCHUNK, bool FULL, bool PER_HEAD>
 const char* prologue_kernel_name() {
   static const std::string name = "qk_prologue_kernel<" + std::to_string(NCHUNK) + ", " + (FULL ? "true" : "false") +
@@ -241,6 +295,14 @@ int launch(const PrologueArgs& a, hipStream_t st, const char** launched) {
 
 int launch_qk_prologue(const PrologueArgs& a, void* stream, const char** launched) {
   hipStream_t st = (hipStream_t)stream;
+  const int64_t chunks = (int64_t)a.B * a.S * (a.H * a.D / 8);
+  if (a.per_head && a.weight != nullptr && (a.H * a.D) % 512 != 0 && chunks < ((int64_t)1 << 31) - (1 << 24)) {
+    const int64_t cus = device_cu_count() > 0 ? device_cu_count() : 256;
+    const int64_t groups = std::min((chunks + kFlat * 256 - 1) / (kFlat * 256), cus * 8);
+    hipLaunchKernelGGL(qk_prologue_flat_kernel, dim3((unsigned)groups), dim3(256), 0, st, a);
+    *launched = "qk_prologue_flat_kernel";
+    return (int)hipGetLastError();
+  }
   switch ((a.H * a.D / 8 + 63) / 64) {  // chunks per lane
     case 1: return launch<1>(a, st, launched);
     case 2: return launch<2>(a, st, launched);
