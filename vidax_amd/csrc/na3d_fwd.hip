@@ -426,20 +426,15 @@ void na3d_wave_kernel(const Na3dArgs a, int n_yb, int n_xb, int n_xg) {
 // TSTACK: 2 (t) x 4 (y) x 16 (x) bricks whose four 4 y x 8 x waves sit two
 // per t plane: one stream of (kt' + 1) planes serves both planes' waves, each
 // scoring only the chunks of its own kt' planes.
-// QUAD: tall bricks whose four waves sit two by two, each 4 y x 8 x (kw' <=
-// 9): at a (3,7,7) window a wave scores 10 of a plane's 14 rows, 480 keys per
-// query against 672 for 8 y x 4 x waves, and a row is staged in 24 slots
-// instead of 32. The steps are as many, so it pays once the grid keeps the
-// CUs busy (kNaQuadMinGroups).
 // FEW: the pipelined form for the 1 x 4 x 32 bricks at head dim 64 and the
 // t-stacked bricks too, for grids that two workgroups per CU hold
 // (kNaFewGroups): a wave then has no others to overlap with.
-template <int SEG, int D, bool TALL = false, bool WIDE = false, bool DEEP = false, bool TSTACK = false, bool QUAD = false,
+template <int SEG, int D, bool TALL = false, bool WIDE = false, bool DEEP = false, bool TSTACK = false,
           bool FEW = false>
 struct PipeCfg {
   static constexpr bool kBlock = ((D == 64 && SEG == 16) || TSTACK) && !FEW;  // block form of the step
   static constexpr bool kHalfStep = WIDE;                           // the two waves of a SIMD half a step apart
-  static constexpr bool kSkip = TSTACK || QUAD;                     // a wave skips chunks outside its t (y) window
+  static constexpr bool kSkip = TSTACK;                             // a wave skips chunks outside its t window
   // block form: row sums of the unrounded probabilities (their x window a
   // mask per score), or, for the tall bricks, of the packed bf16 ones
   static constexpr bool kSumF32 = !TALL;
@@ -447,13 +442,12 @@ struct PipeCfg {
   static_assert(!WIDE || TALL, "wide bricks are tall bricks");
   static_assert(!DEEP || WIDE, "deep bricks are wide bricks");
   static_assert(!TSTACK || (!TALL && SEG == 16), "t-stacked bricks hold 1 x 4 x 8 waves on 16-key segments");
-  static_assert(!QUAD || (TALL && !WIDE && D == 64), "quad bricks are narrow tall bricks at head dim 64");
   static_assert(!kHalfStep || kBlock, "the half-step barriers are between the block form's blocks");
   static constexpr int kWaves = WIDE ? 8 : 4;
   static constexpr int kThreads = kWaves * 64;
   static constexpr int kQT = DEEP || TSTACK ? 2 : 1;     // t planes per brick
   static constexpr int kWT = DEEP ? 2 : 1;               // t planes per wave
-  static constexpr int kWX = TSTACK || QUAD ? kWaves / 2 : kWaves;  // waves side by side in x
+  static constexpr int kWX = TSTACK ? kWaves / 2 : kWaves;  // waves side by side in x
   static constexpr int kBrickY = TALL ? (DEEP ? 4 : 8) : 4;
   static constexpr int kBrickX = TALL ? (WIDE ? 32 : 16) : (TSTACK ? 16 : 32);
   static constexpr int kQX = kBrickX / kWX;              // x columns per wave
@@ -461,7 +455,7 @@ struct PipeCfg {
   static constexpr int kRB = D * 2;                      // bytes of one key
   static constexpr int kRows = SEG == 16 ? 2 : 1;        // key rows per step
   // key slots per LDS row (>= kBrickX - kQX + SEG, a multiple of 8)
-  static constexpr int kNS = TALL ? (WIDE ? 48 : QUAD ? 24 : 32) : (TSTACK ? 24 : (SEG == 16 ? 40 : 64));
+  static constexpr int kNS = TALL ? (WIDE ? 48 : 32) : (TSTACK ? 24 : (SEG == 16 ? 40 : 64));
   // An LDS key row is D/64 half-planes of kNS slots x 128 bytes (d 0-63,
   // then d 64-127); one 1 KiB DMA copy fills 8 slots of one half-plane.
   static constexpr int kHalfL = kNS * 128;               // one half-plane of a row
@@ -482,11 +476,11 @@ struct PipeCfg {
   static_assert(kNS % kKeysPerCopy == 0 && kHalfL % 256 == 0, "whole copies per row, bank-aligned planes");
 };
 
-template <int SEG, int D, bool TALL, bool WIDE = false, bool DEEP = false, bool TSTACK = false, bool QUAD = false,
+template <int SEG, int D, bool TALL, bool WIDE = false, bool DEEP = false, bool TSTACK = false,
           bool FEW = false>
 __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int n_xb, unsigned char* smem) {
-  using C = PipeCfg<SEG, D, TALL, WIDE, DEEP, TSTACK, QUAD, FEW>;
-  static_assert(C::kQY * (QUAD ? 2 : 1) == C::kBrickY, "the waves of a brick cover its y rows");
+  using C = PipeCfg<SEG, D, TALL, WIDE, DEEP, TSTACK, FEW>;
+  static_assert(C::kQY == C::kBrickY, "the waves of a brick cover its y rows");
   static_assert(C::kBrickX - C::kQX + SEG <= C::kNS, "a wave's segment stays inside the LDS row");
   VX_LDS unsigned char* const lds = (VX_LDS unsigned char*)smem;
   const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
@@ -548,16 +542,15 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
   const int n_steps = (nrows + C::kRows - 1) / C::kRows;
 
   // ---- this wave's queries: t planes tw..tw+kWT-1 (tw = t, or t + 1 for the
-  // second pair of t-stacked waves), y rows yw..yw+kQY-1 (yw = y0, or y0 + 4
-  // for the second pair of quad waves), x columns xq0..xq0+kQX-1.
-  const int tw = QUAD ? t : t + wave / C::kWX;
-  const int yw = QUAD ? y0 + wave / C::kWX * C::kQY : y0;
+  // second pair of t-stacked waves), y rows y0..y0+kQY-1, x columns
+  // xq0..xq0+kQX-1.
+  const int tw = t + wave / C::kWX;
   const int xq0 = x0 + C::kQX * (wave % C::kWX);
   const int ox = uni(window_start(min(xq0, W - 1), W, kw) - X_lo);  // wave's first x slot, <= kBrickX - kQX
 
   // ---- this lane's query and its window.
-  const int tq = tw + col / (C::kQX * C::kQY), yq = yw + col / C::kQX % C::kQY, xq = xq0 + col % C::kQX;
-  const bool wave_in = yw < Hs && xq0 < W && tw < T;  // wave-uniform: some query of the wave is in the grid
+  const int tq = tw + col / (C::kQX * C::kQY), yq = y0 + col / C::kQX % C::kQY, xq = xq0 + col % C::kQX;
+  const bool wave_in = y0 < Hs && xq0 < W && tw < T;  // wave-uniform: some query of the wave is in the grid
   const int tqc = min(tq, T - 1), yqc = min(yq, Hs - 1), xqc = min(xq, W - 1);
   const int sy = window_start(yqc, Hs, kh) - Y_lo;
   const int st = window_start(tqc, T, kt) - t_lo;  // (deep bricks: the lane's first plane in the box)
@@ -797,15 +790,13 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
 
   // Whether some row of chunk c (rows r) lies in this wave's t window
   // (t-stacked bricks: st is the wave's first plane in the box, its lanes
-  // share one t plane) or in the union of its y windows (quad bricks).
+  // share one t plane).
   const int st_w = TSTACK ? uni(st) : 0;
-  const int sy_w = QUAD ? uni(window_start(min(yw, Hs - 1), Hs, kh) - Y_lo) : 0;
-  const int ny_w = QUAD ? uni(window_start(min(yw + C::kQY - 1, Hs - 1), Hs, kh) - Y_lo) + kh - sy_w : 0;
   auto chunk_active = [&](const StepRows& r, int c) -> bool {
     if constexpr (!C::kSkip) return true;
     const int r0 = c * C::kRows;
-    const bool in0 = QUAD ? (unsigned)(r.yr0 - sy_w) < (unsigned)ny_w : (unsigned)(r.tr0 - st_w) < (unsigned)kt;
-    const bool in1 = QUAD ? (unsigned)(r.yr1 - sy_w) < (unsigned)ny_w : (unsigned)(r.tr1 - st_w) < (unsigned)kt;
+    const bool in0 = (unsigned)(r.tr0 - st_w) < (unsigned)kt;
+    const bool in1 = (unsigned)(r.tr1 - st_w) < (unsigned)kt;
     return (r0 < nrows && in0) || (r0 + 1 < nrows && in1);
   };
 
@@ -1130,7 +1121,7 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
 
   const float lt = halves_sum(l_run);
   const float inv = lt > 0.f ? 1.0f / lt : 0.f;
-  store_na_rows<kDB, C::kQX, C::kQY>(O, inv, og, tok_stride, tw, yw, xq0, T, Hs, W, lane);
+  store_na_rows<kDB, C::kQX, C::kQY>(O, inv, og, tok_stride, tw, y0, xq0, T, Hs, W, lane);
 }
 
 // Head dim 64: three waves per SIMD for the 32-key segments (three 32 KiB
@@ -1149,23 +1140,16 @@ void na3d_pipe_kernel(const Na3dArgs a, int n_yb, int n_xb) {
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void na3d_pipe_few_kernel(const Na3dArgs a, int n_yb, int n_xb) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[PipeCfg<16, 64>::kSmem];
-  na3d_pipe_body<16, 64, false, false, false, false, false, true>(a, n_yb, n_xb, smem);
+  na3d_pipe_body<16, 64, false, false, false, false, true>(a, n_yb, n_xb, smem);
 }
 
 // Head dim 64: four waves per SIMD (at most 128 VGPRs; the workgroup's 32 KiB
 // of LDS allows four per CU), so that more workgroups cover each other's
 // per-step waits: 2.56 -> 2.31 ms at the (11, 11, 11) window on 33x88x160.
-// quad: the 2 x 2 waves of 4 y x 8 x (head dim 64, kw' <= 9).
 template <int D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : 2, D == 64 ? 4 : 2)))
-void na3d_tall_kernel(const Na3dArgs a, int n_yb, int n_xb, int quad) {
+void na3d_tall_kernel(const Na3dArgs a, int n_yb, int n_xb) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[PipeCfg<16, D, true>::kSmem];
-  if constexpr (D == 64) {
-    if (quad) {
-      na3d_pipe_body<16, D, true, false, false, false, true>(a, n_yb, n_xb, smem);
-      return;
-    }
-  }
   na3d_pipe_body<16, D, true>(a, n_yb, n_xb, smem);
 }
 
@@ -1201,14 +1185,9 @@ void na3d_tstack_kernel(const Na3dArgs a, int n_yb, int n_xb) {
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void na3d_tstack_few_kernel(const Na3dArgs a, int n_yb, int n_xb) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[PipeCfg<16, 128, false, false, false, true>::kSmem];
-  na3d_pipe_body<16, 128, false, false, false, true, false, true>(a, n_yb, n_xb, smem);
+  na3d_pipe_body<16, 128, false, false, false, true, true>(a, n_yb, n_xb, smem);
 }
 
-// Workgroups from which the tall bricks at head dim 64 with kw' <= 9 take the
-// 2 x 2 waves (12 per CU). Same box, (3,7,7) windows, 8 x 4 -> 4 x 8 waves:
-// 720 workgroups 24.1 -> 24.8 us, 1296 37.3 -> 39.6, 1680 46.2 -> 47.0, 2592
-// 68.2 -> 68.2, 15120 458 -> 425; 4080 at (5,9,9) 182 -> 170.
-constexpr int64_t kNaQuadMinGroups = 3072;
 // Workgroups up to which the 1 x 4 x 32 bricks at head dim 64 run pipelined
 // steps: two per CU. Same box, block -> pipelined, 11 x 20 planes: 240
 // workgroups at (3,7,7) 12.5 -> 11.2 us, 480 15.1 -> 13.5, 600 17.7 -> 22.0,
@@ -1226,11 +1205,10 @@ int launch_na3d_fwd(const Na3dArgs& a, void* stream, const char** launched) {
       const int n_xb = (a.W + 15) / 16;
       dim3 grid((unsigned)a.T * n_yb * n_xb, a.NH, a.B);
       if (a.D == 128) {
-        hipLaunchKernelGGL((na3d_tall_kernel<128>), grid, dim3(256), 0, st, a, n_yb, n_xb, 0);
+        hipLaunchKernelGGL((na3d_tall_kernel<128>), grid, dim3(256), 0, st, a, n_yb, n_xb);
         *launched = "na3d_tall_kernel<128>";
       } else {
-        const int quad = a.kw <= 9 && (int64_t)grid.x * grid.y * grid.z >= kNaQuadMinGroups;
-        hipLaunchKernelGGL((na3d_tall_kernel<64>), grid, dim3(256), 0, st, a, n_yb, n_xb, quad);
+        hipLaunchKernelGGL((na3d_tall_kernel<64>), grid, dim3(256), 0, st, a, n_yb, n_xb);
         *launched = "na3d_tall_kernel<64>";
       }
       return (int)hipGetLastError();
