@@ -161,3 +161,30 @@ def test_masked_calls_under_graph_capture(gpu):
         torch.cuda.synchronize()
         for a, b in zip(outs, eager):
             assert torch.equal(a, b), step
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Sk", [2 ** 31 - 100, 2 ** 31 - 1])
+def test_masks_of_the_longest_rows(gpu, Sk):
+    """seq_k up to 2^31 - 1: the key counters run past 2^31 (round_up(seq_k,
+    64) and the step behind the last pass), so they are 64-bit. The inputs are
+    one element read at key stride 0."""
+    print(f"[case] mask rows of {Sk} keys", flush=True)
+    L = _lib.lib()
+    width = (Sk + 63) // 64 * 64
+    stream = torch.cuda.current_stream().cuda_stream
+    one = torch.ones(1, dtype=torch.uint8, device=gpu)
+    rows = torch.full((width,), 7, dtype=torch.uint8, device=gpu)
+    kv_len = torch.zeros(1, dtype=torch.int32, device=gpu)
+    _lib.raise_for(L.vx_key_masks_fwd(one.data_ptr(), _lib.strides2((0, 0)), None, None, 1, Sk, kv_len.data_ptr(),
+                                      rows.data_ptr(), None, width, stream))
+    torch.cuda.synchronize()
+    assert kv_len.item() == Sk
+    assert (rows[:Sk] == 1).all() and (rows[Sk:] == 0).all()
+    del rows
+    bias = torch.full((1,), 2.5, device=gpu)
+    out = torch.full((width,), 7.0, device=gpu)
+    zero = (ctypes.c_int64 * 4)(0, 0, 0, 0)
+    _lib.raise_for(L.vx_full_bias_fwd(bias.data_ptr(), zero, None, None, 1, 1, 1, Sk, out.data_ptr(), stream))
+    torch.cuda.synchronize()
+    assert (out[:Sk] == 2.5).all() and (out[Sk:] == 0).all()

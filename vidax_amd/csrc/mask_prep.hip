@@ -28,7 +28,7 @@ constexpr int kKeysPerThread = 16;
 __global__ __launch_bounds__(kKeyThreads) void key_mask_kernel(const KeyMaskArgs a) {
   __shared__ int wave_last[kKeyThreads / 64];
   const int b = blockIdx.x;
-  const int width = (a.Sk + 63) & ~63;
+  const int64_t width = ((int64_t)a.Sk + 63) & ~(int64_t)63;  // (64-bit counters: seq_k goes up to 2^31 - 1)
   const uint8_t* vp = a.valid != nullptr ? a.valid + b * a.valid_strides[0] : nullptr;
   const float* bp = a.bias != nullptr ? a.bias + b * a.bias_strides[0] : nullptr;
   uint8_t* vo = a.valid_rows != nullptr ? a.valid_rows + b * a.row_stride : nullptr;
@@ -36,7 +36,7 @@ __global__ __launch_bounds__(kKeyThreads) void key_mask_kernel(const KeyMaskArgs
   const bool v16 = a.valid_strides[1] == 1 && ((uintptr_t)vp & 15) == 0;
   const bool b16 = a.bias_strides[1] == 1 && ((uintptr_t)bp & 15) == 0;
   int last = 0;
-  for (int k0 = threadIdx.x * kKeysPerThread; k0 < width; k0 += kKeyThreads * kKeysPerThread) {
+  for (int64_t k0 = threadIdx.x * kKeysPerThread; k0 < width; k0 += kKeyThreads * kKeysPerThread) {
     const bool whole = k0 + kKeysPerThread <= a.Sk;
     uint32_t vw[4] = {0, 0, 0, 0};  // validity, one byte (0 or 1) per key
     uint32_t bw[16];                // bias bits
@@ -77,7 +77,7 @@ __global__ __launch_bounds__(kKeyThreads) void key_mask_kernel(const KeyMaskArgs
         if (vp != nullptr) ok = ok && ((vw[i >> 2] >> (8 * (i & 3))) & 0xffu) != 0;
         // above -inf: neither -inf nor NaN (tested on the bits)
         if (bp != nullptr) ok = ok && bw[i] != kNegInfBits && (bw[i] & 0x7fffffffu) <= 0x7f800000u;
-        if (ok) last = k0 + i + 1;
+        if (ok) last = (int)(k0 + i + 1);
       }
     }
   }
@@ -95,17 +95,20 @@ __global__ __launch_bounds__(kKeyThreads) void key_mask_kernel(const KeyMaskArgs
 
 // ---- full bias: rows of round_up(Sk, 64) fp32 values, one per (batch item,
 // head, query) of the broadcast extents, each bias + (mask ? 0 : -inf), the
-// padding 0 (no score there is used). One wave per row, 4 keys per lane and
-// pass; bound by the row stores (4 bytes per score), so nothing is gained by
-// wider loads of a mask byte.
+// padding 0 (no score there is used). One wave per kBiasSeg keys of a row, 4
+// keys per lane and pass; bound by the row stores (4 bytes per score), so
+// nothing is gained by wider loads of a mask byte.
 constexpr int kBiasWaves = 4;
+constexpr int kBiasSeg = 4096;
 
 __global__ __launch_bounds__(kBiasWaves * 64) void full_bias_kernel(const FullBiasArgs a) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t rows = (int64_t)a.n[0] * a.n[1] * a.n[2];
-  const int width = (a.Sk + 63) & ~63;
-  for (int64_t r = (int64_t)blockIdx.x * kBiasWaves + wave; r < rows; r += (int64_t)gridDim.x * kBiasWaves) {
+  const int64_t width = ((int64_t)a.Sk + 63) & ~(int64_t)63;
+  const int64_t n_seg = (width + kBiasSeg - 1) / kBiasSeg, items = (int64_t)a.n[0] * a.n[1] * a.n[2] * n_seg;
+  for (int64_t w = (int64_t)blockIdx.x * kBiasWaves + wave; w < items; w += (int64_t)gridDim.x * kBiasWaves) {
+    const int64_t r = w / n_seg, k_lo = (w - r * n_seg) * kBiasSeg;
+    const int64_t k_hi = min(k_lo + kBiasSeg, width);
     const int64_t bh = r / a.n[2];
     const int q = (int)(r - bh * a.n[2]);
     const int b = (int)(bh / a.n[1]), h = (int)(bh - (int64_t)b * a.n[1]);
@@ -115,11 +118,11 @@ __global__ __launch_bounds__(kBiasWaves * 64) void full_bias_kernel(const FullBi
     const uint8_t* mp =
         a.mask != nullptr ? a.mask + b * a.mask_strides[0] + h * a.mask_strides[1] + q * a.mask_strides[2] : nullptr;
     uint32_t* orow = (uint32_t*)a.out + r * width;
-    for (int k0 = lane * 4; k0 < width; k0 += 256) {
+    for (int64_t k0 = k_lo + lane * 4; k0 < k_hi; k0 += 256) {
       u32x4 o = {0, 0, 0, 0};
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int k = k0 + e;
+        const int64_t k = k0 + e;
         if (k < a.Sk) {
           if (bp != nullptr) o[e] = bp[k * a.bias_strides[3]];
           // x + -inf: -inf, or NaN where x is NaN or +inf
@@ -135,15 +138,16 @@ __global__ __launch_bounds__(kBiasWaves * 64) void full_bias_kernel(const FullBi
 }  // namespace
 
 int launch_key_masks(const KeyMaskArgs& a, void* stream) {
-  const int need = (a.Sk + kKeysPerThread - 1) / kKeysPerThread;
-  const int threads = std::min(kKeyThreads, (need + 63) / 64 * 64);
+  const int64_t need = ((int64_t)a.Sk + kKeysPerThread - 1) / kKeysPerThread;
+  const int threads = (int)std::min<int64_t>(kKeyThreads, (need + 63) / 64 * 64);
   hipLaunchKernelGGL(key_mask_kernel, dim3(a.B), dim3(threads), 0, (hipStream_t)stream, a);
   return (int)hipGetLastError();
 }
 
 int launch_full_bias(const FullBiasArgs& a, void* stream) {
-  const int64_t rows = (int64_t)a.n[0] * a.n[1] * a.n[2];
-  const int64_t groups = std::min<int64_t>((rows + kBiasWaves - 1) / kBiasWaves, 8192);
+  const int64_t n_seg = ((int64_t)a.Sk + kBiasSeg - 1) / kBiasSeg;
+  const int64_t items = (int64_t)a.n[0] * a.n[1] * a.n[2] * n_seg;
+  const int64_t groups = std::min<int64_t>((items + kBiasWaves - 1) / kBiasWaves, 8192);
   hipLaunchKernelGGL(full_bias_kernel, dim3((unsigned)groups), dim3(kBiasWaves * 64), 0, (hipStream_t)stream, a);
   return (int)hipGetLastError();
 }
