@@ -188,3 +188,42 @@ def test_masks_of_the_longest_rows(gpu, Sk):
     _lib.raise_for(L.vx_full_bias_fwd(bias.data_ptr(), zero, None, None, 1, 1, 1, Sk, out.data_ptr(), stream))
     torch.cuda.synchronize()
     assert (out[:Sk] == 2.5).all() and (out[Sk:] == 0).all()
+
+
+def _neg_view(x):
+    """x's values in a view whose memory holds them negated (the imaginary
+    part of a conjugate, as torch gives it)."""
+    y = torch.complex(torch.zeros_like(x), -x).conj().imag
+    assert y.is_neg() and torch.equal(y, x)
+    return y
+
+
+def test_as_dtype_resolves_negated_views():
+    x = torch.arange(6.0).reshape(2, 3)
+    y = _lib.as_dtype(_neg_view(x), x.device, torch.float32)
+    assert not y.is_neg() and torch.equal(y, x)
+    assert _lib.as_dtype(x, x.device, torch.float32) is x
+
+
+@pytest.mark.gpu
+def test_negated_views(gpu):
+    """Biases, norm weights and rope tables given as views that torch marks as
+    negated count with their values, not with what their memory holds."""
+    from vidax_amd import (create_abs_rope3d_freqs, dot_product_attention, flash_attention, na3d_qk_norm_rope,
+                           rms_norm)
+    print("[case] negated views", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(6)
+    q, k, v = (torch.randn((1, 64, 2, 64), generator=g, device=gpu).to(torch.bfloat16) for _ in range(3))
+    kb = torch.randn((1, 1, 1, 64), generator=g, device=gpu)
+    fb = torch.randn((1, 2, 64, 64), generator=g, device=gpu)
+    for b in (kb, fb, fb[:, :, :, :1]):
+        assert torch.equal(dot_product_attention(q, k, v, bias=_neg_view(b)), dot_product_attention(q, k, v, bias=b))
+    assert torch.equal(flash_attention(q, k, v, key_bias=_neg_view(kb).reshape(1, 64)),
+                       flash_attention(q, k, v, key_bias=kb.reshape(1, 64)))
+    x = torch.randn((1, 2, 3, 5, 3, 64), generator=g, device=gpu).to(torch.bfloat16)
+    w = torch.randn(64, generator=g, device=gpu)
+    freqs = create_abs_rope3d_freqs(2, 3, 5, 64, device=gpu)
+    assert torch.equal(na3d_qk_norm_rope(x, _neg_view(w), tuple(_neg_view(t) for t in freqs)),
+                       na3d_qk_norm_rope(x, w, freqs))
+    y = x.reshape(1, -1, 3, 64)
+    assert torch.equal(rms_norm(y, _neg_view(w)), rms_norm(y, w))

@@ -228,7 +228,9 @@ def launch(dev: torch.device, entry, *args) -> None:
 
 
 def as_dtype(x, dev: torch.device, dtype: torch.dtype) -> torch.Tensor:
-    """x as a tensor of this dtype on dev (x itself when it is one already)."""
-    if isinstance(x, torch.Tensor) and x.dtype == dtype and x.device == dev:
-        return x
-    return torch.as_tensor(x, device=dev).to(dtype)
+    """x as a tensor of this dtype on dev, its memory holding its values (x
+    itself when it is one already; a view that only marks its values as
+    negated, as the imaginary part of a conjugate does, is copied)."""
+    if not (isinstance(x, torch.Tensor) and x.dtype == dtype and x.device == dev):
+        x = torch.as_tensor(x, device=dev).to(dtype)
+    return x.resolve_neg() if x.is_neg() else x

@@ -146,7 +146,7 @@ def _full_bias(bias, B: int, H: int, Sq: int, Sk: int, dev, mask=None) -> Tuple[
                              f"({B}, {H}, {Sq}, {Sk})")
         return x
 
-    x = expand(bias, "bias").to(torch.float32) if bias is not None else None
+    x = _lib.as_dtype(expand(bias, "bias"), dev, torch.float32) if bias is not None else None
     m = expand(mask, "mask").to(torch.bool) if mask is not None else None
     width = (Sk + 63) // 64 * 64
     if m is None and (x.shape[3] == Sk and x.stride(3) == 1 and Sk == width and x.data_ptr() % 16 == 0 and
@@ -363,7 +363,7 @@ def dot_product_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         if kb is None:
             full = bias
         else:
-            key_bias = kb.to(torch.float32)
+            key_bias = _lib.as_dtype(kb, q.device, torch.float32)
     if mask is not None:
         km = _key_only(torch.as_tensor(mask, device=q.device), B, Sk, "mask")
         if km is None:

@@ -67,10 +67,10 @@ def _check_x(x: torch.Tensor, name: str = "x") -> None:
 def _tables(freqs, seq: int, half: int, device) -> Tuple[torch.Tensor, torch.Tensor, int]:
     cos, sin = freqs
     if half % 4 == 0 and all(isinstance(t, torch.Tensor) and t.dtype == torch.float32 and t.device == device and
-                             t.is_contiguous() and t.numel() == seq * half for t in (cos, sin)):
+                             t.is_contiguous() and t.numel() == seq * half and not t.is_neg() for t in (cos, sin)):
         return cos, sin, half
-    cos = torch.as_tensor(cos, device=device).to(torch.float32).reshape(-1, half)
-    sin = torch.as_tensor(sin, device=device).to(torch.float32).reshape(-1, half)
+    cos = _lib.as_dtype(cos, device, torch.float32).reshape(-1, half)
+    sin = _lib.as_dtype(sin, device, torch.float32).reshape(-1, half)
     if cos.shape[0] != seq or sin.shape[0] != seq:
         raise ValueError(f"rope tables hold {cos.shape[0]} positions, the sequence has {seq}")
     stride = (half + 3) // 4 * 4
