@@ -423,8 +423,13 @@ int32_t vx_na3d_plan(int32_t t, int32_t h, int32_t w, int32_t head_dim, int32_t 
 /*
  * Name of the kernel launched by the last successful vx_*_fwd call on the
  * calling thread ("" before the first), recorded by the launcher from the
- * launched instantiation. For tests and profiling: it observes the launch
- * itself rather than a copy of the launch rule.
+ * launched instantiation (of a call that splits its keys, the attention
+ * kernel, not the merging one). For tests and profiling: it observes the
+ * launch itself rather than a copy of the launch rule. It can differ from the
+ * plans above where the device and the grid decide: grids of at most one
+ * 128-query workgroup per compute unit run flash_pair_kernel<mask_kind,
+ * head_dim> or flash_pair_split_kernel<...>, and neighbourhood grids of few
+ * workgroups na3d_pipe_few_kernel or na3d_tstack_few_kernel.
  */
 const char* vx_last_launch(void);
 

@@ -88,7 +88,8 @@ def test_local_attention(gpu, B, Sq, Sk, H, D, scale, seed):
     q, k, v, _ = O.make_flash_inputs(B, Sq, Sk, H, D, seed)
     out = local_attention(_t(q, gpu), _t(k, gpu), _t(v, gpu), scale=scale)
     torch.cuda.synchronize()
-    assert _lib.last_launch().startswith(("flash_fwd_kernel<0,", "flash_fwd_split_kernel<0,")), _lib.last_launch()
+    assert _lib.last_launch().startswith(("flash_fwd_kernel<0,", "flash_pair_kernel<0,", "flash_pair_split_kernel<0,")), \
+        _lib.last_launch()
     assert out.shape == (B, Sq, H, D) and out.dtype == torch.bfloat16
     ref = O.attention(q, k, v, scale=D ** -0.5 if scale is None else scale)
     _check(out, ref, "oracle")
@@ -487,7 +488,7 @@ def test_flash_eight_wave_two_batch_items(gpu, D):
     _check(out[:, torch.from_numpy(rows).to(gpu)], ref, f"8 waves B=2 D={D}")
 
 
-@pytest.mark.parametrize("shape", [(2, 300, 700, 3), (1, 8192, 1100, 24)], ids=["4 waves", "8 waves"])
+@pytest.mark.parametrize("shape", [(2, 300, 700, 3), (1, 8192, 1100, 24)], ids=["pairs", "8 waves"])
 @pytest.mark.parametrize("D", [128, 64])
 def test_flash_dominant_key_bias(gpu, shape, D):
     """A key bias that dominates the logits (+-40, runs of -inf in the middle
@@ -496,7 +497,8 @@ def test_flash_dominant_key_bias(gpu, shape, D):
     the reference point has to follow the bias, not q.k."""
     from vidax_amd import _lib, flash_attention
     B, Sq, Sk, H = shape
-    name = f"flash_fwd_kernel<2, {D}, {4 if Sq < 1000 else 8}>"
+    # (18 query tiles of 11 key tiles run as pairs)
+    name = f"flash_pair_kernel<2, {D}>" if Sq < 1000 else f"flash_fwd_kernel<2, {D}, 8>"
     _say(f"flash dominant key bias {name} B={B} Sq={Sq} Sk={Sk} H={H} D={D}")
     seed = 130 + (0 if D == 128 else 1) + (0 if Sq < 1000 else 2)
     q, k, v, _ = O.make_flash_inputs(B, Sq, Sk, H, D, seed)
@@ -724,9 +726,14 @@ def _plain_flash(q, k, v, kw, scale=None):
 
 SPLIT_CASES = [
     # B, Sq, Sk, H, D, seed, mask, expected kernel
-    (1, 2048, 1500, 3, 128, 160, None, "flash_fwd_split_kernel<0, 128, 4>"),          # every item split
-    (2, 700, 2100, 2, 128, 161, ("kv_len", 0, 2100), "flash_fwd_split_kernel<0, 128, 4>"),
-    (1, 900, 1100, 3, 64, 162, ("tail_pad", 0, 200), "flash_fwd_split_kernel<1, 64, 4>"),
+    (1, 2048, 1500, 3, 128, 160, None, "flash_pair_split_kernel<0, 128>"),            # every item split, as pairs
+    (2, 700, 2100, 2, 128, 161, ("kv_len", 0, 2100), "flash_pair_split_kernel<0, 128>"),
+    (1, 900, 1600, 3, 64, 162, ("tail_pad", 0, 200), "flash_pair_split_kernel<1, 64>"),
+    (1, 900, 1100, 3, 64, 162, ("tail_pad", 0, 200), "flash_pair_kernel<1, 64>"),     # 18 key tiles: one pair
+    # 4 waves, above one workgroup per CU: 516 items (4 split), 600 items (88 split)
+    (1, 5400, 1100, 12, 128, 164, None, "flash_fwd_split_kernel<0, 128, 4>"),
+    (2, 3200, 1100, 12, 64, 165, ("tail_pad", 0, 200), "flash_fwd_split_kernel<1, 64, 4>"),
+    (2, 3200, 1100, 12, 128, 166, ("kv_len", 0, 1100), "flash_fwd_split_kernel<0, 128, 4>"),
     (1, 8192, 2048, 25, 128, 163, None, "flash_fwd_split_kernel<0, 128, 8>"),         # 800 items: 32 split
 ]
 
@@ -770,7 +777,7 @@ def test_flash_key_bias_is_not_split(gpu):
     tq, tk, tv = _t(q, gpu), _t(k, gpu), _t(v, gpu)
     kb = torch.from_numpy(bias).to(gpu)
     out = flash_attention(tq, tk, tv, key_bias=kb)
-    assert _lib.last_launch() == "flash_fwd_kernel<2, 128, 4>", _lib.last_launch()
+    assert _lib.last_launch() == "flash_pair_kernel<2, 128>", _lib.last_launch()
     plain = _plain_flash(tq, tk, tv, {"key_bias": kb})
     torch.cuda.synchronize()
     _check(out, O.attention(q, k, v, key_bias=bias), "split key_bias vs oracle")
@@ -802,14 +809,14 @@ def test_masked_self_attention_key_valid_patterns(gpu, pattern):
         valid[1, :] = False
     out = masked_self_attention(q, k, v, key_valid=valid).reshape(B, S, H, D)
     launched = _lib.last_launch()
-    assert launched.startswith("flash_fwd_kernel<1, ") or launched.startswith("flash_fwd_split_kernel<1, "), launched
+    assert launched == "flash_pair_kernel<1, 128>", launched
     rows = _rows(S, 64, 41)
     ref = O.attention_rows(_np(q), _np(k), _np(v), rows, key_valid=_np(valid).astype(bool))
     _check(out[:, torch.from_numpy(rows).to(gpu)], ref, f"key_valid {pattern} ({launched})")
     if pattern != "holes":
         by_len = flash_attention(q, k, v, kv_len=_last_valid_plus_one(valid))
         torch.cuda.synchronize()
-        assert _lib.last_launch().startswith(("flash_fwd_kernel<0, ", "flash_fwd_split_kernel<0, "))
+        assert _lib.last_launch() == "flash_pair_kernel<0, 128>", _lib.last_launch()
         same = torch.equal(out, by_len)
         d = (out.float() - by_len.float()).abs()
         print(f"  validity kernel vs kv_len alone: equal={same} max {d.max().item():.3e}", flush=True)
@@ -839,14 +846,14 @@ def test_dot_product_attention_key_bias_forms(gpu, form):
         bias[:, 300:333] = float("-inf")
     out = dot_product_attention(q, k, v, bias=bias[:, None, None, :])
     launched = _lib.last_launch()
-    assert launched.startswith("flash_fwd_kernel<2, "), launched
+    assert launched == "flash_pair_kernel<2, 128>", launched
     rows = _rows(S, 64, 43)
     ref = O.attention_rows(_np(q), _np(k), _np(v), rows, key_bias=_np(bias))
     _check(out[:, torch.from_numpy(rows).to(gpu)], ref, f"key bias form {form} ({launched})")
     if form != "general":
         as_mask = dot_product_attention(q, k, v, mask=(bias > float("-inf"))[:, None, None, :])
         torch.cuda.synchronize()
-        assert _lib.last_launch().startswith(("flash_fwd_kernel<1, ", "flash_fwd_split_kernel<1, "))
+        assert _lib.last_launch() == "flash_pair_kernel<1, 128>", _lib.last_launch()
         d = (out.float() - as_mask.float()).abs()
         print(f"  key bias vs validity mask: equal={torch.equal(out, as_mask)} max {d.max().item():.3e}",
               flush=True)
@@ -873,7 +880,7 @@ def test_flash_pairs(gpu, B, Sq, Sk, H, D, mask, kind):
     """Grids that leave CUs idle run two groups of four waves per query tile,
     each over half of the key tiles, merged in LDS: against the oracle at the
     edges of the rule and of the halves, with every mask form that runs pairs."""
-    from vidax_amd import flash_attention
+    from vidax_amd import _lib, flash_attention
     _say(f"flash pairs B={B} Sq={Sq} Sk={Sk} H={H} D={D} mask={mask} {kind}")
     q, k, v, extra = O.make_flash_inputs(B, Sq, Sk, H, D, 190)
     rng = np.random.default_rng(191)
@@ -892,7 +899,15 @@ def test_flash_pairs(gpu, B, Sq, Sk, H, D, mask, kind):
         extra["bias"][..., 1::7] = -np.inf
     out = flash_attention(_t(q, gpu), _t(k, gpu), _t(v, gpu),
                           **{n: torch.from_numpy(x).to(gpu) for n, x in extra.items()})
+    launched = _lib.last_launch()
     torch.cuda.synchronize()
+    tiles = -(-Sk // 64)
+    m = (1 if "key_valid" in extra else 0) | (2 if "key_bias" in extra else 0) | (4 if "bias" in extra else 0)
+    if tiles < (6 if D == 64 else 16 if m & 4 else 10):
+        want = f"flash_fwd_kernel<{m}, {D}, 4>"
+    else:
+        want = f"flash_pair_{'split_' if tiles >= 24 and not m & 6 else ''}kernel<{m}, {D}>"
+    assert launched == want, (launched, want)
     if "bias" in extra:
         extra["bias"] = np.broadcast_to(extra["bias"], (B, H, Sq, Sk))
     ref = O.attention(q, k, v, **extra)

@@ -88,6 +88,7 @@ def test_key_masks(gpu, Sk, form):
     vn, bn = valid.cpu().numpy(), bias.cpu().numpy()
     for use_v, use_b in ((True, False), (False, True), (True, True)):
         m = _KeyMasks(valid if use_v else None, bias if use_b else None, want_len=True)
+        assert _lib.last_launch() == "key_mask_kernel"
         torch.cuda.synchronize()
         buf = m.buf.cpu().numpy()
         ok = (vn if use_v else True) & ((bn > -np.inf) if use_b else True)
@@ -130,6 +131,8 @@ def test_full_bias(gpu, Sk, bias_shape, mask_shape):
             tb = None if tb is None else tb.transpose(-1, -2).contiguous().transpose(-1, -2)
             tm = None if tm is None else tm.transpose(-1, -2).contiguous().transpose(-1, -2)
         x, st = _full_bias(tb, B, H, Sq, Sk, gpu, tm)
+        if x is not tb:
+            assert _lib.last_launch() == "full_bias_kernel"
         got = torch.as_strided(x, (B, H, Sq, Sk), (*st, 1)).cpu().numpy()
         assert x.data_ptr() % 16 == 0 and all(s % 4 == 0 for s in st)
         assert np.array_equal(got, ref, equal_nan=True)

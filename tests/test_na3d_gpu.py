@@ -55,10 +55,12 @@ NA_CASES = [
 ]
 
 
-def _expected_kernel(H, W, kw, D, T=1, kt=1):
+def _expected_kernel(H, W, kw, D, T=1, kt=1, heads=1):
     """The NA kernel for a clamped x window kw' = min(kw, W) (and t window
-    kt' = min(kt, T)), written out here independently of the library's plan."""
+    kt' = min(kt, T)) on `heads` = B * NH grids, written out here independently
+    of the library's plan and launcher."""
     k = min(kw, W)
+    few = 2 * torch.cuda.get_device_properties(0).multi_processor_count  # two workgroups per CU
     if k <= 9:
         # head dim 64: 1 x 8 x 16 bricks unless they cover more of the y-x
         # plane than the 1 x 4 x 32 ones
@@ -66,8 +68,10 @@ def _expected_kernel(H, W, kw, D, T=1, kt=1):
             return "na3d_tall_kernel<64>"
         # head dim 128 with a t window of 2 or more: bricks two t planes deep
         if D == 128 and min(kt, T) >= 2:
-            return "na3d_tstack_kernel<128>"
-        return f"na3d_pipe_kernel<16, {D}>"
+            groups = heads * -(-T // 2) * -(-H // 4) * -(-W // 16)
+            return "na3d_tstack_few_kernel" if groups <= few else "na3d_tstack_kernel<128>"
+        groups = heads * T * -(-H // 4) * -(-W // 32)
+        return "na3d_pipe_few_kernel" if D == 64 and groups <= few else f"na3d_pipe_kernel<16, {D}>"
     if k <= 13:
         # head dim 64: 32-wide bricks unless they leave more ragged columns
         if D == 64 and -(-W // 32) * 32 == -(-W // 16) * 16:
@@ -85,7 +89,7 @@ def _run(gpu, shape, ks, seed, D):
     q, k, v = O.make_na3d_inputs(B, T, H, W, NH, D, seed)
     out = neighborhood_attention_3d(_t(q, gpu), _t(k, gpu), _t(v, gpu), ks)
     launched = _lib.last_launch()
-    assert launched == _expected_kernel(H, W, ks[2], D, T, ks[0]), launched
+    assert launched == _expected_kernel(H, W, ks[2], D, T, ks[0], B * NH), launched
     torch.cuda.synchronize()
     _check(out.float().cpu().numpy(), O.na3d(q, k, v, ks), f"oracle ({launched})")
 
@@ -181,7 +185,7 @@ def test_na3d_row_offsets(gpu, shift, D, H, W):
     q[:, :, :, ::2, :, 0] = shift
     q[:, :, :, 1::2, :, 0] = 0.0
     out = neighborhood_attention_3d(_t(q, gpu), _t(k, gpu), _t(v, gpu), (3, 7, 7))
-    assert _lib.last_launch() == _expected_kernel(H, W, 7, D, T, 3), _lib.last_launch()
+    assert _lib.last_launch() == _expected_kernel(H, W, 7, D, T, 3, B * NH), _lib.last_launch()
     torch.cuda.synchronize()
     _check(out.float().cpu().numpy(), O.na3d(q, k, v, (3, 7, 7)), "oracle")
 
@@ -255,7 +259,7 @@ def test_na3d_stage5_sampled_rows(gpu):
     B, T, H, W, NH = 1, 33, 88, 160, 4
     q, k, v = O.make_na3d_inputs(B, T, H, W, NH, 64, 5)
     out = neighborhood_attention_3d(_t(q, gpu), _t(k, gpu), _t(v, gpu), (11, 11, 11))
-    assert _lib.last_launch() == _expected_kernel(H, W, 11, 64, T, 11), _lib.last_launch()
+    assert _lib.last_launch() == _expected_kernel(H, W, 11, 64, T, 11, B * NH), _lib.last_launch()
     o = out.float().cpu().numpy()
     rng = np.random.default_rng(55)
     rows = {(0, 0), (32, 87), (16, 7), (16, 8), (5, 44), (27, 80), (1, 86), (31, 3)}
@@ -280,7 +284,7 @@ def test_na3d_wide_window_sampled_rows(gpu):
     B, T, H, W, NH = 1, 21, 45, 80, 24
     q, k, v = O.make_na3d_inputs(B, T, H, W, NH, 128, 6)
     out = neighborhood_attention_3d(_t(q, gpu), _t(k, gpu), _t(v, gpu), (3, 7, 31))
-    assert _lib.last_launch() == _expected_kernel(H, W, 31, 128, T, 3), _lib.last_launch()
+    assert _lib.last_launch() == _expected_kernel(H, W, 31, 128, T, 3, B * NH), _lib.last_launch()
     o = out.float().cpu().numpy()
     rows = [(0, 0), (20, 44), (10, 3), (10, 4), (7, 41), (13, 22)]
     ref = O.na3d(q, k, v, (3, 7, 31), ty_rows=rows)
@@ -306,7 +310,7 @@ def test_na3d_tall_bricks_many_workgroups(gpu, shape, ks, seed):
     assert B * T * -(-H // 8) * -(-W // 16) * NH >= 3072
     out = neighborhood_attention_3d(q, k, v, ks)
     launched = _lib.last_launch()
-    assert launched == "na3d_tall_kernel<64>" == _expected_kernel(H, W, ks[2], 64, T, ks[0]), launched
+    assert launched == "na3d_tall_kernel<64>" == _expected_kernel(H, W, ks[2], 64, T, ks[0], B * NH), launched
     heads = [0, NH // 2 + 1, NH - 1]
     few = [x[..., heads, :].contiguous() for x in (q, k, v)]
     out_few = neighborhood_attention_3d(*few, ks)
@@ -318,24 +322,32 @@ def test_na3d_tall_bricks_many_workgroups(gpu, shape, ks, seed):
 
 @pytest.mark.parametrize("T,H,W,D,window,few,many", [
     (3, 11, 20, 64, (3, 7, 7), 56, 58),     # 1 x 4 x 32 bricks: 504 and 522 workgroups
-    (2, 9, 33, 64, (1, 5, 9), 40, 48),      # one-plane windows, ragged x: 480 and 576
+    (2, 9, 61, 64, (1, 5, 9), 40, 48),      # one-plane windows, ragged x: 480 and 576
     (4, 10, 33, 128, (3, 7, 7), 28, 29),    # t-stacked: 504 and 522
     (3, 7, 17, 128, (2, 5, 9), 64, 66),     # an odd t plane, idle waves: 512 and 528
 ])
 def test_na3d_few_and_many_workgroups(gpu, T, H, W, D, window, few, many):
     """Grids that two workgroups per CU hold run pipelined steps, larger ones
-    block steps. Both score the same keys; the heads of the larger grid repeat
-    those of the smaller one, so each output may differ by the order of fp32
-    sums and one bf16 rounding (2^-7 of a value's binade)."""
-    from vidax_amd import neighborhood_attention_3d
+    block steps: the names tell which, and a few heads of both are checked
+    against the oracle. Both score the same keys; the heads of the larger grid
+    repeat those of the smaller one, so each output may differ by the order of
+    fp32 sums and one bf16 rounding (2^-7 of a value's binade)."""
+    from vidax_amd import _lib, neighborhood_attention_3d
     print(f"[case] na3d few/many {T}x{H}x{W} D={D} {window} NH={few}/{many}", flush=True)
     g = torch.Generator(device=gpu).manual_seed(11)
     x = [torch.randn((1, T, H, W, few, D), generator=g, device=gpu).to(torch.bfloat16) for _ in range(3)]
     x[0] = x[0] * D ** -0.5
     heads = torch.arange(many, device=gpu) % few
     a = neighborhood_attention_3d(*x, window)
+    name_a = _lib.last_launch()
     b = neighborhood_attention_3d(*[t[..., heads, :].contiguous() for t in x], window)
+    name_b = _lib.last_launch()
     torch.cuda.synchronize()
-    a = a[..., heads, :].float()
-    d = (a - b.float()).abs()
-    assert (d <= 2.0 ** -7 * a.abs() + 1e-5).all(), d.max().item()
+    assert name_a == _expected_kernel(H, W, window[2], D, T, window[0], few) and "_few_" in name_a, name_a
+    assert name_b == _expected_kernel(H, W, window[2], D, T, window[0], many) and "_few_" not in name_b, name_b
+    d = (a[..., heads, :].float() - b.float()).abs()
+    assert (d <= 2.0 ** -7 * a[..., heads, :].float().abs() + 1e-5).all(), d.max().item()
+    some = [0, few // 2 + 1, few - 1]
+    ref = O.na3d(*(t[..., some, :].float().cpu().numpy() for t in x), window)
+    _check(a[..., some, :].float().cpu().numpy(), ref, "few vs oracle")
+    _check(b[..., some, :].float().cpu().numpy(), ref, "many vs oracle")

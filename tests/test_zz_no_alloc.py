@@ -35,12 +35,12 @@ def _call(entry, q, k, v, out, kv_len=None, ws=None):
 def test_noalloc_matches_workspace_entry(gpu):
     from vidax_amd import _lib
     cases = [
-        # B, Sq, Sk, H, seed, kv_len: the first splits 220 of 732 items (28 MiB of
-        # scratch), the second every one of its 24 items over a smaller span
-        (1, 7800, 7800, 12, 180, None),
-        (2, 700, 2100, 2, 181, [700, 2100]),
+        # B, Sq, Sk, H, seed, kv_len, kernel: the first splits 220 of 732 items (28 MiB
+        # of scratch), the second every one of its 24 items over a smaller span (as pairs)
+        (1, 7800, 7800, 12, 180, None, "flash_fwd_split_kernel<0, 128, 4>"),
+        (2, 700, 2100, 2, 181, [700, 2100], "flash_pair_split_kernel<0, 128>"),
     ]
-    for B, Sq, Sk, H, seed, kvl in cases:
+    for B, Sq, Sk, H, seed, kvl, kernel in cases:
         print(f"[case] noalloc B={B} Sq={Sq} Sk={Sk} H={H} kv_len={kvl}", flush=True)
         q, k, v, _ = O.make_flash_inputs(B, Sq, Sk, H, 128, seed)
         t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(gpu).to(torch.bfloat16)
@@ -55,7 +55,7 @@ def test_noalloc_matches_workspace_entry(gpu):
         name_ws = _call("ws", tq, tk, tv, out_ws, kv_len, ws)
         torch.cuda.synchronize()
         print(f"  launched {name_na} / {name_ws}", flush=True)
-        assert name_na == name_ws == "flash_fwd_split_kernel<0, 128, 4>"
+        assert name_na == name_ws == kernel
         assert torch.equal(out_na, out_ws), "noalloc output differs from the workspace entry point"
         rows = np.unique(np.linspace(0, Sq - 1, 64).astype(int))
         ref = O.attention(q[:, rows], k, v, kv_len=np.array(kvl, np.int32) if kvl is not None else None)

@@ -769,22 +769,20 @@ void flash_fwd_split_kernel(const FlashArgs a, int n_full, int n_qt) {
 // Two groups of four waves per 128-query tile (flash_tile's PAIR), for grids
 // that leave a CU to each workgroup: the same two waves per SIMD that two
 // workgroups per CU give larger grids, with half the key tiles each, merged in
-// LDS. One workgroup per item, or per half of its keys (a.split_items > 0,
-// every item split).
+// LDS. One workgroup per item.
 template <int MASK, int D>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void flash_pair_kernel(const FlashArgs a, int n_qt) {
-  const int w = blockIdx.x;
-  int item = w, k_lo = 0, k_hi = a.Sk, part = -1;
-  if (a.split_items > 0) {
-    part = w;
-    item = w >> 1;
-    if (part & 1)
-      k_lo = a.k_mid;
-    else
-      k_hi = a.k_mid;
-  }
-  const int qt = item % n_qt, bh = item / n_qt;
+  const int item = blockIdx.x, qt = item % n_qt, bh = item / n_qt;
+  flash_tile<MASK, D, 4, true>(a, qt, bh % a.H, bh / a.H, 0, a.Sk, -1);
+}
+
+// One pair per half of an item's keys (every item split), writing partials.
+template <int MASK, int D>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void flash_pair_split_kernel(const FlashArgs a, int n_qt) {
+  const int part = blockIdx.x, item = part >> 1, qt = item % n_qt, bh = item / n_qt;
+  const int k_lo = part & 1 ? a.k_mid : 0, k_hi = part & 1 ? a.Sk : a.k_mid;
   flash_tile<MASK, D, 4, true>(a, qt, bh % a.H, bh / a.H, k_lo, k_hi, part);
 }
 
@@ -1434,6 +1432,18 @@ const char* flash_split_kernel_name() {
   return name.c_str();
 }
 
+template <int MASK, int D>
+const char* flash_pair_kernel_name() {
+  static const std::string name = "flash_pair_kernel<" + std::to_string(MASK) + ", " + std::to_string(D) + ">";
+  return name.c_str();
+}
+
+template <int MASK, int D>
+const char* flash_pair_split_kernel_name() {
+  static const std::string name = "flash_pair_split_kernel<" + std::to_string(MASK) + ", " + std::to_string(D) + ">";
+  return name.c_str();
+}
+
 // Key tiles from which a grid of at most one workgroup per CU runs pairs: a
 // pair's second start and its merge cost 1.5-2 us (64 KiB through LDS), and it
 // takes two tiles in the time of 1.5 (with the full bias at head dim 128,
@@ -1458,21 +1468,21 @@ template <int MASK, int WAVES, int D>
 int launch_one(const FlashArgs& a, hipStream_t stream, const char** launched) {
   const int n_qt = (a.Sq + WAVES * 32 - 1) / (WAVES * 32);
   if constexpr (WAVES == 4 && kPairMask<MASK>) {
-    // (launched under the planned kernel's name: the host-side plan does not
-    // know the device)
     const int64_t n = (int64_t)n_qt * a.H * a.B, cus = device_cu_count();
     const int tiles = (a.Sk + kBN - 1) / kBN;
     if (n <= cus && tiles >= kPairMinTiles<MASK, D>) {
-      FlashArgs p = a;
-      if (p.split_items != n || 2 * n > cus || tiles < kPairSplitMinTiles) p.split_items = 0;
-      hipLaunchKernelGGL((flash_pair_kernel<MASK, D>), dim3((unsigned)(p.split_items > 0 ? 2 * n : n)), dim3(512), 0,
-                         stream, p, n_qt);
       if constexpr (!(MASK & (kMaskFull | kMaskBias))) {
-        if (p.split_items > 0)
-          hipLaunchKernelGGL((flash_combine_kernel<D, WAVES>), dim3(p.split_items), dim3(WAVES * 64), 0, stream, p, 0,
+        if (a.split_items == n && 2 * n <= cus && tiles >= kPairSplitMinTiles) {
+          hipLaunchKernelGGL((flash_pair_split_kernel<MASK, D>), dim3((unsigned)(2 * n)), dim3(512), 0, stream, a,
                              n_qt);
+          hipLaunchKernelGGL((flash_combine_kernel<D, WAVES>), dim3((unsigned)n), dim3(WAVES * 64), 0, stream, a, 0,
+                             n_qt);
+          *launched = flash_pair_split_kernel_name<MASK, D>();
+          return (int)hipGetLastError();
+        }
       }
-      *launched = a.split_items > 0 ? flash_split_kernel_name<MASK, D, WAVES>() : flash_kernel_name<MASK, D, WAVES>();
+      hipLaunchKernelGGL((flash_pair_kernel<MASK, D>), dim3((unsigned)n), dim3(512), 0, stream, a, n_qt);
+      *launched = flash_pair_kernel_name<MASK, D>();
       return (int)hipGetLastError();
     }
   }

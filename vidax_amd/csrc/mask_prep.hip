@@ -137,18 +137,20 @@ __global__ __launch_bounds__(kBiasWaves * 64) void full_bias_kernel(const FullBi
 
 }  // namespace
 
-int launch_key_masks(const KeyMaskArgs& a, void* stream) {
+int launch_key_masks(const KeyMaskArgs& a, void* stream, const char** launched) {
   const int64_t need = ((int64_t)a.Sk + kKeysPerThread - 1) / kKeysPerThread;
   const int threads = (int)std::min<int64_t>(kKeyThreads, (need + 63) / 64 * 64);
   hipLaunchKernelGGL(key_mask_kernel, dim3(a.B), dim3(threads), 0, (hipStream_t)stream, a);
+  *launched = "key_mask_kernel";
   return (int)hipGetLastError();
 }
 
-int launch_full_bias(const FullBiasArgs& a, void* stream) {
+int launch_full_bias(const FullBiasArgs& a, void* stream, const char** launched) {
   const int64_t n_seg = ((int64_t)a.Sk + kBiasSeg - 1) / kBiasSeg;
   const int64_t items = (int64_t)a.n[0] * a.n[1] * a.n[2] * n_seg;
   const int64_t groups = std::min<int64_t>((items + kBiasWaves - 1) / kBiasWaves, 8192);
   hipLaunchKernelGGL(full_bias_kernel, dim3((unsigned)groups), dim3(kBiasWaves * 64), 0, (hipStream_t)stream, a);
+  *launched = "full_bias_kernel";
   return (int)hipGetLastError();
 }
 

@@ -1236,11 +1236,13 @@ int launch_na3d_fwd(const Na3dArgs& a, void* stream, const char** launched) {
       const int n_yb = (a.Hs + 3) / 4;
       const int n_xb = (a.W + 15) / 16;
       dim3 grid((unsigned)((a.T + 1) / 2) * n_yb * n_xb, a.NH, a.B);
-      if ((int64_t)grid.x * grid.y * grid.z <= kNaFewGroups)
+      if ((int64_t)grid.x * grid.y * grid.z <= kNaFewGroups) {
         hipLaunchKernelGGL(na3d_tstack_few_kernel, grid, dim3(256), 0, st, a, n_yb, n_xb);
-      else
+        *launched = "na3d_tstack_few_kernel";
+      } else {
         hipLaunchKernelGGL((na3d_tstack_kernel<128>), grid, dim3(256), 0, st, a, n_yb, n_xb);
-      *launched = "na3d_tstack_kernel<128>";
+        *launched = "na3d_tstack_kernel<128>";
+      }
       return (int)hipGetLastError();
     }
     case kNaPipe16:
@@ -1254,12 +1256,11 @@ int launch_na3d_fwd(const Na3dArgs& a, void* stream, const char** launched) {
       } else if (a.D == 128) {
         hipLaunchKernelGGL((na3d_pipe_kernel<32, 128>), grid, dim3(256), 0, st, a, n_yb, n_xb);
         *launched = "na3d_pipe_kernel<32, 128>";
+      } else if (a.variant == kNaPipe16 && (int64_t)grid.x * grid.y * grid.z <= kNaFewGroups) {
+        hipLaunchKernelGGL(na3d_pipe_few_kernel, grid, dim3(256), 0, st, a, n_yb, n_xb);
+        *launched = "na3d_pipe_few_kernel";
       } else if (a.variant == kNaPipe16) {
-        // (one name for both: the host-side plan does not know the grid)
-        if ((int64_t)grid.x * grid.y * grid.z <= kNaFewGroups)
-          hipLaunchKernelGGL(na3d_pipe_few_kernel, grid, dim3(256), 0, st, a, n_yb, n_xb);
-        else
-          hipLaunchKernelGGL((na3d_pipe_kernel<16, 64>), grid, dim3(256), 0, st, a, n_yb, n_xb);
+        hipLaunchKernelGGL((na3d_pipe_kernel<16, 64>), grid, dim3(256), 0, st, a, n_yb, n_xb);
         *launched = "na3d_pipe_kernel<16, 64>";
       } else {
         hipLaunchKernelGGL((na3d_pipe_kernel<32, 64>), grid, dim3(256), 0, st, a, n_yb, n_xb);

@@ -610,8 +610,10 @@ int32_t vx_key_masks_fwd(const uint8_t* valid, const int64_t* valid_strides, con
   a.row_stride = row_stride;
   int32_t rc;
   if ((rc = injected()) != VX_OK) return rc;
-  const int err = vx::launch_key_masks(a, stream);
+  const char* launched = "";
+  const int err = vx::launch_key_masks(a, stream, &launched);
   if (err != 0) return fail(VX_ERR_LAUNCH, "key mask launch failed (hipError_t %d)", err);
+  g_last_launch = launched;
   return ok();
 }
 
@@ -644,8 +646,10 @@ int32_t vx_full_bias_fwd(const float* bias, const int64_t* bias_strides, const u
   a.out = out;
   int32_t rc;
   if ((rc = injected()) != VX_OK) return rc;
-  const int err = vx::launch_full_bias(a, stream);
+  const char* launched = "";
+  const int err = vx::launch_full_bias(a, stream, &launched);
   if (err != 0) return fail(VX_ERR_LAUNCH, "full bias launch failed (hipError_t %d)", err);
+  g_last_launch = launched;
   return ok();
 }
 

@@ -162,8 +162,8 @@ int noalloc_scratch(void** ptr, int64_t* bytes);
 int launch_flash_fwd(const FlashArgs& a, void* stream, const char** launched);
 int launch_na3d_fwd(const Na3dArgs& a, void* stream, const char** launched);
 int launch_qk_prologue(const PrologueArgs& a, void* stream, const char** launched);
-int launch_key_masks(const KeyMaskArgs& a, void* stream);    // (no kernel name)
-int launch_full_bias(const FullBiasArgs& a, void* stream);
+int launch_key_masks(const KeyMaskArgs& a, void* stream, const char** launched);
+int launch_full_bias(const FullBiasArgs& a, void* stream, const char** launched);
 
 // Measurement only: n_groups one-wave workgroups each store (XCD id, HW_ID,
 // shader clock counter, real-time counter) as four uint64 at out + 4 * group;
