@@ -28,7 +28,8 @@ extern "C" {
 #define VX_ERR_UNSUPPORTED 2      /* a valid request this build has no kernel for   */
 #define VX_ERR_LAUNCH 3           /* the HIP runtime refused the launch             */
 
-/* Version of this ABI (major * 10000 + minor * 100 + patch): 1.8.0. */
+/* Version of this ABI (major * 10000 + minor * 100 + patch): 1.9.0.
+ * (1.9: the mask preparation entries, the device plan, and head_dim weights for per-head norms.) */
 int32_t vx_abi_version(void);
 
 /* Message describing the most recent failure on the calling thread ("" if none). */
@@ -86,6 +87,10 @@ int32_t vx_flash_attn_fwd(const void* q, const void* k, const void* v, void* out
  * resident ones), the query tiles of that round are each computed as two
  * workgroups over the two halves of the keys, whose fp32 partial results go
  * to the workspace and are merged by a second kernel on the same stream.
+ * A grid of at most half as many 128-query workgroups as the device has
+ * compute units, over at least 24 64-key tiles, splits every query tile so.
+ * (Below, up to one workgroup per compute unit, a tile's keys are halved
+ * inside one workgroup and nothing goes to the workspace.)
  * That needs vx_flash_attn_workspace_size() bytes (0: no split for this
  * shape on this device); with a smaller workspace (or NULL), or with a
  * key_bias, the call runs without the split, as vx_flash_attn_fwd. The workspace must be 16-byte
@@ -410,6 +415,16 @@ int32_t vx_flash_attn_plan(int32_t batch, int32_t seq_q, int32_t seq_k, int32_t 
                            int32_t mask_kind, char* kernel_name, int32_t name_len);
 
 /*
+ * The kernel vx_flash_attn_ws_fwd (with its workspace) or
+ * vx_flash_attn_bias_fwd launches for a shape on a device with num_cus compute
+ * units (host only, no GPU), written as by vx_flash_attn_plan: the plan above,
+ * or flash_fwd_split_kernel<mask_kind, head_dim, waves>, flash_pair_kernel<
+ * mask_kind, head_dim> or flash_pair_split_kernel<mask_kind, head_dim>.
+ */
+int32_t vx_flash_attn_device_plan(int32_t batch, int32_t seq_q, int32_t seq_k, int32_t num_heads, int32_t head_dim,
+                                  int32_t mask_kind, int32_t num_cus, char* kernel_name, int32_t name_len);
+
+/*
  * Launch plan of vx_na3d_fwd (host only): the name of the kernel chosen by
  * the clamped x window (at head dim 64 also by the grid's h and w, which
  * decide the brick shape; and by the clamped t window min(kernel_t, t), which
@@ -425,11 +440,10 @@ int32_t vx_na3d_plan(int32_t t, int32_t h, int32_t w, int32_t head_dim, int32_t 
  * calling thread ("" before the first), recorded by the launcher from the
  * launched instantiation (of a call that splits its keys, the attention
  * kernel, not the merging one). For tests and profiling: it observes the
- * launch itself rather than a copy of the launch rule. It can differ from the
- * plans above where the device and the grid decide: grids of at most one
- * 128-query workgroup per compute unit run flash_pair_kernel<mask_kind,
- * head_dim> or flash_pair_split_kernel<...>, and neighbourhood grids of few
- * workgroups na3d_pipe_few_kernel or na3d_tstack_few_kernel.
+ * launch itself rather than a copy of the launch rule. It can differ from
+ * vx_flash_attn_plan and vx_na3d_plan where the device and the grid decide
+ * (vx_flash_attn_device_plan; neighbourhood grids of few workgroups run
+ * na3d_pipe_few_kernel or na3d_tstack_few_kernel).
  */
 const char* vx_last_launch(void);
 

@@ -32,7 +32,7 @@ def test_header_symbols_are_exported():
 
 
 def test_abi_version():
-    assert _lib.lib().vx_abi_version() == 10800
+    assert _lib.lib().vx_abi_version() == 10900
 
 
 def _flash_check(**kw):
@@ -564,3 +564,34 @@ def test_flash_kernel_name_with_the_key_split():
     assert flash_kernel_name(1, 7800, 7800, 12, 128, 2, num_cus=256) == "flash_fwd_kernel<2, 128, 4>"
     assert flash_kernel_name(1, 32760, 32760, 40, num_cus=256) == "flash_fwd_kernel<0, 128, 8>"   # 5120 tiles
     assert flash_kernel_name(2, 32760, 512, 40, num_cus=256) == "flash_stream_kernel<128>"
+
+
+def test_pairs_in_the_plan():
+    """4-wave grids of at most one workgroup per compute unit run pairs, and
+    only those that split (both halves' pairs on a unit each, 24 key tiles and
+    more, no bias) ask for a workspace. 2 heads x 52 query tiles = 104 items."""
+    from vidax_amd.attention import flash_kernel_name
+    part = 4 * 64 * (4 * 16 + 2) * 4
+    assert _split((1, 6650, 23 * 64, 2, 128)) == (0, 0, 0)
+    assert _split((1, 6650, 24 * 64, 2, 128)) == (104, 12 * 64, 2 * 104 * part)
+    assert _split((1, 16384, 1600, 1, 128)) == (128, 12 * 64, 2 * 128 * part)   # n = CUs / 2
+    assert _split((1, 16385, 1600, 1, 128)) == (0, 0, 0)                        # n = CUs / 2 + 1
+    assert _split((1, 1560, 1560, 12, 128)) == (0, 0, 0)                        # 156 items: one pair each
+    assert _split((1, 32768, 1600, 1, 128)) == (0, 0, 0)                        # n = CUs
+    assert _split((1, 32769, 1600, 1, 128)) == (0, 0, 0)                        # n = CUs + 1: a round above half full
+    assert _split((1, 65664, 1600, 1, 128)) == (1, 12 * 64, 2 * part)           # 513 items: one split
+
+    def name(Sq, Sk, H, D=128, mask=0, cus=256):
+        return flash_kernel_name(1, Sq, Sk, H, D, mask, num_cus=cus)
+    assert name(6650, 24 * 64, 2) == "flash_pair_split_kernel<0, 128>"
+    assert name(6650, 23 * 64, 2) == "flash_pair_kernel<0, 128>"
+    assert name(6650, 24 * 64, 2, mask=2) == "flash_pair_kernel<2, 128>"
+    assert name(6650, 24 * 64, 2, mask=3) == "flash_fwd_kernel<3, 128, 4>"
+    assert name(6650, 24 * 64, 2, mask=6) == "flash_fwd_kernel<6, 128, 4>"
+    assert name(6650, 24 * 64, 2, cus=104) == "flash_pair_kernel<0, 128>"
+    assert name(6650, 24 * 64, 2, cus=103) == "flash_fwd_kernel<0, 128, 4>"   # 104 of 206 slots
+    assert name(32769, 1600, 1) == "flash_fwd_kernel<0, 128, 4>"
+    assert name(200, 64 * 10, 4) == "flash_pair_kernel<0, 128>" and name(200, 64 * 9, 4) == "flash_fwd_kernel<0, 128, 4>"
+    assert name(200, 64 * 6, 4, 64) == "flash_pair_kernel<0, 64>" and name(200, 64 * 5, 4, 64) == "flash_fwd_kernel<0, 64, 4>"
+    assert name(200, 64 * 16, 4, mask=4) == "flash_pair_kernel<4, 128>"
+    assert name(200, 64 * 15, 4, mask=4) == "flash_fwd_kernel<4, 128, 4>"

@@ -9,6 +9,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+from typing import Optional
 
 import torch  # noqa: F401  (must precede the dlopen below)
 
@@ -47,6 +48,7 @@ EXPORTED_SYMBOLS = (
     "vx_debug_clock_stamp",
     "vx_key_masks_fwd",
     "vx_full_bias_fwd",
+    "vx_flash_attn_device_plan",
 )
 
 _lock = threading.Lock()
@@ -120,6 +122,8 @@ def lib() -> ctypes.CDLL:
             h.vx_debug_inject_error.argtypes = [_i32]
             h.vx_flash_attn_plan.restype = _i32
             h.vx_flash_attn_plan.argtypes = [_i32] * 6 + [ctypes.c_char_p, _i32]
+            h.vx_flash_attn_device_plan.restype = _i32
+            h.vx_flash_attn_device_plan.argtypes = [_i32] * 7 + [ctypes.c_char_p, _i32]
             h.vx_na3d_plan.restype = _i32
             h.vx_na3d_plan.argtypes = [_i32] * 7 + [ctypes.c_char_p, _i32]
             h.vx_na3d_qprep_fwd.restype = _i32
@@ -160,10 +164,16 @@ def last_launch() -> str:
     return lib().vx_last_launch().decode("utf-8", "replace")
 
 
-def flash_plan(batch: int, seq_q: int, seq_k: int, num_heads: int, head_dim: int, mask_kind: int) -> str:
-    """Kernel vx_flash_attn_fwd would launch for this shape (host-side plan)."""
+def flash_plan(batch: int, seq_q: int, seq_k: int, num_heads: int, head_dim: int, mask_kind: int,
+               num_cus: Optional[int] = None) -> str:
+    """Kernel of this shape from the host-side plan: by tile size alone or, with
+    the device's compute units, as vx_flash_attn_ws_fwd launches it."""
     buf = ctypes.create_string_buffer(64)
-    raise_for(lib().vx_flash_attn_plan(batch, seq_q, seq_k, num_heads, head_dim, mask_kind, buf, 64))
+    shape = (batch, seq_q, seq_k, num_heads, head_dim, mask_kind)
+    if num_cus is None:
+        raise_for(lib().vx_flash_attn_plan(*shape, buf, 64))
+    else:
+        raise_for(lib().vx_flash_attn_device_plan(*shape, num_cus, buf, 64))
     return buf.value.decode()
 
 

@@ -280,22 +280,14 @@ def flash_kernel_name(batch: int, seq_q: int, seq_k: int, num_heads: int, head_d
     launch plan: the gfx950 tile table or VIDAX_FLASH_BLOCK_SIZES). mask_kind:
     1 key validity, 2 key bias, 4 full bias (bits).
 
-    Without num_cus: the kernel of vx_flash_attn_fwd, which never splits its
-    keys. With num_cus (the device's compute units): the kernel of
-    vx_flash_attn_ws_fwd given its workspace, as flash_attention calls it,
-    i.e. flash_fwd_split_kernel<...> for the grids whose last round the key
-    split evens out (vx_flash_attn_split_plan; never with a key or full bias)."""
-    name = _lib.flash_plan(int(batch), int(seq_q), int(seq_k), int(num_heads), int(head_dim), int(mask_kind))
-    if num_cus is not None and int(mask_kind) in (0, 1) and name.startswith("flash_fwd_kernel<"):
-        items = ctypes.c_int32(0)
-        key = ctypes.c_int32(0)
-        nbytes = ctypes.c_int64(0)
-        _lib.raise_for(_lib.lib().vx_flash_attn_split_plan(int(batch), int(seq_q), int(seq_k), int(num_heads),
-                                                           int(head_dim), int(num_cus), ctypes.byref(items),
-                                                           ctypes.byref(key), ctypes.byref(nbytes)))
-        if items.value > 0:
-            name = name.replace("flash_fwd_kernel<", "flash_fwd_split_kernel<")
-    return name
+    Without num_cus: the kernel by tile size alone. With num_cus (the device's
+    compute units): the kernel of vx_flash_attn_ws_fwd given its workspace, as
+    flash_attention calls it (vx_flash_attn_device_plan): also
+    flash_fwd_split_kernel<...> for the grids whose last round the key split
+    evens out, flash_pair_kernel<...> and flash_pair_split_kernel<...> for
+    those of at most one 128-query workgroup per compute unit."""
+    return _lib.flash_plan(int(batch), int(seq_q), int(seq_k), int(num_heads), int(head_dim), int(mask_kind),
+                           None if num_cus is None else int(num_cus))
 
 
 def _single_device(mesh) -> None:

@@ -89,7 +89,6 @@ constexpr int kMaskSlot = 320;
 // Mask kinds (template argument, bits): validity bytes per key, additive bias
 // per key, additive bias per (query, key) of each head (read per query row
 // straight from global memory: meant for the short sequences that use it).
-constexpr int kMaskNone = 0, kMaskValid = 1, kMaskBias = 2, kMaskFull = 4;
 constexpr float kRescaleSlack = 8.0f;         // log2 units
 constexpr float kSumLimit = 256.0f;           // 2^kRescaleSlack
 static_assert(kSumLimit == (float)(1 << (int)kRescaleSlack), "the tile-sum limit is 2^slack");
@@ -1444,44 +1443,21 @@ const char* flash_pair_split_kernel_name() {
   return name.c_str();
 }
 
-// Key tiles from which a grid of at most one workgroup per CU runs pairs: a
-// pair's second start and its merge cost 1.5-2 us (64 KiB through LDS), and it
-// takes two tiles in the time of 1.5 (with the full bias at head dim 128,
-// whose loads bound it, less). Same box, B=1 H=12, one group -> pair: head dim
-// 128 8 tiles 13.2 -> 13.5 us, 10 15.5 -> 14.9, 16 21.8 -> 20.8, key validity
-// 10 tiles 21.0 -> 19.4, full bias 12 34.3 -> 34.8, 16 44.2 -> 43.5; head dim
-// 64 4 tiles 6.6 -> 7.2, 6 8.1 -> 8.0, 8 9.6 -> 9.2, 16 16.7 -> 13.3, full
-// bias 8 17.5 -> 16.0. 25 tiles at head dim 128 (two key halves on two
-// workgroups before) 33.7 -> 28.7.
-template <int MASK, int D>
-constexpr int kPairMinTiles = D == 64 ? 6 : (MASK & kMaskFull) ? 16 : 10;
-// The rare mask pairs with a key bias keep one group.
-template <int MASK>
-constexpr bool kPairMask = MASK != (kMaskValid | kMaskBias) && !((MASK & kMaskFull) && (MASK & kMaskBias));
-// Key tiles from which such a grid, where it fills at most half the CUs, runs
-// the key halves of its items as two pairs: the partials and the merging
-// launch cost ~10 us (one pair -> two: head dim 64 16 tiles 13.3 -> 15.9 us,
-// head dim 128 16 21.3 -> 22.2, 25 27.3 -> 25.3).
-constexpr int kPairSplitMinTiles = 24;
-
 template <int MASK, int WAVES, int D>
 int launch_one(const FlashArgs& a, hipStream_t stream, const char** launched) {
   const int n_qt = (a.Sq + WAVES * 32 - 1) / (WAVES * 32);
-  if constexpr (WAVES == 4 && kPairMask<MASK>) {
-    const int64_t n = (int64_t)n_qt * a.H * a.B, cus = device_cu_count();
-    const int tiles = (a.Sk + kBN - 1) / kBN;
-    if (n <= cus && tiles >= kPairMinTiles<MASK, D>) {
-      if constexpr (!(MASK & (kMaskFull | kMaskBias))) {
-        if (a.split_items == n && 2 * n <= cus && tiles >= kPairSplitMinTiles) {
-          hipLaunchKernelGGL((flash_pair_split_kernel<MASK, D>), dim3((unsigned)(2 * n)), dim3(512), 0, stream, a,
-                             n_qt);
-          hipLaunchKernelGGL((flash_combine_kernel<D, WAVES>), dim3((unsigned)n), dim3(WAVES * 64), 0, stream, a, 0,
-                             n_qt);
+  if constexpr (WAVES == 4 && flash_pair_min_tiles(MASK, D) > 0) {
+    if (a.pair) {
+      const unsigned n = (unsigned)n_qt * a.H * a.B;
+      if constexpr (!(MASK & (kMaskFull | kMaskBias))) {  // bias paths are not split
+        if (a.split_items > 0) {
+          hipLaunchKernelGGL((flash_pair_split_kernel<MASK, D>), dim3(2 * n), dim3(512), 0, stream, a, n_qt);
+          hipLaunchKernelGGL((flash_combine_kernel<D, WAVES>), dim3(n), dim3(WAVES * 64), 0, stream, a, 0, n_qt);
           *launched = flash_pair_split_kernel_name<MASK, D>();
           return (int)hipGetLastError();
         }
       }
-      hipLaunchKernelGGL((flash_pair_kernel<MASK, D>), dim3((unsigned)n), dim3(512), 0, stream, a, n_qt);
+      hipLaunchKernelGGL((flash_pair_kernel<MASK, D>), dim3(n), dim3(512), 0, stream, a, n_qt);
       *launched = flash_pair_kernel_name<MASK, D>();
       return (int)hipGetLastError();
     }

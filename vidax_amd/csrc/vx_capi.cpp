@@ -190,22 +190,39 @@ void flash_kernel_label(int32_t mask_kind, int32_t D, int32_t waves, int32_t str
 // runs ceil(n_items / slots) rounds; when the last round holds r <= slots/2
 // items, running each of those as two workgroups over half the keys (and
 // merging the halves) makes that round take half as long. Key sequences
-// shorter than kMinSplitTiles key tiles are not split.
+// shorter than kMinSplitTiles key tiles are not split, nor are calls with a
+// key or full bias.
+//
+// 4-wave grids of at most one workgroup per compute unit run pairs instead
+// (flash_pair_min_tiles, kPairSplitMinTiles), split only where the pairs of
+// both key halves still find a compute unit each.
 constexpr int32_t kMinSplitTiles = 16;
 
 struct SplitPlan {
   int32_t items = 0;  // items split in two (0: none)
   int32_t k_mid = 0;  // first key of the second half (a multiple of the key tile)
   int64_t ws_bytes = 0;
+  int32_t pair = 0;   // the items run as pairs
 };
 
 SplitPlan flash_split_plan(int32_t B, int32_t Sq, int32_t Sk, int32_t H, int32_t D, int32_t waves,
-                           int32_t num_cus) {
+                           int32_t mask_kind, int32_t num_cus) {
   SplitPlan p;
   const int64_t tiles = ((int64_t)Sk + kKeyTile - 1) / kKeyTile;
-  if (num_cus <= 0 || tiles < kMinSplitTiles) return p;
+  if (num_cus <= 0) return p;
   const int64_t n_qt = ((int64_t)Sq + waves * 32 - 1) / (waves * 32);
   const int64_t n_items = n_qt * H * B;
+  const bool bias = (mask_kind & (vx::kMaskBias | vx::kMaskFull)) != 0;
+  const int32_t pair_tiles = vx::flash_pair_min_tiles(mask_kind, D);
+  if (waves == 4 && pair_tiles > 0 && n_items <= num_cus && tiles >= pair_tiles) {
+    p.pair = 1;
+    if (bias || 2 * n_items > num_cus || tiles < vx::kPairSplitMinTiles) return p;
+    p.items = (int32_t)n_items;
+    p.k_mid = (int32_t)(tiles / 2 * kKeyTile);
+    p.ws_bytes = 2 * n_items * vx::flash_part_floats(waves, D) * (int64_t)sizeof(float);
+    return p;
+  }
+  if (bias || tiles < kMinSplitTiles) return p;
   const int64_t slots = (int64_t)num_cus * (waves == 4 ? 2 : 1);
   const int64_t rounds = (n_items + slots - 1) / slots;
   const int64_t r = n_items - (rounds - 1) * slots;
@@ -325,6 +342,7 @@ int32_t flash_check(const void* q, const void* k, const void* v, const void* out
     args->split_items = 0;
     args->k_mid = 0;
     args->ws = nullptr;
+    args->pair = 0;
     args->q = q;
     args->k = k;
     args->v = v;
@@ -544,6 +562,16 @@ int32_t prologue_check(const void* x, const void* out, const float* weight, floa
   return ok();
 }
 
+// The split plan of checked arguments on the current device (the persistent
+// short-key kernel is not split).
+SplitPlan device_plan(const vx::FlashArgs& a) {
+  if (a.stream) return SplitPlan{};
+  const int32_t mask_kind = (a.key_valid != nullptr ? vx::kMaskValid : 0) |
+                            (a.key_bias != nullptr ? vx::kMaskBias : 0) |
+                            (a.full_bias != nullptr ? vx::kMaskFull : 0);
+  return flash_split_plan(a.B, a.Sq, a.Sk, a.H, a.D, a.waves, mask_kind, vx::device_cu_count());
+}
+
 int32_t injected() {
   const int32_t code = g_inject.load(std::memory_order_relaxed);
   if (code != 0) return fail(code, "error injected by vx_debug_inject_error(%d)", code);
@@ -554,7 +582,7 @@ int32_t injected() {
 
 extern "C" {
 
-int32_t vx_abi_version(void) { return 10800; }
+int32_t vx_abi_version(void) { return 10900; }
 
 const char* vx_last_error(void) { return g_error; }
 
@@ -664,7 +692,7 @@ int32_t vx_flash_attn_split_plan(int32_t batch, int32_t seq_q, int32_t seq_k, in
   const int32_t rc = flash_plan(batch, seq_q, seq_k, num_heads, 0, &waves, &stream);
   if (rc != VX_OK) return rc;
   const SplitPlan p =
-      stream ? SplitPlan{} : flash_split_plan(batch, seq_q, seq_k, num_heads, head_dim, waves, num_cus);
+      stream ? SplitPlan{} : flash_split_plan(batch, seq_q, seq_k, num_heads, head_dim, waves, 0, num_cus);
   if (split_items != nullptr) *split_items = p.items;
   if (split_key != nullptr) *split_key = p.k_mid;
   if (workspace_bytes != nullptr) *workspace_bytes = p.ws_bytes;
@@ -694,11 +722,8 @@ int32_t vx_flash_attn_ws_fwd(const void* q, const void* k, const void* v, void* 
   if (workspace != nullptr && !aligned16(workspace))
     return fail(VX_ERR_INVALID_ARGUMENT, "workspace must be 16-byte aligned");
   if ((rc = injected()) != VX_OK) return rc;
-  // (calls with a key bias, and the persistent short-key kernel, are not split)
-  const SplitPlan p = key_bias != nullptr || args.stream
-                          ? SplitPlan{}
-                          : flash_split_plan(batch, seq_q, seq_k, num_heads, head_dim, args.waves,
-                                             vx::device_cu_count());
+  const SplitPlan p = device_plan(args);
+  args.pair = p.pair;
   if (p.items > 0 && workspace != nullptr && workspace_bytes >= p.ws_bytes) {
     args.split_items = p.items;
     args.k_mid = p.k_mid;
@@ -722,6 +747,22 @@ int32_t vx_flash_attn_plan(int32_t batch, int32_t seq_q, int32_t seq_k, int32_t 
   const int32_t rc = flash_plan(batch, seq_q, seq_k, num_heads, mask_kind, &waves, &stream);
   if (rc != VX_OK) return rc;
   flash_kernel_label(mask_kind, head_dim, waves, stream, kernel_name, name_len);
+  return ok();
+}
+
+int32_t vx_flash_attn_device_plan(int32_t batch, int32_t seq_q, int32_t seq_k, int32_t num_heads, int32_t head_dim,
+                                  int32_t mask_kind, int32_t num_cus, char* kernel_name, int32_t name_len) {
+  int32_t rc = vx_flash_attn_plan(batch, seq_q, seq_k, num_heads, head_dim, mask_kind, kernel_name, name_len);
+  if (rc != VX_OK) return rc;
+  int32_t waves = 0, stream = 0;
+  if ((rc = flash_plan(batch, seq_q, seq_k, num_heads, mask_kind, &waves, &stream)) != VX_OK) return rc;
+  if (stream || kernel_name == nullptr || name_len <= 0) return ok();
+  const SplitPlan p = flash_split_plan(batch, seq_q, seq_k, num_heads, head_dim, waves, mask_kind, num_cus);
+  if (p.pair)
+    snprintf(kernel_name, (size_t)name_len, "flash_pair_%skernel<%d, %d>", p.items > 0 ? "split_" : "", mask_kind,
+             head_dim);
+  else if (p.items > 0)
+    snprintf(kernel_name, (size_t)name_len, "flash_fwd_split_kernel<%d, %d, %d>", mask_kind, head_dim, waves);
   return ok();
 }
 
@@ -762,6 +803,7 @@ int32_t vx_flash_attn_fwd(const void* q, const void* k, const void* v, void* out
                            num_heads, head_dim, q_strides, k_strides, v_strides, out_strides, scale, &args);
   if (rc != VX_OK) return rc;
   if ((rc = injected()) != VX_OK) return rc;
+  args.pair = device_plan(args).pair;
   const char* launched = "";
   const int err = vx::launch_flash_fwd(args, stream, &launched);
   if (err != 0) return fail(VX_ERR_LAUNCH, "flash attention launch failed (hipError_t %d)", err);
@@ -779,10 +821,8 @@ int32_t vx_flash_attn_noalloc_fwd(const void* q, const void* k, const void* v, v
                            num_heads, head_dim, q_strides, k_strides, v_strides, out_strides, scale, &args);
   if (rc != VX_OK) return rc;
   if ((rc = injected()) != VX_OK) return rc;
-  const SplitPlan p = key_bias != nullptr || args.stream
-                          ? SplitPlan{}
-                          : flash_split_plan(batch, seq_q, seq_k, num_heads, head_dim, args.waves,
-                                             vx::device_cu_count());
+  const SplitPlan p = device_plan(args);
+  args.pair = p.pair;
   if (p.items > 0) {
     void* ws = nullptr;
     int64_t cap = 0;
@@ -828,6 +868,7 @@ int32_t vx_flash_attn_bias_fwd(const void* q, const void* k, const void* v, void
                            bias_strides);
   if (rc != VX_OK) return rc;
   if ((rc = injected()) != VX_OK) return rc;
+  args.pair = device_plan(args).pair;
   const char* launched = "";
   const int err = vx::launch_flash_fwd(args, stream, &launched);
   if (err != 0) return fail(VX_ERR_LAUNCH, "flash attention launch failed (hipError_t %d)", err);
