@@ -915,3 +915,43 @@ def test_flash_pairs(gpu, B, Sq, Sk, H, D, mask, kind):
         assert (out[0] == 0).all()
         out, ref = out[1:], ref[1:]
     _check(out, ref, "oracle")
+
+
+@pytest.mark.parametrize("D,Sk,short,mask", [
+    (128, 640, 5, None),          # 10 key tiles: pairs; items of 5 and fewer
+    (128, 1024, 9, None),         # one tile below the rule
+    (64, 384, 5, None),
+    (128, 704, 3, "key_valid"),
+    (64, 448, 4, "key_bias"),
+    (64, 512, 5, "full_bias"),
+])
+def test_flash_pairs_of_short_items(gpu, D, Sk, short, mask):
+    """Where kv_len ends an item's keys below the pairs' key tiles, one group
+    of waves takes them all: bit for bit the call on `short` key tiles, which
+    runs flash_fwd_kernel. A long item of the same call still runs two."""
+    from vidax_amd import _lib, flash_attention
+    _say(f"flash pairs of short items D={D} Sk={Sk} {short} tiles {mask}")
+    B, Sq, H, n = 3, 150, 2, 64 * short
+    q, k, v, _ = O.make_flash_inputs(B, Sq, Sk, H, D, 210)
+    q, k, v = _t(q, gpu), _t(k, gpu), _t(v, gpu)
+    kv = torch.tensor([n - 7, 0 if mask is None else n - 64, Sk], dtype=torch.int32, device=gpu)
+    g = torch.Generator(device=gpu).manual_seed(211)
+    kw = {}
+    if mask == "key_valid":
+        kw["key_valid"] = torch.rand((B, Sk), generator=g, device=gpu) < 0.7
+    elif mask == "key_bias":
+        kw["key_bias"] = torch.randn((B, Sk), generator=g, device=gpu)
+    elif mask == "full_bias":
+        kw["bias"] = torch.randn((1, H, Sq, Sk), generator=g, device=gpu)
+    out = flash_attention(q, k, v, kv_len=kv, **kw)
+    assert _lib.last_launch().startswith("flash_pair_kernel<"), _lib.last_launch()
+    cut = {name: x[..., :n].contiguous()[:2 if x.shape[0] == B else 1] for name, x in kw.items()}
+    ref = flash_attention(q[:2], k[:2, :n].contiguous(), v[:2, :n].contiguous(), kv_len=kv[:2], **cut)
+    assert _lib.last_launch().startswith("flash_fwd_kernel<"), _lib.last_launch()
+    torch.cuda.synchronize()
+    assert torch.equal(out[:2], ref)
+    np_kw = {name: x.cpu().numpy() for name, x in kw.items()}
+    if "bias" in np_kw:
+        np_kw["bias"] = np.broadcast_to(np_kw["bias"], (B, H, Sq, Sk))
+    _check(out[2:], O.attention(*(_np(x) for x in (q, k, v)), kv_len=kv.cpu().numpy().clip(min=1), **np_kw)[2:],
+           "long item vs oracle")

@@ -130,9 +130,17 @@ __device__ __forceinline__ void store_out_lines(const f32x16 (&O)[kDB], float in
 // PAIR: a workgroup of two groups of WAVES waves on the same query tile, each
 // with its own LDS rings and half of the key tiles; group 0 issues both
 // groups' copies and takes group 1's accumulators from LDS at the end.
+//
+// smem: kTileSmem bytes of LDS.
+template <int MASK, int D, int WAVES>
+constexpr int kGroupSmem = FCfg<D, WAVES>::kSmemBytes + (MASK != kMaskNone ? FCfg<D, WAVES>::kMaskRing * kMaskSlot : 0);
+// (a pair: both groups' rings, then group 1's reference points and row sums)
+template <int MASK, int D, int WAVES, bool PAIR = false>
+constexpr int kTileSmem = PAIR ? 2 * kGroupSmem<MASK, D, WAVES> + WAVES * 64 * 8 : kGroupSmem<MASK, D, WAVES>;
+
 template <int MASK, int D, int WAVES, bool PAIR = false>
 __device__ __forceinline__ void flash_tile(const FlashArgs& a, const int qtile, const int head, const int b,
-                                           const int k_lo, const int k_hi, const int part) {
+                                           const int k_lo, const int k_hi, const int part, unsigned char* smem) {
   using C = FCfg<D, WAVES>;
   constexpr int kWaves = C::kWaves, kThreads = C::kThreads, kNB = C::kNB;
   constexpr int kTileBytes = C::kTileBytes, kVBuf = C::kVBuf, kKBuf = C::kKBuf;
@@ -142,11 +150,9 @@ __device__ __forceinline__ void flash_tile(const FlashArgs& a, const int qtile, 
   constexpr bool MASKED = MASK != kMaskNone;
   constexpr int kMaskCopies = (MASK & kMaskValid ? 1 : 0) + (MASK & kMaskBias ? 1 : 0);
   constexpr bool kFull = (MASK & kMaskFull) != 0;
-  constexpr int kGroupBytes = kSmemBytes + (MASKED ? kMaskRing * kMaskSlot : 0);
+  constexpr int kGroupBytes = kGroupSmem<MASK, D, WAVES>;
   static_assert(kGroupBytes % 256 == 0, "the second group's rings start on a bank boundary");
   static_assert(!PAIR || kSmemBytes >= WAVES * 64 * kDB * 64, "group 1's accumulators fit its rings");
-  // (a pair: both groups' rings, then group 1's reference points and row sums)
-  __shared__ __attribute__((aligned(16))) unsigned char smem[PAIR ? 2 * kGroupBytes + kThreads * 8 : kGroupBytes];
 
   const int lane = threadIdx.x & 63;
   const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
@@ -742,7 +748,8 @@ __device__ __forceinline__ void flash_tile(const FlashArgs& a, const int qtile, 
 template <int MASK, int D, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void flash_fwd_kernel(const FlashArgs a) {
-  flash_tile<MASK, D, WAVES>(a, blockIdx.x, blockIdx.y, blockIdx.z, 0, a.Sk, -1);
+  __shared__ __attribute__((aligned(16))) unsigned char smem[kTileSmem<MASK, D, WAVES>];
+  flash_tile<MASK, D, WAVES>(a, blockIdx.x, blockIdx.y, blockIdx.z, 0, a.Sk, -1, smem);
 }
 
 // Key-split launch: items (query tile fastest, then head, then batch item)
@@ -751,6 +758,7 @@ void flash_fwd_kernel(const FlashArgs a) {
 template <int MASK, int D, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void flash_fwd_split_kernel(const FlashArgs a, int n_full, int n_qt) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem[kTileSmem<MASK, D, WAVES>];
   const int w = blockIdx.x;
   int item = w, k_lo = 0, k_hi = a.Sk, part = -1;
   if (w >= n_full) {
@@ -762,18 +770,38 @@ void flash_fwd_split_kernel(const FlashArgs a, int n_full, int n_qt) {
       k_hi = a.k_mid;
   }
   const int qt = item % n_qt, bh = item / n_qt;
-  flash_tile<MASK, D, WAVES>(a, qt, bh % a.H, bh / a.H, k_lo, k_hi, part);
+  flash_tile<MASK, D, WAVES>(a, qt, bh % a.H, bh / a.H, k_lo, k_hi, part, smem);
 }
 
 // Two groups of four waves per 128-query tile (flash_tile's PAIR), for grids
 // that leave a CU to each workgroup: the same two waves per SIMD that two
 // workgroups per CU give larger grids, with half the key tiles each, merged in
-// LDS. One workgroup per item.
+// LDS.
+//
+// An item whose keys end (kv_len) below a.pair tiles runs one group of four
+// waves, as flash_fwd_kernel does: the second group's start and the merge cost
+// more than they give there (same box, 640 keys, 12 heads x 512 queries, head
+// dim 128: kv_len 64 6.5 us as one group, 8.1 as two; 300 10.8 and 12.3; head
+// dim 64: 4.8 and 5.8, 7.9 and 8.7). The other group's waves end at once.
+template <int MASK, int D>
+__device__ __forceinline__ void flash_pair_tile(const FlashArgs& a, const int qtile, const int head, const int b,
+                                                const int k_lo, const int k_hi, const int part) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem[kTileSmem<MASK, D, 4, true>];
+  int kv_end = k_hi;
+  if (a.kv_len != nullptr) kv_end = min(max(a.kv_len[b], 0), k_hi);
+  const int tiles = __builtin_amdgcn_readfirstlane((kv_end + kBN - 1) / kBN - k_lo / kBN);
+  if (tiles >= a.pair)
+    flash_tile<MASK, D, 4, true>(a, qtile, head, b, k_lo, k_hi, part, smem);
+  else if (threadIdx.x < 256)
+    flash_tile<MASK, D, 4>(a, qtile, head, b, k_lo, k_hi, part, smem);
+}
+
+// One pair per item.
 template <int MASK, int D>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void flash_pair_kernel(const FlashArgs a, int n_qt) {
   const int item = blockIdx.x, qt = item % n_qt, bh = item / n_qt;
-  flash_tile<MASK, D, 4, true>(a, qt, bh % a.H, bh / a.H, 0, a.Sk, -1);
+  flash_pair_tile<MASK, D>(a, qt, bh % a.H, bh / a.H, 0, a.Sk, -1);
 }
 
 // One pair per half of an item's keys (every item split), writing partials.
@@ -782,7 +810,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void flash_pair_split_kernel(const FlashArgs a, int n_qt) {
   const int part = blockIdx.x, item = part >> 1, qt = item % n_qt, bh = item / n_qt;
   const int k_lo = part & 1 ? a.k_mid : 0, k_hi = part & 1 ? a.Sk : a.k_mid;
-  flash_tile<MASK, D, 4, true>(a, qt, bh % a.H, bh / a.H, k_lo, k_hi, part);
+  flash_pair_tile<MASK, D>(a, qt, bh % a.H, bh / a.H, k_lo, k_hi, part);
 }
 
 // Merges the two key halves of each split item: with M the larger reference

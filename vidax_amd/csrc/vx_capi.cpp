@@ -202,7 +202,7 @@ struct SplitPlan {
   int32_t items = 0;  // items split in two (0: none)
   int32_t k_mid = 0;  // first key of the second half (a multiple of the key tile)
   int64_t ws_bytes = 0;
-  int32_t pair = 0;   // the items run as pairs
+  int32_t pair = 0;   // the items run as pairs, from this many key tiles
 };
 
 SplitPlan flash_split_plan(int32_t B, int32_t Sq, int32_t Sk, int32_t H, int32_t D, int32_t waves,
@@ -215,7 +215,7 @@ SplitPlan flash_split_plan(int32_t B, int32_t Sq, int32_t Sk, int32_t H, int32_t
   const bool bias = (mask_kind & (vx::kMaskBias | vx::kMaskFull)) != 0;
   const int32_t pair_tiles = vx::flash_pair_min_tiles(mask_kind, D);
   if (waves == 4 && pair_tiles > 0 && n_items <= num_cus && tiles >= pair_tiles) {
-    p.pair = 1;
+    p.pair = pair_tiles;
     if (bias || 2 * n_items > num_cus || tiles < vx::kPairSplitMinTiles) return p;
     p.items = (int32_t)n_items;
     p.k_mid = (int32_t)(tiles / 2 * kKeyTile);

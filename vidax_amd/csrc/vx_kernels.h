@@ -34,8 +34,9 @@ struct FlashArgs {
   int32_t split_items;
   int32_t k_mid;
   float* ws;
-  // 1: two groups of four waves per 128-query tile (waves 4, grids of at most
-  // one such tile per compute unit); with split_items > 0 (every item split)
+  // > 0: two groups of four waves per 128-query tile (waves 4, grids of at
+  // most one such tile per compute unit) for items of at least `pair` key
+  // tiles, one group for shorter ones; with split_items > 0 (every item split)
   // one such pair per half of an item's keys
   int32_t pair;
 };
