@@ -567,31 +567,66 @@ def test_flash_kernel_name_with_the_key_split():
 
 
 def test_pairs_in_the_plan():
-    """4-wave grids of at most one workgroup per compute unit run pairs, and
-    only those that split (both halves' pairs on a unit each, 24 key tiles and
-    more, no bias) ask for a workspace. 2 heads x 52 query tiles = 104 items."""
+    """Most 4-wave grids of at most one workgroup per compute unit run pairs,
+    and only those that split ask for a workspace. 256 compute units, heads of
+    512 queries: H items / 4 each, by key tiles."""
     from vidax_amd.attention import flash_kernel_name
-    part = 4 * 64 * (4 * 16 + 2) * 4
-    assert _split((1, 6650, 23 * 64, 2, 128)) == (0, 0, 0)
-    assert _split((1, 6650, 24 * 64, 2, 128)) == (104, 12 * 64, 2 * 104 * part)
-    assert _split((1, 16384, 1600, 1, 128)) == (128, 12 * 64, 2 * 128 * part)   # n = CUs / 2
-    assert _split((1, 16385, 1600, 1, 128)) == (0, 0, 0)                        # n = CUs / 2 + 1
-    assert _split((1, 1560, 1560, 12, 128)) == (0, 0, 0)                        # 156 items: one pair each
-    assert _split((1, 32768, 1600, 1, 128)) == (0, 0, 0)                        # n = CUs
-    assert _split((1, 32769, 1600, 1, 128)) == (0, 0, 0)                        # n = CUs + 1: a round above half full
-    assert _split((1, 65664, 1600, 1, 128)) == (1, 12 * 64, 2 * part)           # 513 items: one split
+    part = {128: 4 * 64 * (4 * 16 + 2) * 4, 64: 4 * 64 * (2 * 16 + 2) * 4}
 
-    def name(Sq, Sk, H, D=128, mask=0, cus=256):
-        return flash_kernel_name(1, Sq, Sk, H, D, mask, num_cus=cus)
-    assert name(6650, 24 * 64, 2) == "flash_pair_split_kernel<0, 128>"
-    assert name(6650, 23 * 64, 2) == "flash_pair_kernel<0, 128>"
-    assert name(6650, 24 * 64, 2, mask=2) == "flash_pair_kernel<2, 128>"
-    assert name(6650, 24 * 64, 2, mask=3) == "flash_fwd_kernel<3, 128, 4>"
-    assert name(6650, 24 * 64, 2, mask=6) == "flash_fwd_kernel<6, 128, 4>"
-    assert name(6650, 24 * 64, 2, cus=104) == "flash_pair_kernel<0, 128>"
-    assert name(6650, 24 * 64, 2, cus=103) == "flash_fwd_kernel<0, 128, 4>"   # 104 of 206 slots
-    assert name(32769, 1600, 1) == "flash_fwd_kernel<0, 128, 4>"
-    assert name(200, 64 * 10, 4) == "flash_pair_kernel<0, 128>" and name(200, 64 * 9, 4) == "flash_fwd_kernel<0, 128, 4>"
-    assert name(200, 64 * 6, 4, 64) == "flash_pair_kernel<0, 64>" and name(200, 64 * 5, 4, 64) == "flash_fwd_kernel<0, 64, 4>"
-    assert name(200, 64 * 16, 4, mask=4) == "flash_pair_kernel<4, 128>"
-    assert name(200, 64 * 15, 4, mask=4) == "flash_fwd_kernel<4, 128, 4>"
+    def kind(items, tiles, D=128, mask=0, cus=256):
+        """1 one group, 2 pair, "s" split pair, "k" 4-wave key split"""
+        assert items % 4 == 0
+        shape = (1, 512, 64 * tiles, items // 4, D)
+        name = flash_kernel_name(*shape, mask, num_cus=cus)
+        got = {f"flash_fwd_kernel<{mask}, {D}, 4>": 1, f"flash_pair_kernel<{mask}, {D}>": 2,
+               f"flash_pair_split_kernel<{mask}, {D}>": "s", f"flash_fwd_split_kernel<{mask}, {D}, 4>": "k"}[name]
+        if mask == 0:
+            want = (items, tiles // 2 * 64, 2 * items * part[D]) if got in ("s", "k") else (0, 0, 0)
+            assert _split(shape, cus) == want, (items, tiles, D)
+        return got
+
+    for items, D, mask, kinds in [
+        # head dim 64: from 6 tiles, split from 24 while both halves find a unit
+        (8, 64, 0, {5: 1, 6: 2, 23: 2, 24: "s", 64: "s"}),
+        (128, 64, 0, {5: 1, 6: 2, 23: 2, 24: "s"}),
+        (132, 64, 0, {5: 1, 6: 2, 24: 2, 64: 2}),
+        (256, 64, 2, {5: 1, 6: 2, 64: 2}),
+        # head dim 128
+        (64, 128, 0, {9: 1, 10: 2, 19: 2, 20: "s", 64: "s"}),
+        (68, 128, 0, {9: 1, 10: 2, 25: 2, 26: "s"}),
+        (96, 128, 1, {9: 1, 10: 2, 25: 2, 26: "s"}),
+        (100, 128, 0, {9: 1, 10: 2, 31: 2, 32: "k"}),
+        (128, 128, 0, {9: 1, 10: 2, 31: 2, 32: "k"}),
+        (132, 128, 0, {13: 1, 14: 2, 64: 2}),
+        (160, 128, 1, {13: 1, 14: 2, 64: 2}),
+        (164, 128, 0, {16: 1, 19: 1, 20: 2, 64: 2}),
+        (224, 128, 0, {16: 1, 19: 1, 20: 2, 64: 2}),
+        (228, 128, 0, {15: 1, 16: 1, 64: 1}),    # 4 query tiles a head
+        (256, 128, 0, {15: 1, 16: 1, 64: 1}),
+        # biases: never split
+        (64, 128, 2, {9: 1, 10: 2, 64: 2}),
+        (128, 128, 2, {9: 1, 10: 2, 64: 2}),
+        (224, 128, 2, {19: 1, 20: 2, 64: 2}),
+        (228, 128, 2, {64: 1}),
+        (64, 128, 4, {15: 1, 16: 2, 64: 2}),
+        (160, 128, 5, {15: 1, 16: 2, 64: 2}),
+        (192, 128, 5, {19: 1, 20: 2, 64: 2}),
+        (196, 128, 4, {24: 1, 64: 1}),
+        (228, 128, 4, {64: 1}),
+        (64, 128, 3, {64: 1}),
+        (64, 128, 6, {64: 1}),
+        (64, 64, 7, {64: 1}),
+    ]:
+        for tiles, want in kinds.items():
+            assert kind(items, tiles, D, mask) == want, (items, D, mask, tiles, want)
+    # up to 256 items, of 7, 8 and 32 query tiles a head
+    for Sq, H, Sk, want in [(896, 13, 1536, "pair_kernel<0, 128>"), (1024, 12, 1408, "pair_split_kernel<0, 128>"),
+                            (1024, 12, 1344, "pair_kernel<0, 128>"), (896, 18, 2048, "fwd_split_kernel<0, 128, 4>"),
+                            (4096, 4, 2048, "pair_split_kernel<0, 128>"), (4096, 4, 1984, "pair_kernel<0, 128>"),
+                            (896, 36, 4000, "fwd_kernel<0, 128, 4>"), (1024, 32, 1536, "pair_kernel<0, 128>"),
+                            (1024, 32, 1472, "fwd_kernel<0, 128, 4>"), (4000, 8, 4000, "pair_kernel<0, 128>")]:
+        assert flash_kernel_name(1, Sq, Sk, H, num_cus=256) == "flash_" + want, (Sq, H, Sk)
+    assert kind(260, 24) == 1                                            # above half of the 512 slots
+    assert _split((1, 65664, 1600, 1, 128)) == (1, 12 * 64, 2 * part[128])   # 513 items: one split
+    assert kind(104, 24, cus=104) == 1 and kind(104, 24, cus=120) == 2   # on fewer units
+    assert _split((1, 1560, 1560, 12, 128)) == (0, 0, 0)                 # 156 items, a pair each: no workspace

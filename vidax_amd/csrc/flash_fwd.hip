@@ -1474,7 +1474,7 @@ const char* flash_pair_split_kernel_name() {
 template <int MASK, int WAVES, int D>
 int launch_one(const FlashArgs& a, hipStream_t stream, const char** launched) {
   const int n_qt = (a.Sq + WAVES * 32 - 1) / (WAVES * 32);
-  if constexpr (WAVES == 4 && flash_pair_min_tiles(MASK, D) > 0) {
+  if constexpr (WAVES == 4 && flash_pair_mask(MASK)) {
     if (a.pair) {
       const unsigned n = (unsigned)n_qt * a.H * a.B;
       if constexpr (!(MASK & (kMaskFull | kMaskBias))) {  // bias paths are not split

@@ -193,9 +193,8 @@ void flash_kernel_label(int32_t mask_kind, int32_t D, int32_t waves, int32_t str
 // shorter than kMinSplitTiles key tiles are not split, nor are calls with a
 // key or full bias.
 //
-// 4-wave grids of at most one workgroup per compute unit run pairs instead
-// (flash_pair_min_tiles, kPairSplitMinTiles), split only where the pairs of
-// both key halves still find a compute unit each.
+// Most 4-wave grids of at most one workgroup per compute unit run pairs
+// instead (flash_pair_min_tiles, flash_pair_split_min_tiles).
 constexpr int32_t kMinSplitTiles = 16;
 
 struct SplitPlan {
@@ -205,24 +204,81 @@ struct SplitPlan {
   int32_t pair = 0;   // the items run as pairs, from this many key tiles
 };
 
+// Key tiles from which a grid of n_items 128-query workgroups (n_qt per head),
+// at most one per compute unit, runs pairs (0: never). A pair's second start
+// and its merge cost 1.5-2 us (64 KiB through LDS), and it reads K and V twice
+// as fast: at head dim 128 on most of the chip that only pays over more tiles,
+// and where enough query tiles share a head's K and V. Same box, pair against
+// one group per item (key bias, or no mask without a workspace):
+//   head dim 64: 4 tiles 1.02, 6 0.95, 10 0.87, 16 0.80; 256 items 0.95-1.01
+//   head dim 128, up to CUs / 2 items: 8 tiles 0.95-1.03, 10 0.89-0.97, 14
+//     0.85-0.95, 24 0.79-0.89; full bias 12 0.92-0.98, 16 0.92-0.95
+//   160 items: 11 tiles 1.04, 13 1.00, 14 0.93-0.96, 24 0.85-0.91
+//   224 items: 16 tiles 0.99-1.05, 20 0.95-1.02, 32 0.89-1.02; full bias 16
+//     1.03, 24 0.96-1.13
+//   256 items: 12 tiles 1.09, 16 1.05; 24 tiles and more 0.82-0.95 with 12 to
+//     40 query tiles a head, 1.03-1.04 with 4
+int32_t flash_pair_min_tiles(int64_t n_items, int64_t n_qt, int32_t mask_kind, int32_t D, int32_t num_cus) {
+  if (!vx::flash_pair_mask(mask_kind)) return 0;
+  if (D == 64) return 6;
+  const bool full = (mask_kind & vx::kMaskFull) != 0;
+  const int64_t n = 8 * n_items, cus = num_cus;
+  if (n <= 4 * cus) return full ? 16 : 10;
+  if (n <= 5 * cus) return full ? 16 : 14;
+  if (n <= 7 * cus) return full && n > 6 * cus ? 0 : 20;
+  return !full && n_qt >= 8 ? 24 : 0;
+}
+
+// Key tiles from which each item of such a grid, at most half the compute
+// units, runs the two halves of its keys as a pair each (0: never): the
+// partials and the merging launch cost ~10 us, and the pairs then read K and V
+// on twice the units. Same box, one pair / two pairs against two one-group
+// workgroups per item (the key split below):
+//   head dim 64: 16 tiles 0.80-0.92 / 0.94-0.99, 24 0.84-0.96 / 0.88-0.95
+//   head dim 128, 64 items: 18 tiles 1.00 / 1.02, 20 1.02 / 0.99, 24 1.06 / 0.98
+//   96 items, 4 query tiles a head: 24 tiles 1.01 / 1.02, 28 1.06 / 1.01, 40
+//     1.12 / 1.00; 12 and more a head: 24 1.01 / 0.93, 32 1.01 / 0.94
+//   128 items, 4 a head: 24 tiles 0.94 / 1.06, 32 0.98 / 1.06, 40 1.02 / 1.09;
+//     16 and more a head: 20 0.92 / 0.97, 32 0.96 / 0.98, 64 1.02 / 0.93
+int32_t flash_pair_split_min_tiles(int64_t n_items, int64_t n_qt, int32_t D, int32_t num_cus) {
+  if (D == 64) return 24;
+  if (4 * n_items <= num_cus) return 20;
+  if (8 * n_items <= 3 * (int64_t)num_cus) return n_qt >= 8 ? 22 : 26;
+  return n_qt >= 8 ? 32 : 0;
+}
+// Where that is never, one pair per item falls behind the key split from this
+// many tiles on (above).
+constexpr int32_t kPairMaxTiles = 32;
+
+// can_split: a workspace for the partials is there (calls with a key or full
+// bias are not split in any case).
 SplitPlan flash_split_plan(int32_t B, int32_t Sq, int32_t Sk, int32_t H, int32_t D, int32_t waves,
-                           int32_t mask_kind, int32_t num_cus) {
+                           int32_t mask_kind, int32_t num_cus, bool can_split) {
   SplitPlan p;
   const int64_t tiles = ((int64_t)Sk + kKeyTile - 1) / kKeyTile;
   if (num_cus <= 0) return p;
   const int64_t n_qt = ((int64_t)Sq + waves * 32 - 1) / (waves * 32);
   const int64_t n_items = n_qt * H * B;
-  const bool bias = (mask_kind & (vx::kMaskBias | vx::kMaskFull)) != 0;
-  const int32_t pair_tiles = vx::flash_pair_min_tiles(mask_kind, D);
-  if (waves == 4 && pair_tiles > 0 && n_items <= num_cus && tiles >= pair_tiles) {
-    p.pair = pair_tiles;
-    if (bias || 2 * n_items > num_cus || tiles < vx::kPairSplitMinTiles) return p;
-    p.items = (int32_t)n_items;
-    p.k_mid = (int32_t)(tiles / 2 * kKeyTile);
-    p.ws_bytes = 2 * n_items * vx::flash_part_floats(waves, D) * (int64_t)sizeof(float);
-    return p;
+  if ((mask_kind & (vx::kMaskBias | vx::kMaskFull)) != 0) can_split = false;
+  if (waves == 4 && n_items <= num_cus) {
+    const int32_t min_tiles = flash_pair_min_tiles(n_items, n_qt, mask_kind, D, num_cus);
+    const bool halves = can_split && 2 * n_items <= num_cus;  // both halves' pairs find a unit each
+    const int32_t split_tiles = flash_pair_split_min_tiles(n_items, n_qt, D, num_cus);
+    if (min_tiles == 0 || tiles < min_tiles) {
+      // one group per item on more than half of the units: a key split would
+      // only add its partials (228 to 256 items, head dim 128, 16-24 key
+      // tiles: one group 0.70-0.84 of the split)
+      if (2 * n_items > num_cus) can_split = false;
+    } else if (!(halves && split_tiles == 0 && tiles >= kPairMaxTiles)) {
+      p.pair = min_tiles;
+      if (!halves || split_tiles == 0 || tiles < split_tiles) return p;
+      p.items = (int32_t)n_items;
+      p.k_mid = (int32_t)(tiles / 2 * kKeyTile);
+      p.ws_bytes = 2 * n_items * vx::flash_part_floats(waves, D) * (int64_t)sizeof(float);
+      return p;
+    }
   }
-  if (bias || tiles < kMinSplitTiles) return p;
+  if (!can_split || tiles < kMinSplitTiles) return p;
   const int64_t slots = (int64_t)num_cus * (waves == 4 ? 2 : 1);
   const int64_t rounds = (n_items + slots - 1) / slots;
   const int64_t r = n_items - (rounds - 1) * slots;
@@ -564,12 +620,12 @@ int32_t prologue_check(const void* x, const void* out, const float* weight, floa
 
 // The split plan of checked arguments on the current device (the persistent
 // short-key kernel is not split).
-SplitPlan device_plan(const vx::FlashArgs& a) {
+SplitPlan device_plan(const vx::FlashArgs& a, bool can_split) {
   if (a.stream) return SplitPlan{};
   const int32_t mask_kind = (a.key_valid != nullptr ? vx::kMaskValid : 0) |
                             (a.key_bias != nullptr ? vx::kMaskBias : 0) |
                             (a.full_bias != nullptr ? vx::kMaskFull : 0);
-  return flash_split_plan(a.B, a.Sq, a.Sk, a.H, a.D, a.waves, mask_kind, vx::device_cu_count());
+  return flash_split_plan(a.B, a.Sq, a.Sk, a.H, a.D, a.waves, mask_kind, vx::device_cu_count(), can_split);
 }
 
 int32_t injected() {
@@ -692,7 +748,7 @@ int32_t vx_flash_attn_split_plan(int32_t batch, int32_t seq_q, int32_t seq_k, in
   const int32_t rc = flash_plan(batch, seq_q, seq_k, num_heads, 0, &waves, &stream);
   if (rc != VX_OK) return rc;
   const SplitPlan p =
-      stream ? SplitPlan{} : flash_split_plan(batch, seq_q, seq_k, num_heads, head_dim, waves, 0, num_cus);
+      stream ? SplitPlan{} : flash_split_plan(batch, seq_q, seq_k, num_heads, head_dim, waves, 0, num_cus, true);
   if (split_items != nullptr) *split_items = p.items;
   if (split_key != nullptr) *split_key = p.k_mid;
   if (workspace_bytes != nullptr) *workspace_bytes = p.ws_bytes;
@@ -722,9 +778,10 @@ int32_t vx_flash_attn_ws_fwd(const void* q, const void* k, const void* v, void* 
   if (workspace != nullptr && !aligned16(workspace))
     return fail(VX_ERR_INVALID_ARGUMENT, "workspace must be 16-byte aligned");
   if ((rc = injected()) != VX_OK) return rc;
-  const SplitPlan p = device_plan(args);
+  SplitPlan p = device_plan(args, true);
+  if (p.items > 0 && (workspace == nullptr || workspace_bytes < p.ws_bytes)) p = device_plan(args, false);
   args.pair = p.pair;
-  if (p.items > 0 && workspace != nullptr && workspace_bytes >= p.ws_bytes) {
+  if (p.items > 0) {
     args.split_items = p.items;
     args.k_mid = p.k_mid;
     args.ws = static_cast<float*>(workspace);
@@ -757,7 +814,7 @@ int32_t vx_flash_attn_device_plan(int32_t batch, int32_t seq_q, int32_t seq_k, i
   int32_t waves = 0, stream = 0;
   if ((rc = flash_plan(batch, seq_q, seq_k, num_heads, mask_kind, &waves, &stream)) != VX_OK) return rc;
   if (stream || kernel_name == nullptr || name_len <= 0) return ok();
-  const SplitPlan p = flash_split_plan(batch, seq_q, seq_k, num_heads, head_dim, waves, mask_kind, num_cus);
+  const SplitPlan p = flash_split_plan(batch, seq_q, seq_k, num_heads, head_dim, waves, mask_kind, num_cus, true);
   if (p.pair)
     snprintf(kernel_name, (size_t)name_len, "flash_pair_%skernel<%d, %d>", p.items > 0 ? "split_" : "", mask_kind,
              head_dim);
@@ -803,7 +860,7 @@ int32_t vx_flash_attn_fwd(const void* q, const void* k, const void* v, void* out
                            num_heads, head_dim, q_strides, k_strides, v_strides, out_strides, scale, &args);
   if (rc != VX_OK) return rc;
   if ((rc = injected()) != VX_OK) return rc;
-  args.pair = device_plan(args).pair;
+  args.pair = device_plan(args, false).pair;
   const char* launched = "";
   const int err = vx::launch_flash_fwd(args, stream, &launched);
   if (err != 0) return fail(VX_ERR_LAUNCH, "flash attention launch failed (hipError_t %d)", err);
@@ -821,7 +878,7 @@ int32_t vx_flash_attn_noalloc_fwd(const void* q, const void* k, const void* v, v
                            num_heads, head_dim, q_strides, k_strides, v_strides, out_strides, scale, &args);
   if (rc != VX_OK) return rc;
   if ((rc = injected()) != VX_OK) return rc;
-  const SplitPlan p = device_plan(args);
+  const SplitPlan p = device_plan(args, true);
   args.pair = p.pair;
   if (p.items > 0) {
     void* ws = nullptr;
@@ -868,7 +925,7 @@ int32_t vx_flash_attn_bias_fwd(const void* q, const void* k, const void* v, void
                            bias_strides);
   if (rc != VX_OK) return rc;
   if ((rc = injected()) != VX_OK) return rc;
-  args.pair = device_plan(args).pair;
+  args.pair = device_plan(args, false).pair;
   const char* launched = "";
   const int err = vx::launch_flash_fwd(args, stream, &launched);
   if (err != 0) return fail(VX_ERR_LAUNCH, "flash attention launch failed (hipError_t %d)", err);

@@ -53,25 +53,11 @@ constexpr int kStreamTabMax = 1024;
 // Mask bits of the flash kernels.
 constexpr int32_t kMaskNone = 0, kMaskValid = 1, kMaskBias = 2, kMaskFull = 4;
 
-// Key tiles from which a grid of at most one 128-query workgroup per compute
-// unit runs pairs (0: never, the rare mask pairs with a key bias). A
-// pair's second start and its merge cost 1.5-2 us (64 KiB through LDS), and it
-// takes two tiles in the time of 1.5 (with the full bias at head dim 128,
-// whose loads bound it, less). Same box, B=1 H=12, one group -> pair: head dim
-// 128 8 tiles 13.2 -> 13.5 us, 10 15.5 -> 14.9, 16 21.8 -> 20.8, key validity
-// 10 tiles 21.0 -> 19.4, full bias 12 34.3 -> 34.8, 16 44.2 -> 43.5; head dim
-// 64 4 tiles 6.6 -> 7.2, 6 8.1 -> 8.0, 8 9.6 -> 9.2, 16 16.7 -> 13.3, full
-// bias 8 17.5 -> 16.0. 25 tiles at head dim 128 (two key halves on two
-// workgroups before) 33.7 -> 28.7.
-constexpr int32_t flash_pair_min_tiles(int32_t mask, int32_t head_dim) {
-  if (mask == (kMaskValid | kMaskBias) || ((mask & kMaskFull) && (mask & kMaskBias))) return 0;
-  return head_dim == 64 ? 6 : (mask & kMaskFull) ? 16 : 10;
+// Whether the flash kernels have pairs for a mask: not for the rare mask
+// combinations with a key bias.
+constexpr bool flash_pair_mask(int32_t mask) {
+  return mask != (kMaskValid | kMaskBias) && !((mask & kMaskFull) && (mask & kMaskBias));
 }
-// Key tiles from which such a grid, where it fills at most half the CUs, runs
-// the key halves of its items as two pairs: the partials and the merging
-// launch cost ~10 us (one pair -> two: head dim 64 16 tiles 13.3 -> 15.9 us,
-// head dim 128 16 21.3 -> 22.2, 25 27.3 -> 25.3).
-constexpr int32_t kPairSplitMinTiles = 24;
 
 // fp32 values of one key-split partial: the lanes' O accumulators, then
 // (reference point, row sum) per lane.
