@@ -64,12 +64,6 @@ __device__ __forceinline__ float sum16(const float (&p)[16]) {
   return (q[0] + q[1]) + (q[2] + q[3]);
 }
 
-// The block's q preparation on the resident Q fragments of one lane (query
-// `tok`, d = 16 * ds + 8 * hf + 0..7 in qr[ds]; lane l ^ 32 holds the other
-// half of the row), with the rounding points of the one-pass prologue kernel.
-// The per-head sum of squares adds the 8-element chunk sums in the order of
-// that kernel's xor-butterfly over the head's D/8 chunks (chunk c = 2*ds+hf
-// pairs with c^8, c^4, c^2 inside the lane and with c^1 in the other half).
 // Output rows of a wave's 32 queries, query r being the token (t + r /
 // (QX QY), y0 + r / QX % QY, x0 + r % QX) of the head's output og (tokens
 // tok_stride apart; rows outside the T x Hs x W grid are dropped): the O^T
@@ -96,46 +90,61 @@ __device__ __forceinline__ void store_na_rows(const f32x16 (&O)[kDB], float inv,
   }
 }
 
-template <int NDS>
+// The block's q preparation on the resident Q fragments of one lane (query
+// `tok`, d = 16 * ds + 8 * hf + 0..7 in qr[ds]; lane l ^ 32 holds the other
+// half of the row), with the rounding points of the one-pass prologue kernel.
+// The per-head sum of squares adds the 8-element chunk sums in the order of
+// that kernel's xor-butterfly over the head's D/8 chunks (chunk c = 2*ds+hf
+// pairs with c^8, c^4, c^2 inside the lane and with c^1 in the other half).
+// G: the d blocks (of 16) whose weights and rotations are loaded, and held, at
+// a time: all where the registers allow, so that the loads overlap; four in the
+// t-stacked block form, whose three waves per SIMD have 168 registers (all
+// eight spilled 89 of them; 21x45x80 NH=24 D=128 (3,7,7) with q preparation
+// 1107 -> 806 us, two at a time 820, one 837).
+template <int G, int NDS>
 __device__ __forceinline__ void prep_q(bf16x8 (&qr)[NDS], int hf, int64_t tok, int tq, int yq, int xq,
                                        const Na3dArgs& a) {
+  static_assert(NDS % G == 0, "whole groups of d blocks");
   constexpr int D = NDS * 16;
-  // all loads first (weights, then the token's rotation tables), so their
-  // latencies overlap
-  f32x4 w[NDS][2], cs[NDS], sn[NDS];
+  f32x4 w[G][2], cs[G], sn[G];
   const bool norm = (a.q_prep & kQPrepNorm) != 0, rope = (a.q_prep & kQPrepRope) != 0;
-  if (norm) {
+  // the group's weights, then its part of the token's rotation tables
+  auto load = [&](int d0) __attribute__((always_inline)) {
+    if (norm) {
 #pragma unroll
-    for (int ds = 0; ds < NDS; ++ds) {
-      const float* wp = a.q_weight + ds * 16 + hf * 8;
-      w[ds][0] = *(const f32x4*)wp;
-      w[ds][1] = *(const f32x4*)(wp + 4);
+      for (int i = 0; i < G; ++i) {
+        const float* wp = a.q_weight + (d0 + i) * 16 + hf * 8;
+        w[i][0] = *(const f32x4*)wp;
+        w[i][1] = *(const f32x4*)(wp + 4);
+      }
     }
-  }
-  if (rope && (a.q_prep & kQPrepRopeAxes)) {
-    // per-axis rows (t rows, then h rows, then w rows of one table): the
-    // lane's 4 pairs 8 ds + 4 hf + 0..3 lie in one axis's part (its
-    // boundaries are multiples of 4) and are read at their own columns of
-    // that axis's row; a few hundred rows shared by every token and head
-    // instead of one table row per token. 32-bit element offsets.
-    const int st = (int)a.q_tab_stride;
-    const int row_t = tq * st, row_h = (a.T + yq) * st, row_w = (a.T + a.Hs + xq) * st;
+    if (rope && (a.q_prep & kQPrepRopeAxes)) {
+      // per-axis rows (t rows, then h rows, then w rows of one table): the
+      // lane's 4 pairs 8 ds + 4 hf + 0..3 lie in one axis's part (its
+      // boundaries are multiples of 4) and are read at their own columns of
+      // that axis's row; a few hundred rows shared by every token and head
+      // instead of one table row per token. 32-bit element offsets.
+      const int st = (int)a.q_tab_stride;
+      const int row_t = tq * st, row_h = (a.T + yq) * st, row_w = (a.T + a.Hs + xq) * st;
 #pragma unroll
-    for (int ds = 0; ds < NDS; ++ds) {
-      const int j = ds * 8 + hf * 4;
-      const int off = (j < a.q_ax_pairs[0] ? row_t : (j < a.q_ax_pairs[1] ? row_h : row_w)) + j;
-      cs[ds] = *(const f32x4*)(a.q_cos + off);
-      sn[ds] = *(const f32x4*)(a.q_sin + off);
-    }
-  } else if (rope) {
-    const float* cr = a.q_cos + tok * a.q_tab_stride + hf * 4;
-    const float* sr = a.q_sin + tok * a.q_tab_stride + hf * 4;
+      for (int i = 0; i < G; ++i) {
+        const int j = (d0 + i) * 8 + hf * 4;
+        const int off = (j < a.q_ax_pairs[0] ? row_t : (j < a.q_ax_pairs[1] ? row_h : row_w)) + j;
+        cs[i] = *(const f32x4*)(a.q_cos + off);
+        sn[i] = *(const f32x4*)(a.q_sin + off);
+      }
+    } else if (rope) {
+      const float* cr = a.q_cos + tok * a.q_tab_stride + hf * 4;
+      const float* sr = a.q_sin + tok * a.q_tab_stride + hf * 4;
 #pragma unroll
-    for (int ds = 0; ds < NDS; ++ds) {
-      cs[ds] = *(const f32x4*)(cr + ds * 8);
-      sn[ds] = *(const f32x4*)(sr + ds * 8);
+      for (int i = 0; i < G; ++i) {
+        cs[i] = *(const f32x4*)(cr + (d0 + i) * 8);
+        sn[i] = *(const f32x4*)(sr + (d0 + i) * 8);
+      }
     }
-  }
+  };
+  load(0);
+  float rinv = 0.f;
   if (norm) {
     float ss[NDS];
 #pragma unroll
@@ -145,24 +154,30 @@ __device__ __forceinline__ void prep_q(bf16x8 (&qr)[NDS], int hf, int64_t tok, i
     for (int m = NDS / 2; m >= 1; m >>= 1)
 #pragma unroll
       for (int ds = 0; ds < m; ++ds) ss[ds] = ss[ds] + ss[ds + m];
-    const float rinv = rms_inv(halves_sum(ss[0]), D, a.q_eps);
-#pragma unroll
-    for (int ds = 0; ds < NDS; ++ds)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) qr[ds][e] = rms_elem((float)qr[ds][e], rinv, w[ds][e >> 2][e & 3]);
+    rinv = rms_inv(halves_sum(ss[0]), D, a.q_eps);
   }
-  if (a.q_prep & kQPrepScale) {
-    const float ps = (float)(bf16)a.q_post_scale;
 #pragma unroll
-    for (int ds = 0; ds < NDS; ++ds)
+  for (int d0 = 0; d0 < NDS; d0 += G) {
+    if (d0 > 0) load(d0);
+    if (norm) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) qr[ds][e] = scale_elem((float)qr[ds][e], ps);
-  }
-  if (rope) {
+      for (int i = 0; i < G; ++i)
 #pragma unroll
-    for (int ds = 0; ds < NDS; ++ds)
+        for (int e = 0; e < 8; ++e) qr[d0 + i][e] = rms_elem((float)qr[d0 + i][e], rinv, w[i][e >> 2][e & 3]);
+    }
+    if (a.q_prep & kQPrepScale) {
+      const float ps = (float)(bf16)a.q_post_scale;
 #pragma unroll
-      for (int p = 0; p < 4; ++p) rope_pair(qr[ds], p, cs[ds][p], sn[ds][p]);
+      for (int i = 0; i < G; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) qr[d0 + i][e] = scale_elem((float)qr[d0 + i][e], ps);
+    }
+    if (rope) {
+#pragma unroll
+      for (int i = 0; i < G; ++i)
+#pragma unroll
+        for (int p = 0; p < 4; ++p) rope_pair(qr[d0 + i], p, cs[i][p], sn[i][p]);
+    }
   }
 }
 
@@ -231,7 +246,7 @@ void na3d_wave_kernel(const Na3dArgs a, int n_yb, int n_xb, int n_xg) {
 #pragma unroll
     for (int ds = 0; ds < kNDS; ++ds) qr[ds] = *(const bf16x8*)(p + ds * 16);
   }
-  if (a.q_prep != 0) prep_q(qr, hf, token(t, yqc, xqc), t, yqc, xqc, a);
+  if (a.q_prep != 0) prep_q<kNDS>(qr, hf, token(t, yqc, xqc), t, yqc, xqc, a);
 
   // Box row and first x slot of the 16-key half chunk starting at box key kb2.
   auto half_row = [&](int kb2, int& trow, int& j0) {
@@ -472,6 +487,7 @@ struct PipeCfg {
   static constexpr int kQK = D / 16;                     // MFMAs of QK^T per chunk
   static constexpr int kPV = 2 * (D / 32);               // MFMAs of PV per chunk
   static constexpr int kSlots = kQK + kPV;
+  static constexpr int kPrepGroup = TSTACK && !FEW ? 4 : D / 16;  // d blocks prepared at a time (prep_q)
   static constexpr int kScoresPerSlot = 16 / kSlots;     // softmax work per slot (1 or 2)
   static_assert(kNS % kKeysPerCopy == 0 && kHalfL % 256 == 0, "whole copies per row, bank-aligned planes");
 };
@@ -780,7 +796,7 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
       *(VX_LDS u32x4*)(lds + C::kV + C::kSlot + off) = u32x4{0, 0, 0, 0};
   }
   // q preparation while the first key rows land (its loads overlap theirs)
-  if (a.q_prep != 0) prep_q(qr, hf, token(tqc, yqc, xqc), tqc, yqc, xqc, a);
+  if (a.q_prep != 0) prep_q<C::kPrepGroup>(qr, hf, token(tqc, yqc, xqc), tqc, yqc, xqc, a);
   wait_vmem<0>();
   __syncthreads();
   f32x16 S = s_init;
