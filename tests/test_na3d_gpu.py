@@ -60,7 +60,7 @@ def _expected_kernel(H, W, kw, D, T=1, kt=1, heads=1):
     kt' = min(kt, T)) on `heads` = B * NH grids, written out here independently
     of the library's plan and launcher."""
     k = min(kw, W)
-    few = 2 * torch.cuda.get_device_properties(0).multi_processor_count  # two workgroups per CU
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
     if k <= 9:
         # head dim 64: 1 x 8 x 16 bricks unless they cover more of the y-x
         # plane than the 1 x 4 x 32 ones
@@ -69,9 +69,10 @@ def _expected_kernel(H, W, kw, D, T=1, kt=1, heads=1):
         # head dim 128 with a t window of 2 or more: bricks two t planes deep
         if D == 128 and min(kt, T) >= 2:
             groups = heads * -(-T // 2) * -(-H // 4) * -(-W // 16)
-            return "na3d_tstack_few_kernel" if groups <= few else "na3d_tstack_kernel<128>"
+            few = groups <= 2 * cus or 3 * cus < groups <= 4 * cus
+            return "na3d_tstack_few_kernel" if few else "na3d_tstack_kernel<128>"
         groups = heads * T * -(-H // 4) * -(-W // 32)
-        return "na3d_pipe_few_kernel" if D == 64 and groups <= few else f"na3d_pipe_kernel<16, {D}>"
+        return "na3d_pipe_few_kernel" if D == 64 and groups <= 2 * cus else f"na3d_pipe_kernel<16, {D}>"
     if k <= 13:
         # head dim 64: 32-wide bricks unless they leave more ragged columns
         if D == 64 and -(-W // 32) * 32 == -(-W // 16) * 16:
@@ -325,6 +326,8 @@ def test_na3d_tall_bricks_many_workgroups(gpu, shape, ks, seed):
     (2, 9, 61, 64, (1, 5, 9), 40, 48),      # one-plane windows, ragged x: 480 and 576
     (4, 10, 33, 128, (3, 7, 7), 28, 29),    # t-stacked: 504 and 522
     (3, 7, 17, 128, (2, 5, 9), 64, 66),     # an odd t plane, idle waves: 512 and 528
+    (3, 7, 17, 128, (2, 5, 9), 97, 96),     # 776 workgroups (above three per CU): few again; 768: many
+    (4, 10, 33, 128, (3, 7, 7), 56, 57),    # 1008 workgroups: few; 1026 (above four per CU): many
 ])
 def test_na3d_few_and_many_workgroups(gpu, T, H, W, D, window, few, many):
     """Grids that two workgroups per CU hold run pipelined steps, larger ones
@@ -347,7 +350,41 @@ def test_na3d_few_and_many_workgroups(gpu, T, H, W, D, window, few, many):
     assert name_b == _expected_kernel(H, W, window[2], D, T, window[0], many) and "_few_" not in name_b, name_b
     d = (a[..., heads, :].float() - b.float()).abs()
     assert (d <= 2.0 ** -7 * a[..., heads, :].float().abs() + 1e-5).all(), d.max().item()
-    some = [0, few // 2 + 1, few - 1]
+    n = min(few, many)
+    some = [0, n // 2 + 1, n - 1]
     ref = O.na3d(*(t[..., some, :].float().cpu().numpy() for t in x), window)
     _check(a[..., some, :].float().cpu().numpy(), ref, "few vs oracle")
     _check(b[..., some, :].float().cpu().numpy(), ref, "many vs oracle")
+
+
+@pytest.mark.parametrize("shape,ks,D,seed", [
+    ((1, 3, 17, 33, 37), (3, 7, 7), 64, 94),     # tall bricks: 1,221 workgroups, total % 8 = 5
+    ((2, 2, 9, 40, 29), (2, 5, 11), 64, 95),     # wide tall bricks, two batch items of 232
+    ((1, 5, 9, 33, 23), (3, 5, 15), 64, 96),     # 32-key segments
+    ((1, 5, 9, 17, 13), (5, 5, 5), 128, 97),     # deep t windows keep their own order
+    ((1, 9, 13, 33, 7), (1, 7, 9), 128, 98),     # 1 x 4 x 32 bricks at head dim 128: 504, launch order
+    ((1, 9, 13, 33, 15), (1, 7, 9), 128, 99),    # 1,080
+    ((2, 7, 11, 17, 9), (3, 3, 12), 128, 100),   # tall bricks at head dim 128
+])
+def test_na3d_head_counts(gpu, shape, ks, D, seed):
+    """Grids that fill the chip give each XCD a contiguous eighth of the (head,
+    brick) sequence, for any head count and totals that 8 does not divide:
+    every head bit for bit as in calls on a few heads alone (the same kernel,
+    in launch order), and some of them against the oracle."""
+    from vidax_amd import _lib, neighborhood_attention_3d
+    B, T, H, W, NH = shape
+    _say(f"na3d head counts shape={shape} kernel={ks} D={D} seed={seed}")
+    g = torch.Generator(device=gpu).manual_seed(seed)
+    q, k, v = (torch.randn((B, T, H, W, NH, D), generator=g, device=gpu) for _ in range(3))
+    q, k, v = (q * D ** -0.5).to(torch.bfloat16), k.to(torch.bfloat16), v.to(torch.bfloat16)
+    out = neighborhood_attention_3d(q, k, v, ks)
+    launched = _lib.last_launch()
+    torch.cuda.synchronize()
+    for h in range(0, NH, 3):
+        few = neighborhood_attention_3d(*(x[..., h:h + 3, :].contiguous() for x in (q, k, v)), ks)
+        if _lib.last_launch() == launched:
+            torch.cuda.synchronize()
+            assert torch.equal(out[..., h:h + 3, :], few), (h, launched)
+    heads = [0, NH - 1]
+    ref = O.na3d(*(x[..., heads, :].float().cpu().numpy() for x in (q, k, v)), ks)
+    _check(out[..., heads, :].float().cpu().numpy(), ref, f"oracle ({launched})")

@@ -442,8 +442,8 @@ void na3d_wave_kernel(const Na3dArgs a, int n_yb, int n_xb, int n_xg) {
 // per t plane: one stream of (kt' + 1) planes serves both planes' waves, each
 // scoring only the chunks of its own kt' planes.
 // FEW: the pipelined form for the 1 x 4 x 32 bricks at head dim 64 and the
-// t-stacked bricks too, for grids that two workgroups per CU hold
-// (kNaFewGroups): a wave then has no others to overlap with.
+// t-stacked bricks too, for grids of few workgroups (few_groups): a wave then
+// has no others to overlap with.
 template <int SEG, int D, bool TALL = false, bool WIDE = false, bool DEEP = false, bool TSTACK = false,
           bool FEW = false>
 struct PipeCfg {
@@ -507,10 +507,17 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
   const int col = lane & 31;
 
   // Workgroups are dispatched round-robin over the 8 XCDs (each with its own
-  // L2). With heads % 8 == 0 the linear workgroup id is remapped so that XCD
-  // x walks the bricks of heads x, x+8, ... in order: the workgroups resident
-  // on one XCD then cover neighbouring bricks of one head and share their
-  // key rows in that XCD's L2.
+  // L2). Grids that fill the chip give each XCD a contiguous eighth of the
+  // (head, brick) sequence, whatever the head count (kNaOrderEighths): the
+  // workgroups resident on one XCD then cover neighbouring bricks of a head
+  // and share their key rows in that XCD's L2, where in launch order each of
+  // the eight reads them, which three or four workgroups per CU made worse
+  // (same box, launch order -> eighths: 21x45x80 NH=12 D=128 (3,7,7) 510 -> 362
+  // us, 16x42x64 NH=12 D=64 187 -> 109; against heads x, x + 8, ... on XCD x,
+  // which needed a multiple of 8: 21x45x80 NH=24 729 -> 712, 16x42x64 NH=24 D=64
+  // (1,7,7) 169 -> 150). Smaller grids keep the head walk for multiples of 8
+  // and the launch order for the rest (9x30x52 NH=2 D=128 eighths +3 %: the
+  // light bricks of the last t plane then all sit on two XCDs).
   const int n_tb = (a.T + C::kQT - 1) / C::kQT;  // t bricks
   const int n_bricks = n_tb * n_yb * n_xb;
   int brick, head;
@@ -527,11 +534,18 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
     const int rest = g / n_tb;
     head = rest / ncol;
     brick = (g - rest * n_tb) * ncol + (rest - head * ncol);    // (tb * n_yb + yb) * n_xb + xb
-  } else if ((a.NH & 7) == 0) {
+  } else if (a.order == kNaOrderLaunch && (a.NH & 7) == 0) {
     const int lin = blockIdx.y * n_bricks + blockIdx.x;  // launch order within a batch item
     const int xcd = lin & 7, j = lin >> 3;
     head = xcd + 8 * (j / n_bricks);
     brick = j % n_bricks;
+  } else if ((!FEW || TSTACK) && a.order == kNaOrderEighths) {
+    const int total = n_bricks * a.NH;
+    const int lin = blockIdx.y * n_bricks + blockIdx.x;  // launch order within a batch item
+    const int xcd = lin & 7, j = lin >> 3;
+    const int g = xcd * (total >> 3) + min(xcd, total & 7) + j;  // the eighths are contiguous ranges of g
+    head = g / n_bricks;
+    brick = g - head * n_bricks;
   } else {
     head = blockIdx.y;
     brick = blockIdx.x;
@@ -639,14 +653,15 @@ __device__ __forceinline__ void na3d_pipe_body(const Na3dArgs& a, int n_yb, int 
   // Box rows are walked with a cursor (its y and plane in the box, its row
   // t * Hs + y of the grid) that advances one row at a time, so no step
   // divides by NY. The rows past the last one are copied but masked (their
-  // index is not below nrows): at head dim 128 the cursor stays on the last
-  // row, whose lines are in the CU's cache (7x33x60 NH=12 (1,7,7), whose
+  // index is not below nrows): at head dim 128 and in the pipelined form the
+  // cursor stays on the last row, whose lines are in the CU's cache (7x33x60 NH=12 (1,7,7), whose
   // bricks walk 10 rows and copy 4 more, 59.5 -> 53.9 us; t-stacked bricks
-  // 21x45x80 NH=24 (3,7,7) 754 -> 742 us); at head dim 64, half the bytes a
-  // row, it wraps to the box's first plane, which spares the scalar unit the
+  // 21x45x80 NH=24 (3,7,7) 754 -> 742 us; 32-key segments at head dim 64,
+  // 7x33x60 NH=12 (1,7,17) 36.7 -> 35.0 us); in the block form at head dim 64,
+  // half the bytes a row, it wraps to the box's first plane, which spares the scalar unit the
   // count (5x22x40 NH=16 (3,7,7) 24.5 -> 23.7 us, 33x88x160 NH=4 (11,11,11)
   // 1.510 -> 1.482 ms).
-  constexpr bool kStay = D == 128 || FEW;
+  constexpr bool kStay = D == 128 || !C::kBlock;
   using Row = std::conditional_t<C::kBlock, int, int64_t>;  // block form: row number; pipelined: its byte offset
   struct Cursor {
     int yr, tr, left;  // left (kStay): rows of the box after this one
@@ -1204,15 +1219,29 @@ void na3d_tstack_few_kernel(const Na3dArgs a, int n_yb, int n_xb) {
   na3d_pipe_body<16, 128, false, false, false, true, true>(a, n_yb, n_xb, smem);
 }
 
-// Workgroups up to which the 1 x 4 x 32 bricks at head dim 64 run pipelined
-// steps: two per CU. Same box, block -> pipelined, 11 x 20 planes: 240
-// workgroups at (3,7,7) 12.5 -> 11.2 us, 480 15.1 -> 13.5, 600 17.7 -> 22.0,
-// 960 25.7 -> 27.6; 432 at (5,7,7) 22.2 -> 19.5, 648 26.4 -> 31.8.
-constexpr int64_t kNaFewGroups = 512;
+// Whether the 1 x 4 x 32 bricks at head dim 64 and the t-stacked bricks run
+// pipelined steps at two workgroups per CU: where those hold the grid in one
+// round, and for the t-stacked bricks where they need two and three per CU need
+// two as well. Same box, block -> pipelined: 11 x 20 planes, NH x (3,7,7) at
+// head dim 64, 240 workgroups 12.5 -> 11.2 us, 480 15.1 -> 13.5, 600 17.7 ->
+// 22.0, 960 25.7 -> 27.6; t-stacked, 288 workgroups (7x33x60) 23.9 -> 21.4,
+// 576 34.4 -> 38.2, 960 (9x30x52) 48.6 -> 45.8, 1152 48.9 -> 49.9.
+bool few_groups(const Na3dArgs& a, int64_t groups, int64_t cus) {
+  if (groups <= 2 * cus) return true;
+  if (a.variant == kNaTStack) return groups > 3 * cus && groups <= 4 * cus;
+  return false;
+}
 
 }  // namespace
 
-int launch_na3d_fwd(const Na3dArgs& a, void* stream, const char** launched) {
+int launch_na3d_fwd(const Na3dArgs& args, void* stream, const char** launched) {
+  Na3dArgs a = args;
+  const int64_t cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  // brick order: eighths for grids that fill the chip (deep t windows have theirs)
+  auto set_order = [&](const dim3& grid) {
+    if (a.order == kNaOrderLaunch && (int64_t)grid.x * grid.y * grid.z > 2 * cus)
+      a.order = kNaOrderEighths;
+  };
   if (a.D != 128 && a.D != 64) return (int)hipErrorNotSupported;
   hipStream_t st = (hipStream_t)stream;
   switch (a.variant) {
@@ -1220,6 +1249,7 @@ int launch_na3d_fwd(const Na3dArgs& a, void* stream, const char** launched) {
       const int n_yb = (a.Hs + 7) / 8;
       const int n_xb = (a.W + 15) / 16;
       dim3 grid((unsigned)a.T * n_yb * n_xb, a.NH, a.B);
+      set_order(grid);
       if (a.D == 128) {
         hipLaunchKernelGGL((na3d_tall_kernel<128>), grid, dim3(256), 0, st, a, n_yb, n_xb);
         *launched = "na3d_tall_kernel<128>";
@@ -1234,6 +1264,7 @@ int launch_na3d_fwd(const Na3dArgs& a, void* stream, const char** launched) {
       const int n_yb = (a.Hs + 7) / 8;
       const int n_xb = (a.W + 31) / 32;
       dim3 grid((unsigned)a.T * n_yb * n_xb, a.NH, a.B);
+      set_order(grid);
       hipLaunchKernelGGL((na3d_tall_wide_kernel<64>), grid, dim3(512), 0, st, a, n_yb, n_xb);
       *launched = "na3d_tall_wide_kernel<64>";
       return (int)hipGetLastError();
@@ -1243,6 +1274,7 @@ int launch_na3d_fwd(const Na3dArgs& a, void* stream, const char** launched) {
       const int n_yb = (a.Hs + 3) / 4;
       const int n_xb = (a.W + 31) / 32;
       dim3 grid((unsigned)((a.T + 1) / 2) * n_yb * n_xb, a.NH, a.B);
+      set_order(grid);
       hipLaunchKernelGGL((na3d_deep_kernel<64>), grid, dim3(512), 0, st, a, n_yb, n_xb);
       *launched = "na3d_deep_kernel<64>";
       return (int)hipGetLastError();
@@ -1252,7 +1284,8 @@ int launch_na3d_fwd(const Na3dArgs& a, void* stream, const char** launched) {
       const int n_yb = (a.Hs + 3) / 4;
       const int n_xb = (a.W + 15) / 16;
       dim3 grid((unsigned)((a.T + 1) / 2) * n_yb * n_xb, a.NH, a.B);
-      if ((int64_t)grid.x * grid.y * grid.z <= kNaFewGroups) {
+      set_order(grid);
+      if (few_groups(a, (int64_t)grid.x * grid.y * grid.z, cus)) {
         hipLaunchKernelGGL(na3d_tstack_few_kernel, grid, dim3(256), 0, st, a, n_yb, n_xb);
         *launched = "na3d_tstack_few_kernel";
       } else {
@@ -1266,13 +1299,14 @@ int launch_na3d_fwd(const Na3dArgs& a, void* stream, const char** launched) {
       const int n_yb = (a.Hs + 3) / 4;
       const int n_xb = (a.W + 31) / 32;
       dim3 grid((unsigned)a.T * n_yb * n_xb, a.NH, a.B);
+      set_order(grid);
       if (a.variant == kNaPipe16 && a.D == 128) {
         hipLaunchKernelGGL((na3d_pipe_kernel<16, 128>), grid, dim3(256), 0, st, a, n_yb, n_xb);
         *launched = "na3d_pipe_kernel<16, 128>";
       } else if (a.D == 128) {
         hipLaunchKernelGGL((na3d_pipe_kernel<32, 128>), grid, dim3(256), 0, st, a, n_yb, n_xb);
         *launched = "na3d_pipe_kernel<32, 128>";
-      } else if (a.variant == kNaPipe16 && (int64_t)grid.x * grid.y * grid.z <= kNaFewGroups) {
+      } else if (a.variant == kNaPipe16 && few_groups(a, (int64_t)grid.x * grid.y * grid.z, cus)) {
         hipLaunchKernelGGL(na3d_pipe_few_kernel, grid, dim3(256), 0, st, a, n_yb, n_xb);
         *launched = "na3d_pipe_few_kernel";
       } else if (a.variant == kNaPipe16) {

@@ -76,7 +76,7 @@ struct Na3dArgs {
   int32_t kt, kh, kw;  // window sizes already clamped to the grid extents
   float scale;
   int32_t variant;     // kernel chosen by the launch plan (Na3dVariant)
-  int32_t order;       // brick order of the pipelined kernels (Na3dOrder), chosen by the launch plan
+  int32_t order;       // brick order (Na3dOrder), chosen by the launch plan and the launcher
   // q preparation applied by the kernel as it loads q (0 = q is used as
   // given): bit 1 per-head RMSNorm with q_weight[D] and q_eps, bit 2 times
   // bf16(q_post_scale), bit 4 rotation of adjacent pairs by the token's
@@ -113,10 +113,11 @@ constexpr int32_t kNaTStackMinKt = 2;
 // t windows (clamped) from which the plan takes the deep bricks
 constexpr int32_t kNaDeepMinKt = 5;
 
-// Order in which the pipelined NA kernels' workgroups take their bricks.
+// Order in which the row-streaming NA kernels' workgroups take their bricks.
 enum Na3dOrder : int32_t {
   kNaOrderLaunch = 0,    // launch order (heads spread over the XCDs when NH % 8 == 0)
   kNaOrderTColumns = 1,  // each XCD walks consecutive t planes of brick columns (deep t windows)
+  kNaOrderEighths = 2,   // each XCD walks a contiguous eighth of the (head, brick) sequence (grids that fill the chip)
 };
 // t windows (clamped) from which the plan picks kNaOrderTColumns: bricks of
 // consecutive t planes then share kt' - 1 of their kt' key planes in an L2
