@@ -475,7 +475,7 @@ def test_per_head_norm_takes_any_weight_view(gpu):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,D", [(1, 64), (3, 64), (4, 64), (3, 128), (30, 64)])
-@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (2, 1, 3, 7), (1, 3, 17, 29)])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (2, 1, 3, 7), (1, 3, 17, 29), (2, 5, 39, 41)])
 @pytest.mark.parametrize("rope,post", [(True, 1.0), (False, 0.125), (True, 0.125)])
 def test_per_head_norm_of_ragged_rows(gpu, H, D, shape, rope, post):
     """Rows that are no multiple of 512 values run one chunk per lane over all

@@ -190,12 +190,15 @@ __global__ __launch_bounds__(kWavesPerBlock * 64) void qk_prologue_kernel(const 
 // half of them idle at 256 values: the block at 33x88x160 NH=4 D=64 (11,11,11)
 // 1664 -> 1599 us). A head's head_dim / 8 lanes stay an aligned
 // group, as rows hold whole heads. Memory-bound: kFlat chunks per lane in
-// flight, a grid's width apart. Needs rows * chunks per row < 2^31 - 2^24.
+// flight, the workgroup's 16 KiB side by side (a grid's width apart they cost
+// long rows up to 10 %: 46,800 rows of 125 x 64, norm only, a wave per row 301
+// us, a grid apart 321, side by side 261; 30 x 64 with rotation 70, 78, 70-74).
+// Needs rows * chunks per row < 2^31 - 2^24.
 constexpr int kFlat = 4;
 __global__ __launch_bounds__(256) void qk_prologue_flat_kernel(const PrologueArgs a) {
   const uint32_t n_chunks = (uint32_t)(a.H * a.D / 8);
   const uint32_t total = (uint32_t)a.B * (uint32_t)a.S * n_chunks;
-  const uint32_t stride = gridDim.x * 256;
+  const uint32_t stride = gridDim.x * (kFlat * 256);
   const float ps = (float)to_bf16(a.post_scale);
   const int hpos = (int)((threadIdx.x * 8) % (uint32_t)a.D);  // (256 chunks are a whole number of heads)
   bf16x8 wb;
@@ -204,13 +207,13 @@ __global__ __launch_bounds__(256) void qk_prologue_flat_kernel(const PrologueArg
 #pragma unroll
     for (int e = 0; e < 8; ++e) wb[e] = to_bf16(e < 4 ? w0[e] : w1[e - 4]);
   }
-  for (uint32_t g0 = blockIdx.x * 256 + threadIdx.x; g0 - threadIdx.x % 64 < total; g0 += kFlat * stride) {
+  for (uint32_t g0 = blockIdx.x * (kFlat * 256) + threadIdx.x; g0 - threadIdx.x % 64 < total; g0 += stride) {
     bf16x8 v[kFlat];
     f32x4 cs[kFlat], sn[kFlat];
     int64_t out[kFlat];
 #pragma unroll
     for (int u = 0; u < kFlat; ++u) {
-      const uint32_t g = min(g0 + u * stride, total - 1);  // (past the end: the last chunk, not stored)
+      const uint32_t g = min(g0 + u * 256, total - 1);  // (past the end: the last chunk, not stored)
       const uint32_t row = g / n_chunks, c = g - row * n_chunks;
       const uint32_t b = row / (uint32_t)a.S, s = row - b * (uint32_t)a.S;
       v[u] = __builtin_nontemporal_load((const bf16x8*)((const bf16*)a.x + b * a.x_bstride + s * a.x_sstride + c * 8));
@@ -233,7 +236,7 @@ __global__ __launch_bounds__(256) void qk_prologue_flat_kernel(const PrologueArg
 #pragma unroll
         for (int p = 0; p < 4; ++p) rope_pair(v[u], p, cs[u][p], sn[u][p]);
       }
-      if (g0 + u * stride < total) __builtin_nontemporal_store(v[u], (bf16x8*)((bf16*)a.out + out[u]));
+      if (g0 + u * 256 < total) __builtin_nontemporal_store(v[u], (bf16x8*)((bf16*)a.out + out[u]));
     }
   }
 }
