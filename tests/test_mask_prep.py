@@ -104,18 +104,21 @@ def test_key_masks(gpu, Sk, form):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("Sk", [1, 3, 64, 77, 257, 512])
+@pytest.mark.parametrize("Sk,Sq", [(1, 5), (3, 5), (64, 5), (77, 5), (257, 5), (512, 5), (1, 64), (504, 130),
+                                   (505, 130), (1024, 64), (1023, 65), (4161, 70)])
 @pytest.mark.parametrize("bias_shape,mask_shape", [
     (None, (1, 1, 5, 0)), ((1, 3, 5, 0), None), ((1, 3, 5, 0), (2, 1, 5, 0)), ((2, 3, 1, 0), (1, 1, 5, 0)),
     ((2, 1, 5, 1), (5, 0)), ((3, 5, 0), (2, 1, 1, 1)),
 ])
-def test_full_bias(gpu, Sk, bias_shape, mask_shape):
-    """A 0 extent stands for Sk."""
+def test_full_bias(gpu, Sk, Sq, bias_shape, mask_shape):
+    """A 0 extent stands for Sk, a 5 for Sq. Inputs of 65536 scores a head
+    and more with the key dim strided and the queries next to each other go
+    through 64 x 64 tiles."""
     from vidax_amd.attention import _full_bias
-    B, H, Sq = 2, 3, 5
+    B, H = 2, 3
     rng = np.random.default_rng(Sk)
-    shape = lambda s: tuple(Sk if n == 0 else n for n in s)
-    print(f"[case] full bias Sk={Sk} bias={bias_shape} mask={mask_shape}", flush=True)
+    shape = lambda s: tuple({0: Sk, 5: Sq}.get(n, n) for n in s)
+    print(f"[case] full bias Sk={Sk} Sq={Sq} bias={bias_shape} mask={mask_shape}", flush=True)
     bias = _biases(shape(bias_shape), rng) if bias_shape else None
     mask = rng.random(shape(mask_shape)) < 0.5 if mask_shape else None
     ref = np.zeros((B, H, Sq, Sk), np.float32)
@@ -132,7 +135,11 @@ def test_full_bias(gpu, Sk, bias_shape, mask_shape):
             tm = None if tm is None else tm.transpose(-1, -2).contiguous().transpose(-1, -2)
         x, st = _full_bias(tb, B, H, Sq, Sk, gpu, tm)
         if x is not tb:
-            assert _lib.last_launch() == "full_bias_kernel"
+            lead = tb if tb is not None else tm
+            qs, ks = [0 if n == 1 else s for n, s in zip(lead.shape, lead.stride())][-2:]
+            tiles = 0 < qs < ks and max(y.shape[-2] for y in (tb, tm) if y is not None) * Sk >= 65536
+            want = "full_bias_transposed_kernel" if tiles else "full_bias_kernel"
+            assert _lib.last_launch() == want, (_lib.last_launch(), qs, ks)
         got = torch.as_strided(x, (B, H, Sq, Sk), (*st, 1)).cpu().numpy()
         assert x.data_ptr() % 16 == 0 and all(s % 4 == 0 for s in st)
         assert np.array_equal(got, ref, equal_nan=True)

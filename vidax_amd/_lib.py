@@ -241,6 +241,8 @@ def as_dtype(x, dev: torch.device, dtype: torch.dtype) -> torch.Tensor:
     """x as a tensor of this dtype on dev, its memory holding its values (x
     itself when it is one already; a view that only marks its values as
     negated, as the imaginary part of a conjugate does, is copied)."""
-    if not (isinstance(x, torch.Tensor) and x.dtype == dtype and x.device == dev):
-        x = torch.as_tensor(x, device=dev).to(dtype)
+    if not (isinstance(x, torch.Tensor) and x.device == dev):
+        x = torch.as_tensor(x, device=dev)
+    if x.dtype != dtype:
+        x = x.to(dtype)
     return x.resolve_neg() if x.is_neg() else x

@@ -101,6 +101,11 @@ __global__ __launch_bounds__(kKeyThreads) void key_mask_kernel(const KeyMaskArgs
 constexpr int kBiasWaves = 4;
 constexpr int kBiasSeg = 4096;
 
+// bits of x + -inf: -inf, or NaN where x is NaN or +inf
+__device__ __forceinline__ uint32_t masked_bits(uint32_t x) {
+  return (x & 0x7fffffffu) > 0x7f800000u || x == 0x7f800000u ? kQuietNanBits : kNegInfBits;
+}
+
 __global__ __launch_bounds__(kBiasWaves * 64) void full_bias_kernel(const FullBiasArgs a) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -125,13 +130,55 @@ __global__ __launch_bounds__(kBiasWaves * 64) void full_bias_kernel(const FullBi
         const int64_t k = k0 + e;
         if (k < a.Sk) {
           if (bp != nullptr) o[e] = bp[k * a.bias_strides[3]];
-          // x + -inf: -inf, or NaN where x is NaN or +inf
-          if (mp != nullptr && mp[k * a.mask_strides[3]] == 0)
-            o[e] = (o[e] & 0x7fffffffu) > 0x7f800000u || o[e] == 0x7f800000u ? kQuietNanBits : kNegInfBits;
+          if (mp != nullptr && mp[k * a.mask_strides[3]] == 0) o[e] = masked_bits(o[e]);
         }
       }
       *(u32x4*)(orow + k0) = o;
     }
+  }
+}
+
+// The same for inputs whose queries lie closer together than their keys (a
+// transposed bias): 64 x 64 tiles through LDS, read along the queries and
+// written along the keys, so that both sides are whole lines (a wave per row
+// read 64 lines for 64 values: a call with 4 heads of 4095 x 4095 768 us, in
+// tiles 248; 8 of 2000 x 2000 299 and 117). One tile per workgroup and pass.
+constexpr int kBiasTile = 64;
+
+__global__ __launch_bounds__(256) void full_bias_transposed_kernel(const FullBiasArgs a) {
+  __shared__ uint32_t tile[kBiasTile][kBiasTile + 1];  // [key][query]
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t width = ((int64_t)a.Sk + 63) & ~(int64_t)63;
+  const int64_t n_kt = width / kBiasTile, n_qt = ((int64_t)a.n[2] + kBiasTile - 1) / kBiasTile;
+  const int64_t items = (int64_t)a.n[0] * a.n[1] * n_qt * n_kt;
+  for (int64_t w = blockIdx.x; w < items; w += gridDim.x) {  // (uniform: every thread passes the barriers)
+    const int64_t bhq = w / n_kt, k0 = (w - bhq * n_kt) * kBiasTile;
+    const int64_t bh = bhq / n_qt, q0 = (bhq - bh * n_qt) * kBiasTile;
+    const int b = (int)(bh / a.n[1]), h = (int)(bh - (int64_t)b * a.n[1]);
+    const int64_t q = q0 + lane;
+    const uint32_t* bp = a.bias != nullptr ? (const uint32_t*)a.bias + b * a.bias_strides[0] + h * a.bias_strides[1] +
+                                                 q * a.bias_strides[2]
+                                           : nullptr;
+    const uint8_t* mp =
+        a.mask != nullptr ? a.mask + b * a.mask_strides[0] + h * a.mask_strides[1] + q * a.mask_strides[2] : nullptr;
+#pragma unroll
+    for (int i = 0; i < kBiasTile / 4; ++i) {
+      const int64_t k = k0 + 4 * i + wave;
+      uint32_t o = 0;
+      if (q < a.n[2] && k < a.Sk) {
+        if (bp != nullptr) o = bp[k * a.bias_strides[3]];
+        if (mp != nullptr && mp[k * a.mask_strides[3]] == 0) o = masked_bits(o);
+      }
+      tile[4 * i + wave][lane] = o;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kBiasTile / 4; ++i) {
+      const int64_t row = q0 + 4 * i + wave;
+      if (row < a.n[2]) ((uint32_t*)a.out)[(bh * a.n[2] + row) * width + k0 + lane] = tile[lane][4 * i + wave];
+    }
+    __syncthreads();
   }
 }
 
@@ -146,6 +193,19 @@ int launch_key_masks(const KeyMaskArgs& a, void* stream, const char** launched) 
 }
 
 int launch_full_bias(const FullBiasArgs& a, void* stream, const char** launched) {
+  // Tiles for transposed inputs, by the bias (four times the mask's bytes) if
+  // both are given; heads of fewer scores stay in the CU's cache, and a wave
+  // per row starts more of them at once (64 x 128 x 12 heads of 128 x 128 22 us
+  // a call, in tiles 26; 2 x 256 x 24 of 256 x 256 25 either way).
+  const int64_t* s = a.bias != nullptr ? a.bias_strides : a.mask_strides;
+  if (s[2] > 0 && s[2] < s[3] && (int64_t)a.n[2] * a.Sk >= 256 * 256) {
+    const int64_t tiles = (int64_t)a.n[0] * a.n[1] * (((int64_t)a.n[2] + kBiasTile - 1) / kBiasTile) *
+                          (((int64_t)a.Sk + kBiasTile - 1) / kBiasTile);
+    hipLaunchKernelGGL(full_bias_transposed_kernel, dim3((unsigned)std::min<int64_t>(tiles, 8192)), dim3(256), 0,
+                       (hipStream_t)stream, a);
+    *launched = "full_bias_transposed_kernel";
+    return (int)hipGetLastError();
+  }
   const int64_t n_seg = ((int64_t)a.Sk + kBiasSeg - 1) / kBiasSeg;
   const int64_t items = (int64_t)a.n[0] * a.n[1] * a.n[2] * n_seg;
   const int64_t groups = std::min<int64_t>((items + kBiasWaves - 1) / kBiasWaves, 8192);
