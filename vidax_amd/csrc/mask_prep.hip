@@ -28,7 +28,7 @@ constexpr int kKeysPerThread = 16;
 __global__ __launch_bounds__(kKeyThreads) void key_mask_kernel(const KeyMaskArgs a) {
   __shared__ int wave_last[kKeyThreads / 64];
   const int b = blockIdx.x;
-  const int64_t width = ((int64_t)a.Sk + 63) & ~(int64_t)63;  // (64-bit counters: seq_k goes up to 2^31 - 1)
+  const uint32_t Sk = (uint32_t)a.Sk, width = (Sk + 63) & ~63u;  // (unsigned counters: seq_k goes up to 2^31 - 1)
   const uint8_t* vp = a.valid != nullptr ? a.valid + b * a.valid_strides[0] : nullptr;
   const float* bp = a.bias != nullptr ? a.bias + b * a.bias_strides[0] : nullptr;
   uint8_t* vo = a.valid_rows != nullptr ? a.valid_rows + b * a.row_stride : nullptr;
@@ -36,8 +36,8 @@ __global__ __launch_bounds__(kKeyThreads) void key_mask_kernel(const KeyMaskArgs
   const bool v16 = a.valid_strides[1] == 1 && ((uintptr_t)vp & 15) == 0;
   const bool b16 = a.bias_strides[1] == 1 && ((uintptr_t)bp & 15) == 0;
   int last = 0;
-  for (int64_t k0 = threadIdx.x * kKeysPerThread; k0 < width; k0 += kKeyThreads * kKeysPerThread) {
-    const bool whole = k0 + kKeysPerThread <= a.Sk;
+  for (uint32_t k0 = threadIdx.x * kKeysPerThread; k0 < width; k0 += kKeyThreads * kKeysPerThread) {
+    const bool whole = k0 + kKeysPerThread <= Sk;
     uint32_t vw[4] = {0, 0, 0, 0};  // validity, one byte (0 or 1) per key
     uint32_t bw[16];                // bias bits
     if (vp != nullptr) {
@@ -48,7 +48,7 @@ __global__ __launch_bounds__(kKeyThreads) void key_mask_kernel(const KeyMaskArgs
       } else {
 #pragma unroll
         for (int i = 0; i < 16; ++i)
-          if (k0 + i < a.Sk) vw[i >> 2] |= (vp[(k0 + i) * a.valid_strides[1]] != 0 ? 1u : 0u) << (8 * (i & 3));
+          if (k0 + i < Sk) vw[i >> 2] |= (vp[(k0 + i) * a.valid_strides[1]] != 0 ? 1u : 0u) << (8 * (i & 3));
       }
     }
     if (bp != nullptr) {
@@ -62,7 +62,7 @@ __global__ __launch_bounds__(kKeyThreads) void key_mask_kernel(const KeyMaskArgs
       } else {
 #pragma unroll
         for (int i = 0; i < 16; ++i)
-          bw[i] = k0 + i < a.Sk ? ((const uint32_t*)bp)[(k0 + i) * a.bias_strides[1]] : kNegInfBits;
+          bw[i] = k0 + i < Sk ? ((const uint32_t*)bp)[(k0 + i) * a.bias_strides[1]] : kNegInfBits;
       }
     }
     if (vo != nullptr) *(u32x4*)(vo + k0) = u32x4{vw[0], vw[1], vw[2], vw[3]};
@@ -73,7 +73,7 @@ __global__ __launch_bounds__(kKeyThreads) void key_mask_kernel(const KeyMaskArgs
     if (a.kv_len != nullptr) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        bool ok = k0 + i < a.Sk;
+        bool ok = k0 + i < Sk;
         if (vp != nullptr) ok = ok && ((vw[i >> 2] >> (8 * (i & 3))) & 0xffu) != 0;
         // above -inf: neither -inf nor NaN (tested on the bits)
         if (bp != nullptr) ok = ok && bw[i] != kNegInfBits && (bw[i] & 0x7fffffffu) <= 0x7f800000u;
@@ -109,11 +109,12 @@ __device__ __forceinline__ uint32_t masked_bits(uint32_t x) {
 __global__ __launch_bounds__(kBiasWaves * 64) void full_bias_kernel(const FullBiasArgs a) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t width = ((int64_t)a.Sk + 63) & ~(int64_t)63;
-  const int64_t n_seg = (width + kBiasSeg - 1) / kBiasSeg, items = (int64_t)a.n[0] * a.n[1] * a.n[2] * n_seg;
+  const uint32_t Sk = (uint32_t)a.Sk, width = (Sk + 63) & ~63u;
+  const uint32_t n_seg = (width + kBiasSeg - 1) / kBiasSeg;
+  const int64_t items = (int64_t)a.n[0] * a.n[1] * a.n[2] * n_seg;
   for (int64_t w = (int64_t)blockIdx.x * kBiasWaves + wave; w < items; w += (int64_t)gridDim.x * kBiasWaves) {
-    const int64_t r = w / n_seg, k_lo = (w - r * n_seg) * kBiasSeg;
-    const int64_t k_hi = min(k_lo + kBiasSeg, width);
+    const int64_t r = w / n_seg;
+    const uint32_t k_lo = (uint32_t)(w - r * n_seg) * kBiasSeg, k_hi = min(k_lo + kBiasSeg, width);
     const int64_t bh = r / a.n[2];
     const int q = (int)(r - bh * a.n[2]);
     const int b = (int)(bh / a.n[1]), h = (int)(bh - (int64_t)b * a.n[1]);
@@ -123,12 +124,12 @@ __global__ __launch_bounds__(kBiasWaves * 64) void full_bias_kernel(const FullBi
     const uint8_t* mp =
         a.mask != nullptr ? a.mask + b * a.mask_strides[0] + h * a.mask_strides[1] + q * a.mask_strides[2] : nullptr;
     uint32_t* orow = (uint32_t*)a.out + r * width;
-    for (int64_t k0 = k_lo + lane * 4; k0 < k_hi; k0 += 256) {
+    for (uint32_t k0 = k_lo + lane * 4; k0 < k_hi; k0 += 256) {
       u32x4 o = {0, 0, 0, 0};
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int64_t k = k0 + e;
-        if (k < a.Sk) {
+        const uint32_t k = k0 + e;
+        if (k < Sk) {
           if (bp != nullptr) o[e] = bp[k * a.bias_strides[3]];
           if (mp != nullptr && mp[k * a.mask_strides[3]] == 0) o[e] = masked_bits(o[e]);
         }
