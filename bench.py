@@ -108,8 +108,7 @@ def _flash_inputs(p, dev):
             if pad[b]:
                 valid[b, Sk - int(pad[b]):] = False
         kw["key_valid"] = valid
-        from vidax_amd.attention import _last_valid_plus_one
-        kw["kv_len"] = _last_valid_plus_one(valid)
+        kw["kv_len"] = (valid * torch.arange(1, Sk + 1, device=dev)).amax(dim=1).to(torch.int32)  # last valid key + 1
         valid_keys = [Sk - int(x) for x in pad]
     if "key_bias_pad" in p:
         lo, hi = p["key_bias_pad"]

@@ -706,13 +706,14 @@ def _plain_flash(q, k, v, kw, scale=None):
     """The same call through vx_flash_attn_fwd, which never splits."""
     import ctypes
     from vidax_amd import _lib
-    from vidax_amd.attention import _mask_rows
     B, Sq, H, D = q.shape
     Sk = k.shape[1]
     out = torch.empty_like(q)
     kvl = kw.get("kv_len")
-    kvd = _mask_rows(kw["key_valid"].to(torch.bool), Sk, torch.uint8, 0) if "key_valid" in kw else None
-    kbs = _mask_rows(kw["key_bias"].float(), Sk, torch.float32, float("-inf")) if "key_bias" in kw else None
+    # rows of whole 64-key tiles, padded with invalid / -inf keys
+    pad = lambda x, dtype, fill: torch.nn.functional.pad(x.to(dtype), (0, -Sk % 64), value=fill).contiguous()
+    kvd = pad(kw["key_valid"].to(torch.bool), torch.uint8, 0) if "key_valid" in kw else None
+    kbs = pad(kw["key_bias"], torch.float32, float("-inf")) if "key_bias" in kw else None
     stride = (kvd if kvd is not None else kbs).shape[1] if (kvd is not None or kbs is not None) else 0
     rc = _lib.lib().vx_flash_attn_fwd(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
@@ -794,7 +795,6 @@ def test_masked_self_attention_key_valid_patterns(gpu, pattern):
     mask must give the same result as kv_len alone (the unmasked kernel), and
     every pattern agrees with the oracle."""
     from vidax_amd import _lib, flash_attention, masked_self_attention
-    from vidax_amd.attention import _last_valid_plus_one
     _say(f"masked_self_attention key_valid pattern={pattern}")
     B, S, H, D = 2, 700, 4, 128
     q, k, v = _torch_inputs(B, S, S, H, 41, gpu)
@@ -814,7 +814,8 @@ def test_masked_self_attention_key_valid_patterns(gpu, pattern):
     ref = O.attention_rows(_np(q), _np(k), _np(v), rows, key_valid=_np(valid).astype(bool))
     _check(out[:, torch.from_numpy(rows).to(gpu)], ref, f"key_valid {pattern} ({launched})")
     if pattern != "holes":
-        by_len = flash_attention(q, k, v, kv_len=_last_valid_plus_one(valid))
+        last = (valid * torch.arange(1, S + 1, device=gpu)).amax(dim=1)
+        by_len = flash_attention(q, k, v, kv_len=last)
         torch.cuda.synchronize()
         assert _lib.last_launch() == "flash_pair_kernel<0, 128>", _lib.last_launch()
         same = torch.equal(out, by_len)

@@ -108,7 +108,8 @@ def test_key_masks(gpu, Sk, form):
                                    (505, 130), (1024, 64), (1023, 65), (4161, 70)])
 @pytest.mark.parametrize("bias_shape,mask_shape", [
     (None, (1, 1, 5, 0)), ((1, 3, 5, 0), None), ((1, 3, 5, 0), (2, 1, 5, 0)), ((2, 3, 1, 0), (1, 1, 5, 0)),
-    ((2, 1, 5, 1), (5, 0)), ((3, 5, 0), (2, 1, 1, 1)),
+    ((2, 1, 5, 1), (5, 0)), ((3, 5, 0), (2, 1, 1, 1)), ((1, 3, 5, 1), None), ((2, 3, 5, 0), None), ((5, 1), None),
+    ((1, 1, 1, 0), None),
 ])
 def test_full_bias(gpu, Sk, Sq, bias_shape, mask_shape):
     """A 0 extent stands for Sk, a 5 for Sq. Inputs of 65536 scores a head

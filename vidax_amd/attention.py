@@ -113,30 +113,14 @@ class _KeyMasks:
                     B, Sk, self.kv_len, self.valid, self.bias, self.stride)
 
 
-def _mask_rows(x: torch.Tensor, sk: int, dtype: torch.dtype, fill) -> torch.Tensor:
-    """(B, Sk) validity (uint8, fill 0) or biases (float32, fill -inf) as the
-    key-mask rows of the kernels: (B, round_up(Sk, 64)) contiguous."""
-    if (dtype, fill) not in ((torch.uint8, 0), (torch.float32, float("-inf"))):
-        raise ValueError("key-mask rows are uint8 filled with 0 or float32 filled with -inf")
-    m = _KeyMasks(x.to(torch.bool) if dtype == torch.uint8 else None,
-                  x.to(torch.float32) if dtype == torch.float32 else None, want_len=False)
-    return m.buf.view(dtype).reshape(x.shape[0], m.stride)
-
-
-def _last_valid_plus_one(valid: torch.Tensor) -> torch.Tensor:
-    """(B, Sk) bool -> int32 (B,) index of the last valid key + 1 (0 if none), on device."""
-    m = _KeyMasks(valid.to(torch.bool), None, want_len=True, want_rows=False)
-    return m.buf.view(torch.int32)[:valid.shape[0]]
-
-
 def _full_bias(bias, B: int, H: int, Sq: int, Sk: int, dev, mask=None) -> Tuple[torch.Tensor, Tuple[int, int, int]]:
     """A bias, a boolean mask (False: -inf) or both, each broadcastable to
     (B, H, Sq, Sk) -- every dim 1 or full, as `jnp.broadcast_to` accepts
     (`src/vidax/core/attention.py:282,533`) -- as the kernel reads it: fp32,
     keys contiguous, every query row readable for round_up(Sk, 64) keys,
     16-byte aligned, strides multiples of 4 (0 for broadcast dims). A bias
-    that has that form already is passed as it is; anything else is written in
-    one launch (vx_full_bias_fwd)."""
+    that has that form already is passed as it is; any other fp32 one is written
+    in one launch (vx_full_bias_fwd), other dtypes are cast first."""
     def expand(t, what):
         x = torch.as_tensor(t, device=dev)
         while x.dim() < 4:
@@ -153,15 +137,11 @@ def _full_bias(bias, B: int, H: int, Sq: int, Sk: int, dev, mask=None) -> Tuple[
                       all(x.stride(i) % 4 == 0 for i in range(3))):
         return x, tuple(0 if x.shape[i] == 1 else x.stride(i) for i in range(3))
     lead = [max(t.shape[i] for t in (x, m) if t is not None) for i in range(3)]
-    if x is not None and not x.is_cuda:
-        out = torch.zeros(lead + [width], dtype=torch.float32, device=dev)
-        out[..., :Sk] = x if m is None else x.masked_fill(~m, float("-inf"))
-    else:
-        out = torch.empty(lead + [width], dtype=torch.float32, device=dev)
-        _lib.launch(out.device, _lib.lib().vx_full_bias_fwd,
-                    x.data_ptr() if x is not None else None, _strides(x, range(4)) if x is not None else None,
-                    m.data_ptr() if m is not None else None, _strides(m, range(4)) if m is not None else None,
-                    lead[0], lead[1], lead[2], Sk, out.data_ptr())
+    out = torch.empty(lead + [width], dtype=torch.float32, device=dev)
+    _lib.launch(out.device, _lib.lib().vx_full_bias_fwd,
+                x.data_ptr() if x is not None else None, _strides(x, range(4)) if x is not None else None,
+                m.data_ptr() if m is not None else None, _strides(m, range(4)) if m is not None else None,
+                lead[0], lead[1], lead[2], Sk, out.data_ptr())
     return out, tuple(0 if lead[i] == 1 else out.stride(i) for i in range(3))
 
 

@@ -174,20 +174,6 @@ __device__ __forceinline__ void lds_dma16(const void* src, uint32_t lds_row) {
                : "memory", "m0");
 }
 
-// Raw buffer resource over [base, base + 4 GiB): no stride, untyped 32-bit
-// data, no range limit in practice (every offset used is below 2^31).
-typedef int i32x4_rsrc __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ i32x4_rsrc raw_rsrc(const void* base) {
-  const uint64_t addr = (uint64_t)(uintptr_t)base;
-  // the base is uniform: keep the resource in scalar registers
-  i32x4_rsrc r;
-  r[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)addr);
-  r[1] = __builtin_amdgcn_readfirstlane((int)(uint32_t)(addr >> 32));  // 48-bit address; stride field 0
-  r[2] = -1;                                                            // num_records
-  r[3] = 0x00020000;                                                    // data format 32, raw access
-  return r;
-}
-
 // A wave-uniform 64-bit value moved to scalar registers, so that address
 // arithmetic on it stays on the scalar unit.
 __device__ __forceinline__ uint64_t uniform_u64(uint64_t x) {
@@ -196,13 +182,16 @@ __device__ __forceinline__ uint64_t uniform_u64(uint64_t x) {
   return ((uint64_t)hi << 32) | lo;
 }
 
-// raw_rsrc from a wave-uniform byte address (kept in scalar registers).
+// Raw buffer resource over [addr, addr + 4 GiB) of a wave-uniform byte address
+// (kept in scalar registers): no stride, untyped 32-bit data, no range limit in
+// practice (every offset used is below 2^31).
+typedef int i32x4_rsrc __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ i32x4_rsrc raw_rsrc_u64(uint64_t addr) {
   i32x4_rsrc r;
   r[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)addr);
-  r[1] = __builtin_amdgcn_readfirstlane((int)(uint32_t)(addr >> 32));
-  r[2] = -1;
-  r[3] = 0x00020000;
+  r[1] = __builtin_amdgcn_readfirstlane((int)(uint32_t)(addr >> 32));  // 48-bit address; stride field 0
+  r[2] = -1;                                                            // num_records
+  r[3] = 0x00020000;                                                    // data format 32, raw access
   return r;
 }
 
