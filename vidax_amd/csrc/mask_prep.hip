@@ -1,10 +1,10 @@
 // Mask preparation of the flash kernels for gfx950: the caller's masks, in
 // whatever strides and widths they come, to the forms the attention kernels
 // stage, one launch each. As chains of six to eight elementwise and reduction
-// launches they took more time than the attention itself: masked
-// self-attention B=2 H=24 S=256 56.6 -> 29.0 us a call, a full bias with a
-// padding mask B=2 H=8 S=512 D=64 63.5 -> 34.2 us, a key bias H=24 S=8192 686
-// -> 677 us.
+// launches they took more time than the attention itself: one launch instead
+// took masked self-attention B=2 H=24 S=256 from 56.6 to 29.0 us a call, a full
+// bias with a padding mask B=2 H=8 S=512 D=64 from 63.5 to 34.2 us, a key bias
+// H=24 S=8192 from 686 to 677 us.
 #include "vx_gfx950.hpp"
 #include "vx_kernels.h"
 

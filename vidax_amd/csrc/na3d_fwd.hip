@@ -1,22 +1,27 @@
 // 3D neighbourhood attention forward for gfx950 (NATTEN semantics with
 // boundary-clamped windows), bf16 in/out, head dim 128 or 64.
 //
-// Three kernels, chosen by the clamped x window kw' (the launch plan of the
-// C ABI, Na3dVariant; at head dim 64 also by how the grid's y x x plane
+// Three kinds of kernel, chosen by the clamped x window kw' (the launch plan of
+// the C ABI, Na3dVariant; at head dim 64 also by how the grid's y x x plane
 // rounds up to each brick shape):
 // - na3d_pipe_kernel<SEG, D> (kw' <= 9 or 13 < kw' <= 25): a workgroup of 4
 //   waves owns a 1 (t) x 4 (y) x 32 (x) query brick of one head and streams
 //   the union of its windows, kt' x NY key rows (t', y'), through LDS with
 //   the DMA copy path; each wave reads the SEG-wide x window its 4 x 8
-//   queries need, 32 keys per step, and runs the flash kernel's software
-//   pipeline (QK^T of the next chunk and PV of the previous one interleaved
-//   with the masking and lazy-rescale softmax of the current one).
+//   queries need, 32 keys per step. A step is either pipelined as in the
+//   flash kernel (QK^T of the next chunk and PV of the previous one
+//   interleaved with the masking and lazy-rescale softmax of the current one,
+//   two sets of scores and probabilities) or in block form (the softmax of a
+//   chunk, then its PV with the next chunk's QK^T, one set of each and one
+//   more wave per SIMD); see the row-streaming kernels below.
 //   na3d_tstack_kernel<128> (kw' <= 9 with t windows of 2 and more, head dim
 //   128) runs the same body on 2 x 4 x 16 bricks, two 4 x 8 waves per t
 //   plane sharing one stream of kt' + 1 planes of 24-key rows (30 % fewer
 //   copied rows per query at a (3,7,7) window, no half-empty brick at
 //   widths of a multiple of 16); a wave whose t window misses the chunks
-//   around a step only copies.
+//   around a step only copies. na3d_pipe_few_kernel and
+//   na3d_tstack_few_kernel are the pipelined forms of the two block-form
+//   kernels for grids of few workgroups.
 // - na3d_tall_kernel<D> (9 < kw' <= 13, and kw' <= 9 at head dim 64 when
 //   its bricks pad the grid no more): the same body on 1 x 8 x 16 bricks
 //   with waves of 8 y x 4 x queries, so that a wave's x window still fits a
@@ -29,7 +34,7 @@
 //   x-positions, with K fragments loaded straight from global memory and V
 //   staged through a wave-private, double-buffered LDS slot; its waves never
 //   synchronise with each other.
-// In all three, every (query, key) pair outside the query's own window is
+// In all of them, every (query, key) pair outside the query's own window is
 // set to -inf before the exponent, so each query attends exactly its
 // kt' x kh' x kw' window.
 #include "vx_gfx950.hpp"
@@ -417,7 +422,7 @@ void na3d_wave_kernel(const Na3dArgs a, int n_yb, int n_xb, int n_xg) {
 //   needs 24 registers fewer, so one more wave fits a SIMD, and those waves
 //   overlap each other. Same box, pipelined -> block: 21x45x80 NH=24 (3,7,7)
 //   at head dim 128 (2 -> 3 waves per SIMD) 0.760 -> 0.747 ms; 5x11x60 NH=32
-//   at head dim 64 (1 x 4 x 32 bricks, 2 -> 4) 27.2 -> 23.4 us. The 32-key
+//   at head dim 64 (1 x 4 x 32 bricks, 2 -> 4) 27.2 -> 24.4 us. The 32-key
 //   segments at head dim 64 (3 -> 4) lost 7 % at a (3,11,15) window and stay
 //   pipelined.
 //
@@ -433,7 +438,7 @@ void na3d_wave_kernel(const Na3dArgs a, int n_yb, int n_xb, int n_xg) {
 // apart (kHalfStep: a barrier before each block of the step, waves 4-7 one
 // barrier behind waves 0-3), so that one wave's MFMA block meets the other's
 // softmax block, and only waves 0-3 copy: stage 5 (33x88x160 NH=4 at (11,11,
-// 11), deep bricks) 1.476 -> 1.434 ms.
+// 11), deep bricks) 1.511 -> 1.465 ms.
 // DEEP: wide bricks two t planes deep, 2 (t) x 4 (y) x 32 (x), waves of 2 t x
 // 4 y x 4 x queries: for a t window of kt' planes the union of a wave's
 // windows is (kt' + 1) x (kh' + 3) rows instead of kt' x (kh' + 7), e.g. 12 x
@@ -1222,10 +1227,10 @@ void na3d_tstack_few_kernel(const Na3dArgs a, int n_yb, int n_xb) {
 // Whether the 1 x 4 x 32 bricks at head dim 64 and the t-stacked bricks run
 // pipelined steps at two workgroups per CU: where those hold the grid in one
 // round, and for the t-stacked bricks where they need two and three per CU need
-// two as well. Same box, block -> pipelined: 11 x 20 planes, NH x (3,7,7) at
-// head dim 64, 240 workgroups 12.5 -> 11.2 us, 480 15.1 -> 13.5, 600 17.7 ->
-// 22.0, 960 25.7 -> 27.6; t-stacked, 288 workgroups (7x33x60) 23.9 -> 21.4,
-// 576 34.4 -> 38.2, 960 (9x30x52) 48.6 -> 45.8, 1152 48.9 -> 49.9.
+// two as well. Same box, block -> pipelined us at (3,7,7): 5x11x20 at head dim
+// 64, 240 workgroups 12.9 -> 11.7, 480 15.1 -> 13.5, 720 18.1 -> 23.0, 960 21.4
+// -> 25.2; t-stacked, 288 workgroups (7x33x60) 23.5 -> 20.6, 576 28.9 -> 32.6,
+// 960 (9x30x52) 48.7 -> 45.5, 1152 (7x33x60) 48.7 -> 49.8.
 bool few_groups(const Na3dArgs& a, int64_t groups, int64_t cus) {
   if (groups <= 2 * cus) return true;
   if (a.variant == kNaTStack) return groups > 3 * cus && groups <= 4 * cus;
