@@ -88,9 +88,10 @@ int32_t vx_flash_attn_fwd(const void* q, const void* k, const void* v, void* out
  * workgroups over the two halves of the keys, whose fp32 partial results go
  * to the workspace and are merged by a second kernel on the same stream.
  * A grid of at most half as many 128-query workgroups as the device has
- * compute units, over at least 24 64-key tiles, splits every query tile so.
- * (Below, up to one workgroup per compute unit, a tile's keys are halved
- * inside one workgroup and nothing goes to the workspace.)
+ * compute units, over 20 to 32 64-key tiles (by its size and head_dim) and
+ * more, splits every query tile so. (Below, up to one workgroup per compute
+ * unit, a tile's keys are halved inside one workgroup and nothing goes to the
+ * workspace.)
  * That needs vx_flash_attn_workspace_size() bytes (0: no split for this
  * shape on this device); with a smaller workspace (or NULL), or with a
  * key_bias, the call runs without the split, as vx_flash_attn_fwd. The workspace must be 16-byte
