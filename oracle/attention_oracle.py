@@ -2,7 +2,7 @@
 
 TEST INFRASTRUCTURE ONLY. Nothing in the product (`vidax_amd`) imports this
 module; only `tests/`, `__graft_entry__.smoke()` and the `cpu_baseline` leg of
-`bench.py` may use it, and only as the checker (or, for the baseline, as the
+`bench.py` may use it, and for expected results only (or, for the baseline, as the
 timed CPU restatement). The product path fails loudly when its HIP library is
 missing instead of falling back to anything here.
 

@@ -1,5 +1,5 @@
 """CPU oracle of the attention prologue (q/k RMSNorm, 3D rotary embedding) --
-test infrastructure only (used by tests/ as the checker).
+test infrastructure only (the expected results of tests/).
 
 Restates, in numpy with the reference's dtype points:
   - RMSNorm, `src/vidax/core/attention.py:149-161`: x to fp32, mean of squares
